@@ -139,6 +139,18 @@ __device__ __forceinline__ T wave_inclusive_scan(T v) {
   return v;
 }
 
+// Wave-wide minimum / maximum of a 32-bit value (all lanes active).
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, dpp_take<0x111, 0xf>(v));  // row_shr:1, 2, 4, 8, then the row broadcasts
+  v = max(v, dpp_take<0x112, 0xf>(v));
+  v = max(v, dpp_take<0x114, 0xf>(v));
+  v = max(v, dpp_take<0x118, 0xf>(v));
+  v = max(v, dpp_take<0x142, 0xa>(v));
+  v = max(v, dpp_take<0x143, 0xc>(v));
+  return readlane_u32(v, 63);
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) { return ~wave_max(~v); }
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
