@@ -123,17 +123,6 @@ __device__ __forceinline__ void add_passing(double sl, double e, uint64_t limit,
   }
 }
 
-// acc += w 2^-sl where the alpha test passes (the voxelizer's form).
-template <typename T>
-__device__ __forceinline__ void add_passing(T sl, typename Bits<T>::type limit, T w, T &acc) {
-  T e = neg_exp2(sl);
-  asm volatile("" : "+v"(e));
-  if (alpha_pass(sl, limit)) {
-    __builtin_amdgcn_sched_barrier(0);
-    acc = fma(w, e, acc);
-  }
-}
-
 // Bits of a limit kept in a T slot (forward records stage it in LDS).
 __device__ __forceinline__ float limit_as_value(uint32_t b) { return __uint_as_float(b); }
 __device__ __forceinline__ double limit_as_value(uint64_t b) {

@@ -153,19 +153,27 @@ __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
     }
     __syncthreads();
     const int cnt = static_cast<int>(min(static_cast<int64_t>(nb), end - base));
+    const uint64_t exec = __builtin_amdgcn_read_exec();
     for (int t = 0; t < cnt; ++t) {
       const V4 mo = s_rec[3 * t];
       const V4 h0 = s_rec[3 * t + 1];
       const V4 h1 = s_rec[3 * t + 2];
       const typename Bits<T>::type lim = bits_of(h1.z);
-      const T dy = py - mo.y, dz = pz - mo.z;
+      const T dx0 = px0 - mo.x, dy = py - mo.y, dz = pz - mo.z;
       const T B = h0.y * dy + h0.z * dz;
       const T C = (h0.w * dy + h1.x * dz) * dy + h1.y * dz * dz;
+      constexpr int kRun = R < 8 ? R : 8;  // voxels per run of exps
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const T dx = (px0 + static_cast<T>(r)) - mo.x;
-        const T sl = (h0.x * dx + B) * dx + C;
-        add_passing(sl, lim, mo.w, acc[r]);
+      for (int r = 0; r < R; r += kRun) {
+        T sl[kRun], e[kRun];
+#pragma unroll
+        for (int k = 0; k < kRun; ++k) {
+          const T dx = dx0 + static_cast<T>(r + k);
+          sl[k] = fma(fma(h0.x, dx, B), dx, C);
+        }
+        neg_exp2_run(sl, e);
+#pragma unroll
+        for (int k = 0; k < kRun; ++k) add_passing(sl[k], e[k], lim, mo.w, acc[r + k], exec);
       }
     }
   }
@@ -197,7 +205,13 @@ __device__ __forceinline__ void load_bwd_record_plain(const T *__restrict__ mean
                                                       int64_t N, bool in_list, const Brick &b,
                                                       BwdRecord<T> &rec) {
   rec.live = in_list && g >= 0 && g < N;
-  rec.o = rec.live ? opac[g] : static_cast<T>(0);
+  // Loaded together (one memory round trip), the opacity tested after.
+  const int64_t gl = rec.live ? g : 0;
+  rec.o = opac[gl];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) rec.m[c] = means3d[3 * gl + c];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) rec.q[c] = conics[6 * gl + c];
   // |alpha| <= |o| for sigma >= 0: nothing passes (non-finite o stays live).
   if (fabs(rec.o) < static_cast<T>(kThr3)) rec.live = false;
   rec.cu.ok = false;
@@ -212,10 +226,6 @@ __device__ __forceinline__ void load_bwd_record_plain(const T *__restrict__ mean
     rec.i1 = -1;
     return;
   }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) rec.m[c] = means3d[3 * g + c];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) rec.q[c] = conics[6 * g + c];
   scaled_conic(rec.q, rec.h);
   bool fin = true;
 #pragma unroll
@@ -330,9 +340,17 @@ __device__ __forceinline__ uint64_t reach_mask(const BwdRecord<T> &rec, const Br
   return reach;
 }
 
+// A batch of the forward below whose records reach at least this share of
+// their 64 rows on average walks every row: no set to step through, uniform
+// reads of the staged records, no transpose.  Measured on trees (7.1 M records
+// of a 250 x 201 x 173 volume, nearly every row reached) 0.888 -> 0.821 ms,
+// and 0.809 ms with equal shares per wave; from 5/8 on the same, and lists of
+// small footprints (0.62 of the rows walked) stay below it.
+constexpr int kDenseShareNum = 3, kDenseShareDen = 4;
+
 // Forward at brick size 8 with culled rows.  S waves per brick; lane =
 // x-row (slice lane / 8, row lane % 8), its 8 voxels in registers.  Wave w
-// takes the batches of 64 records w, w + S, w + 2S, ... of the brick's list.
+// takes the w-th of S equal shares of the brick's list, in batches of 64.
 // Per batch, each lane loads one record and the rows it reaches
 // (reach_mask); a 64 x 64 bit transpose hands each row's lane the set of
 // batch records that reach that row; each lane then walks its own set in
@@ -367,19 +385,52 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
   const T py = static_cast<T>(b.oj + lj) + half;
   const T pz = static_cast<T>(b.oi + li) + half;
   const T px0 = static_cast<T>(b.ok) + half;
-  const int64_t start = tile_offsets[key];
-  const int64_t end = (key == n_keys - 1) ? n_isects : static_cast<int64_t>(tile_offsets[key + 1]);
+  const int64_t l0 = tile_offsets[key];
+  const int64_t l1 = (key == n_keys - 1) ? n_isects : static_cast<int64_t>(tile_offsets[key + 1]);
+  const int64_t start = l0 + (l1 - l0) * w / S, end = l0 + (l1 - l0) * (w + 1) / S;
   T acc[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) acc[k] = 0;
-  for (int64_t base = start + 64 * w; base < end; base += 64 * S) {
-    const int64_t idx = base + lane;
+  // Adds batch record t to the lane's row.  The mask the alpha test restores
+  // is the caller's (lanes whose set is exhausted stay off).
+  const auto add_record = [&](int t, uint64_t exec) {
+    const V4 qa = s_rec[w][t][0], qh = s_rec[w][t][1], qr = s_rec[w][t][2];
+    const V4 q0 = s_rec[w][t][3], q1 = s_rec[w][t][4];
+    const T dxs[R] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    const typename Bits<T>::type lim = bits_of(qr.y);
+    const T dy = py - qa.x, dz = pz - qa.y;
+    const T B = qh.x * dy + qh.y * dz;
+    const T C = (qh.z * dy + qh.w * dz) * dy + qr.x * dz * dz;
+    T sl[R], e[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) sl[k] = (qa.w * dxs[k] + B) * dxs[k] + C;
+    neg_exp2_run(sl, e);
+#pragma unroll
+    for (int k = 0; k < R; ++k) add_passing(sl[k], e[k], lim, qa.z, acc[k], exec);
+  };
+  // The ids of the wave's next batch, loaded a batch ahead (one memory round
+  // trip fewer before the records' own loads).
+  int64_t idx = start + lane;
+  int32_t next_id = idx < end ? flatten_ids[idx] : -1;
+  bool all_rows = false;  // uniform: an earlier batch reached nearly every row
+  for (int64_t base = start; base < end; base += 64) {
     const bool in = idx < end;
-    const int64_t g = in ? static_cast<int64_t>(flatten_ids[idx]) : -1;
+    const int64_t at = idx, g = in ? static_cast<int64_t>(next_id) : -1;
+    idx += 64;
+    next_id = idx < end ? flatten_ids[idx] : -1;
     BwdRecord<T> rec;
-    load_bwd_record(means3d, conics, opac, g, N, in, b, rec);
-    const uint64_t reach = rec.live ? reach_mask(rec, b, px0 - rec.m[0]) : 0ull;
-    if (reach_out != nullptr && in) reach_out[idx] = reach;
+    uint64_t reach = 0;
+    // A caller that takes the masks needs every batch's; otherwise, once a
+    // batch of the brick reached nearly every row, the next ones walk them
+    // all (a row that a record does not reach adds exact zeros).
+    const bool cull = reach_out != nullptr || !all_rows;
+    if (cull) {
+      load_bwd_record(means3d, conics, opac, g, N, in, b, rec);
+      reach = rec.live ? reach_mask(rec, b, px0 - rec.m[0]) : 0ull;
+      if (reach_out != nullptr && in) reach_out[at] = reach;
+    } else {
+      load_bwd_record_plain(means3d, conics, opac, g, N, in, b, rec);
+    }
     V4 a, hq, hr, d0, d1;
     a.x = rec.m[1];
     a.y = rec.m[2];
@@ -390,7 +441,7 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
     hq.z = rec.h[3];
     hq.w = rec.h[4];
     hr.x = rec.h[5];
-    hr.y = limit_as_value(rec.lim);
+    hr.y = limit_as_value(rec.live ? rec.lim : static_cast<typename Bits<T>::type>(0));
     hr.z = 0;
     hr.w = 0;
     // The column offsets from the voxel centres x_k + 1/2 = px0 + k (exact),
@@ -417,26 +468,26 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
     s_rec[w][lane][2] = hr;
     s_rec[w][lane][3] = d0;
     s_rec[w][lane][4] = d1;
+    const int cnt = static_cast<int>(min(static_cast<int64_t>(64), end - base));
+    // Walking every row in step costs about kDenseShare of walking each
+    // row's own set, record for record (uniform reads, no set to step
+    // through, no transpose).
+    if (cull) all_rows = wave_sum(__popcll(reach)) * kDenseShareDen >= 64 * cnt * kDenseShareNum;
+    uint64_t mine = 0;
     // Bit t of lane r's set: batch record t reaches row r.
-    uint64_t mine = transpose_bits64(reach, static_cast<uint32_t>(lane));
+    if (!all_rows) mine = transpose_bits64(reach, static_cast<uint32_t>(lane));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    while (mine != 0ull) {
-      const int t = static_cast<int>(__builtin_ctzll(mine));
-      mine &= mine - 1ull;
-      const V4 qa = s_rec[w][t][0], qh = s_rec[w][t][1], qr = s_rec[w][t][2];
-      const V4 q0 = s_rec[w][t][3], q1 = s_rec[w][t][4];
-      const T dxs[R] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-      const typename Bits<T>::type lim = bits_of(qr.y);
-      const T dy = py - qa.x, dz = pz - qa.y;
-      const T B = qh.x * dy + qh.y * dz;
-      const T C = (qh.z * dy + qh.w * dz) * dy + qr.x * dz * dz;
-#pragma unroll
-      for (int k = 0; k < R; ++k) {
-        const T dx = dxs[k];
-        const T sl = (qa.w * dx + B) * dx + C;
-        add_passing(sl, lim, qa.z, acc[k]);
+    if (all_rows) {
+      const uint64_t exec = __builtin_amdgcn_read_exec();
+#pragma unroll 1
+      for (int t = 0; t < cnt; ++t) add_record(t, exec);
+    } else {
+      while (mine != 0ull) {
+        const int t = static_cast<int>(__builtin_ctzll(mine));
+        mine &= mine - 1ull;
+        add_record(t, __builtin_amdgcn_read_exec());
       }
     }
   }
@@ -474,9 +525,11 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
 // kReach: the slices' row ranges come from `reach` (bit 8 * slice + row of
 // the reached rows, as voxel_bwd_chunk_kernel computes them) instead of
 // slice_rows.
+// v: the gradient at the brick's first voxel, with the given slice and row
+// strides; every row 16-byte aligned.
 template <typename T, int R, bool kReach = false>
 __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const Brick &b,
-                                                 const T *__restrict__ v_vol, int64_t plane,
+                                                 const T *__restrict__ v, int64_t plane,
                                                  uint32_t D2, T dx0, T &T0, T &T1, T &T2, T &Y0,
                                                  T &Z0, T &Y1, T &Z1, T &YY, T &YZ, T &ZZ,
                                                  uint64_t reach = 0) {
@@ -504,7 +557,7 @@ __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const 
       slice_rows(rec, b, in_slice, dz, dx0, j0, j1);
     }
     const T h4dz = rec.h[4] * dz, h5dzz = rec.h[5] * dz * dz, Bz = rec.h[2] * dz;
-    const T *__restrict__ vslice = v_vol + static_cast<int64_t>(i) * plane + b.ok;
+    const T *__restrict__ vslice = v + static_cast<int64_t>(li) * plane;
 #pragma unroll 1
     for (int lj = 0; lj < R; ++lj) {
       const int j = b.oj + lj;
@@ -514,21 +567,23 @@ __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const 
       const T B = fma(rec.h[1], dy, Bz);
       const T C = fma(fma(rec.h[3], dy, h4dz), dy, h5dzz);
       const typename Bits<T>::type lim = in_row ? rec.lim : 0;
-      const T *__restrict__ vrow = vslice + static_cast<int64_t>(j) * D2;
+      const T *__restrict__ vrow = vslice + static_cast<int64_t>(lj) * D2;
       T vv[R];
 #pragma unroll
       for (int q = 0; q < R / kq; ++q)
         *reinterpret_cast<Q *>(vv + q * kq) = *reinterpret_cast<const Q *>(vrow + q * kq);
       T s0 = 0, s1 = 0;
+      // Explicit FMAs keep the row-invariant products of dx_k from being
+      // hoisted into extra registers.
+      T sl[R], e[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) sl[k] = fma(fma(rec.h[0], dxk[k], B), dxk[k], C);
+      neg_exp2_run(sl, e);
 #pragma unroll
       for (int k = 0; k < R; ++k) {
-        // Explicit FMAs keep the row-invariant products of dx_k from being
-        // hoisted into extra registers.
         const T dx = dxk[k];
-        const T sl = fma(fma(rec.h[0], dx, B), dx, C);
-        const T e = neg_exp2(sl);
-        const T p = vv[k] * e;  // unconditional, not a branch around the load and exp
-        const T w = alpha_pass(sl, lim) ? p : static_cast<T>(0);
+        const T p = vv[k] * e[k];  // unconditional, not a branch around the load and exp
+        const T w = alpha_pass(sl[k], lim) ? p : static_cast<T>(0);
         wk[k] += w;
         s0 += w;
         s1 = fma(w, dx, s1);
@@ -550,6 +605,64 @@ __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const 
     T1 += wx;
     T2 += wx * dxk[k];
   }
+}
+
+// The rows of one record's brick with masked loads, for bricks of any size
+// and extent (guard: voxel_row's kGuard, uniform per wave).
+template <typename T, int R, bool kExact>
+__device__ __forceinline__ void voxel_brick_rows(const BwdRecord<T> &rec, const Brick &b,
+                                                 const T *__restrict__ v_vol, int64_t plane,
+                                                 uint32_t D2, T dx0, int nts, bool vec, bool guard,
+                                                 T &T0, T &T1, T &T2, T &Y0, T &Z0, T &Y1, T &Z1,
+                                                 T &YY, T &YZ, T &ZZ) {
+  const T half = static_cast<T>(0.5);
+      // Rolled loops: unrolled, the slices and rows multiply the registers.
+#pragma unroll 1
+      for (int li = 0; li < R; ++li) {
+        if (!kExact && li >= nts) break;
+        const int i = b.oi + li;
+        const bool in_slice = rec.live && i >= rec.i0 && i <= rec.i1;
+        if (ballot(in_slice) == 0) continue;
+        const T dz = (static_cast<T>(i) + half) - rec.m[2];
+        // Rows of this slice the lane's ellipsoid can reach.
+        int j0, j1;
+        slice_rows(rec, b, in_slice, dz, dx0, j0, j1);
+        const T h4dz = rec.h[4] * dz, h5dzz = rec.h[5] * dz * dz, Bz = rec.h[2] * dz;
+#pragma unroll 1
+        for (int lj = 0; lj < R; ++lj) {
+          if (!kExact && lj >= nts) break;
+          const int j = b.oj + lj;
+          const bool in_row = j >= j0 && j <= j1;
+          if (ballot(in_row) == 0) continue;
+          const T dy = (static_cast<T>(j) + half) - rec.m[1];
+          const T B = rec.h[1] * dy + Bz;
+          const T C = (rec.h[3] * dy + h4dz) * dy + h5dzz;
+          const T *__restrict__ vrow =
+              v_vol +
+              (in_row ? static_cast<int64_t>(i) * plane + static_cast<int64_t>(j) * D2 : 0) + b.ok;
+          T vv[R];
+          if (vec)
+            load_grad_row<T, R, true>(vrow, in_row, b.nk, nts, vv);
+          else
+            load_grad_row<T, R, false>(vrow, in_row, b.nk, nts, vv);
+          T s0 = 0, s1 = 0, s2 = 0;
+          if (guard)
+            voxel_row<T, R, kExact, true>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
+          else
+            voxel_row<T, R, kExact, false>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
+          T0 += s0;
+          T1 += s1;
+          T2 += s2;
+          const T dys0 = dy * s0, dzs0 = dz * s0;
+          Y0 += dys0;
+          Z0 += dzs0;
+          YY += dy * dys0;
+          YZ += dz * dys0;
+          ZZ += dz * dzs0;
+          Y1 += dy * s1;
+          Z1 += dz * s1;
+        }
+      }
 }
 
 // Records in brick order (tile_offsets, flatten_ids; isect_ids optional),
@@ -600,55 +713,11 @@ __global__ __launch_bounds__(kBwdThreads) void voxel_bwd_kernel(
   if constexpr (kExact && R % Quad<T>::n == 0)
     full = vec && ballot(b.ni < nts || b.nj < nts || b.nk < nts) == 0;
   if (full && ballot(rec.live) != 0) {
-    voxel_brick_full<T, R>(rec, b, v_vol, plane, D2, dx0, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+    voxel_brick_full<T, R>(rec, b, v_vol + b.oi * plane + static_cast<int64_t>(b.oj) * D2 + b.ok,
+                           plane, D2, dx0, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
   } else if (ballot(rec.live) != 0) {
-    // Rolled loops: unrolled, the slices and rows multiply the registers.
-#pragma unroll 1
-    for (int li = 0; li < R; ++li) {
-      if (!kExact && li >= nts) break;
-      const int i = b.oi + li;
-      const bool in_slice = rec.live && i >= rec.i0 && i <= rec.i1;
-      if (ballot(in_slice) == 0) continue;
-      const T dz = (static_cast<T>(i) + half) - rec.m[2];
-      // Rows of this slice the lane's ellipsoid can reach.
-      int j0, j1;
-      slice_rows(rec, b, in_slice, dz, dx0, j0, j1);
-      const T h4dz = rec.h[4] * dz, h5dzz = rec.h[5] * dz * dz, Bz = rec.h[2] * dz;
-#pragma unroll 1
-      for (int lj = 0; lj < R; ++lj) {
-        if (!kExact && lj >= nts) break;
-        const int j = b.oj + lj;
-        const bool in_row = j >= j0 && j <= j1;
-        if (ballot(in_row) == 0) continue;
-        const T dy = (static_cast<T>(j) + half) - rec.m[1];
-        const T B = rec.h[1] * dy + Bz;
-        const T C = (rec.h[3] * dy + h4dz) * dy + h5dzz;
-        const T *__restrict__ vrow =
-            v_vol +
-            (in_row ? static_cast<int64_t>(i) * plane + static_cast<int64_t>(j) * D2 : 0) + b.ok;
-        T vv[R];
-        if (vec)
-          load_grad_row<T, R, true>(vrow, in_row, b.nk, nts, vv);
-        else
-          load_grad_row<T, R, false>(vrow, in_row, b.nk, nts, vv);
-        T s0 = 0, s1 = 0, s2 = 0;
-        if (guard)
-          voxel_row<T, R, kExact, true>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
-        else
-          voxel_row<T, R, kExact, false>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
-        T0 += s0;
-        T1 += s1;
-        T2 += s2;
-        const T dys0 = dy * s0, dzs0 = dz * s0;
-        Y0 += dys0;
-        Z0 += dzs0;
-        YY += dy * dys0;
-        YZ += dz * dys0;
-        ZZ += dz * dzs0;
-        Y1 += dy * s1;
-        Z1 += dz * s1;
-      }
-    }
+    voxel_brick_rows<T, R, kExact>(rec, b, v_vol, plane, D2, dx0, nts, vec, guard, T0, T1, T2, Y0,
+                                   Z0, Y1, Z1, YY, YZ, ZZ);
   }
   if (!key_ok) return;
   // Per-voxel terms of VoxelizeToVoxelsBwd.cu:409-421 summed over the brick
@@ -682,6 +751,65 @@ __global__ __launch_bounds__(kBwdThreads) void voxel_bwd_kernel(
   atomic_add(v_opac + g, go);
 }
 
+// The row of a record's ten partials: the per-voxel terms of
+// VoxelizeToVoxelsBwd.cu:409-421 summed over the brick.
+template <typename T>
+__device__ __forceinline__ void store_partials(T *__restrict__ rows, int64_t e,
+                                               const BwdRecord<T> &rec, T T0, T T1, T T2, T Y0,
+                                               T Z0, T Y1, T Z1, T YY, T YZ, T ZZ) {
+  const T half = static_cast<T>(0.5), o = rec.o;
+  const T *q = rec.q;
+  const T v[10] = {o * (q[0] * T1 + q[1] * Y0 + q[2] * Z0),
+                   o * (q[3] * Y0 + q[4] * Z0 + q[1] * T1),
+                   o * (q[5] * Z0 + q[4] * Y0 + q[2] * T1),
+                   -half * o * T2,
+                   -o * Y1,
+                   -o * Z1,
+                   -half * o * YY,
+                   -o * YZ,
+                   -half * o * ZZ,
+                   T0};
+  store_row(rows, e, v);
+}
+
+// One record's sums over the voxels of its brick inside the volume, one
+// voxel at a time (rare: see voxel_bwd_chunk_kernel's `apart`).
+// The record is loaded again, so that it need not stay in registers.
+template <typename T>
+__device__ __forceinline__ void voxel_sums_apart(const T *__restrict__ means3d,
+                                                 const T *__restrict__ conics,
+                                                 const T *__restrict__ opac, int64_t g, int64_t N,
+                                                 const Brick &b, const T *__restrict__ v_vol,
+                                                 int64_t plane, uint32_t D2, T &T0, T &T1, T &T2,
+                                                 T &Y0, T &Z0, T &Y1, T &Z1, T &YY, T &YZ, T &ZZ) {
+  const T half = static_cast<T>(0.5);
+  BwdRecord<T> rec;
+  load_bwd_record_plain(means3d, conics, opac, g, N, true, b, rec);
+  const T dx0 = (static_cast<T>(b.ok) + half) - rec.m[0];
+#pragma unroll 1
+  for (int q = 0; q < b.ni * b.nj * b.nk; ++q) {
+    const int k = q % b.nk, j = b.oj + q / b.nk % b.nj, i = b.oi + q / b.nk / b.nj;
+    const T dx = dx0 + static_cast<T>(k);
+    const T dy = (static_cast<T>(j) + half) - rec.m[1];
+    const T dz = (static_cast<T>(i) + half) - rec.m[2];
+    const T B = fma(rec.h[1], dy, rec.h[2] * dz);
+    const T C = fma(fma(rec.h[3], dy, rec.h[4] * dz), dy, rec.h[5] * dz * dz);
+    const T sl = fma(fma(rec.h[0], dx, B), dx, C);
+    if (!alpha_pass(sl, rec.lim)) continue;
+    const T w = v_vol[i * plane + static_cast<int64_t>(j) * D2 + b.ok + k] * neg_exp2(sl);
+    T0 += w;
+    T1 = fma(w, dx, T1);
+    T2 = fma(w * dx, dx, T2);
+    Y0 = fma(w, dy, Y0);
+    Z0 = fma(w, dz, Z0);
+    Y1 = fma(w * dx, dy, Y1);
+    Z1 = fma(w * dx, dz, Z1);
+    YY = fma(w * dy, dy, YY);
+    YZ = fma(w * dy, dz, YZ);
+    ZZ = fma(w * dz, dz, ZZ);
+  }
+}
+
 // ------------------------------------------- chunked backward (rows) ---
 //
 // A wave of 64 records walks the union of its lanes' reached rows, which is
@@ -697,25 +825,38 @@ __global__ __launch_bounds__(kBwdThreads) void voxel_bwd_kernel(
 // once per chunk index, and the chunk sums are added to the record's LDS
 // accumulators one chunk index at a time in increasing order, so each
 // record's chunks add in index order and the result does not depend on
-// scheduling.  Every brick must lie inside
-// the volume with 16-byte gradient rows, the gradient volume must span at
-// most 2^32 bytes and a slice fewer than 2^24 (the caller checks).
+// scheduling.
+//
+// The lanes of a step read the gradient rows of different records: loaded
+// from memory, 64 lanes times 32 bytes through the vector cache's return path
+// each step, that path was busy 92-98 % of the kernel's time.  A block
+// therefore stages its bricks' gradients in LDS when its records lie in at
+// most kStageBricks consecutive bricks, zero beyond the volume, so that
+// ragged volumes walk like any other.  Blocks over more bricks (short lists)
+// read rows from memory, element by element at the volume's ragged ends.
+// Six bricks and the other arrays take 28 KB, which with 96 VGPRs keeps five
+// waves per SIMD: 0.399 -> 0.381 ms for 3.2 M records of a 256^3 volume, 5.49
+// -> 5.30 ms for 39 M of a 512^3 one; a 250 x 201 x 173 volume of 100k
+// Gaussians, which took the masked walk of voxel_bwd_kernel before, went from
+// 449 to 374 us forward and backward.  The records' fields reach the lanes
+// that walk them by lane shuffles from the registers of the lanes that loaded
+// them; staged in LDS (39 KB, four waves) the rows pass took 0.397 ms.
 
 constexpr int kChunkRows = 8;
 constexpr int kChunkWaves = 4;
+constexpr uint32_t kStageBricks = 6;
 // A chunked item costs about 1.3 times a row of the dense walk (indexing,
 // the walk, the chunk sums), so a wave whose records reach more than this
 // many of their 64 x 64 (record, row) pairs takes the dense walk instead
 // (large footprints, e.g. the binary-tree model on a 128^3 volume).
 constexpr int kDenseItems = 3072;
 
-template <typename T>
-struct ChunkRecord {
-  T c[3];  // the brick's first voxel centre minus the mean (x, y, z)
-  T h[6];
-  typename Bits<T>::type lim;  // 0 for dead records
-  uint32_t brick0;             // byte offset of the brick's first voxel in v_vol
-};
+__device__ __forceinline__ uint32_t shfl_bits(uint32_t v, int src) {
+  return static_cast<uint32_t>(__shfl(static_cast<int>(v), src, 64));
+}
+__device__ __forceinline__ uint64_t shfl_bits(uint64_t v, int src) {
+  return static_cast<uint64_t>(__shfl(static_cast<long long>(v), src, 64));
+}
 
 // Chunks of one chunked wave: its records reach at most kDenseItems rows, in
 // chunks of up to kChunkRows, at most one short chunk per record.
@@ -725,25 +866,26 @@ constexpr int kMaxChunks = kDenseItems / kChunkRows + 64;
 // over the same lists, voxel_fwd_reach_kernel) instead of the culling
 // setup and the per-slice row ranges.
 template <typename T, bool kGiven>
-__global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
+__global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
     const T *__restrict__ means3d, const T *__restrict__ conics, const T *__restrict__ opac,
     const int32_t *__restrict__ tile_offsets, const int64_t *__restrict__ isect_ids,
     const int32_t *__restrict__ flatten_ids, const int32_t *__restrict__ isect_src,
     int64_t n_isects, uint32_t n_keys, uint32_t koff, int64_t N, const T *__restrict__ v_vol,
-    uint32_t D2, uint32_t D1, uint32_t D0, uint32_t n2, uint32_t n1, T *__restrict__ rows,
-    const uint64_t *__restrict__ reach) {
+    uint32_t D2, uint32_t D1, uint32_t D0, uint32_t n2, uint32_t n1, bool vec,
+    T *__restrict__ rows, const uint64_t *__restrict__ reach) {
   constexpr int R = kChunkRows;
+  constexpr uint32_t kBrick = R * R * R;
   using Q = typename Quad<T>::type;
   constexpr int kq = Quad<T>::n;
-  __shared__ WordMajor<ChunkRecord<T>, 64> s_rec[kChunkWaves];
   __shared__ uint64_t s_rows[kChunkWaves][64];  // reached rows: bit 8 * slice + row
   __shared__ T s_acc[kChunkWaves][10][64];
   // Chunk entries: record lane | first row << 6 | chunk index << 12.
   __shared__ uint16_t s_chunk[kChunkWaves][kMaxChunks];
+  __shared__ uint32_t s_key_min[kChunkWaves], s_key_max[kChunkWaves];
+  __shared__ __align__(16) T s_v[kStageBricks * kBrick];
   const uint32_t w = wave_index(), lane = lane_id();
   const int64_t rb = static_cast<int64_t>(xcd_swizzle(blockIdx.x, gridDim.x)) *
                          (64 * kChunkWaves) + 64 * static_cast<int64_t>(w);
-  if (rb >= n_isects) return;  // uniform per wave; the waves share no barrier
   const int64_t r = rb + lane;
   const bool in_list = r < n_isects;
   uint32_t key;
@@ -752,13 +894,49 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
   // fewer before the record's own loads).
   const int32_t fid = in_list ? flatten_ids[r] : -1;
   const uint64_t reach_r = kGiven && in_list ? reach[r] : 0ull;
-  if (isect_ids != nullptr) {
+  if (rb >= n_isects) {  // uniform per wave: no records, only its share of the staging
+    key_ok = false;
+    key = 0;
+  } else if (isect_ids != nullptr) {
     const int64_t k = in_list ? isect_ids[r] : 0;
     key_ok = key_ok && k >= 0 && k < static_cast<int64_t>(n_keys);
     key = key_ok ? static_cast<uint32_t>(k) : 0u;
   } else {
     key = wave_record_key(tile_offsets, n_keys, n_isects, rb, r);
   }
+  const uint32_t k_min = wave_min(key_ok ? key : 0xffffffffu);
+  const uint32_t k_max = wave_max(key_ok ? key : 0u);
+  if (lane == 0) {
+    s_key_min[w] = k_min;
+    s_key_max[w] = k_max;
+  }
+  __syncthreads();
+  uint32_t key0 = s_key_min[0], key1 = s_key_max[0];
+#pragma unroll
+  for (uint32_t ww = 1; ww < kChunkWaves; ++ww) {
+    key0 = min(key0, s_key_min[ww]);
+    key1 = max(key1, s_key_max[ww]);
+  }
+  if (key0 > key1) return;  // uniform over the block: no record in range
+  const int64_t plane = static_cast<int64_t>(D1) * D2;
+  const bool staged = key1 - key0 < kStageBricks;
+  if (staged) {
+    for (uint32_t k = key0; k <= key1; ++k) {
+      const Brick sb = brick_of(k + koff, n2, n1, R, D2, D1, D0);
+      const T *__restrict__ src = v_vol + sb.oi * plane + static_cast<int64_t>(sb.oj) * D2 + sb.ok;
+#pragma unroll
+      for (uint32_t h = 0; h < kBrick; h += 64 * kChunkWaves) {
+        const int q = static_cast<int>(h + threadIdx.x);
+        const int i = q >> 6, j = (q >> 3) & 7, c = q & 7;
+        s_v[(k - key0) * kBrick + static_cast<uint32_t>(q)] =
+            (i < sb.ni && j < sb.nj && c < sb.nk) ? src[i * plane + static_cast<int64_t>(j) * D2 + c]
+                                                  : static_cast<T>(0);
+      }
+    }
+    __syncthreads();
+  }
+  if (rb >= n_isects) return;  // uniform per wave; no barrier follows
+  if (!key_ok) key = key0;
   const int64_t g = key_ok ? static_cast<int64_t>(fid) : -1;
   const Brick b = brick_of(key + koff, n2, n1, R, D2, D1, D0);
   BwdRecord<T> rec;
@@ -766,10 +944,13 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
     load_bwd_record_plain(means3d, conics, opac, g, N, key_ok, b, rec);
   else
     load_bwd_record(means3d, conics, opac, g, N, key_ok, b, rec);
+  // A record whose sigma may be NaN passes the alpha test there whatever the
+  // gradient: in a ragged brick, where the walk below also evaluates columns
+  // beyond the volume, it is summed apart, voxel by voxel.
+  const bool apart = rec.live && rec.lim == Bits<T>::kSign &&
+                     (b.ni < R || b.nj < R || b.nk < R);
+  if (apart) rec.live = false;
   const T half = static_cast<T>(0.5);
-  const uint32_t plane = D1 * D2;  // the caller checks D2 D1 D0 sizeof(T) <= 2^32
-  const uint32_t plane_b = plane * static_cast<uint32_t>(sizeof(T)),
-                 row_b = D2 * static_cast<uint32_t>(sizeof(T));
   const T dx0 = (static_cast<T>(b.ok) + half) - rec.m[0];
 
   // The record's reached rows; the items are its set bits in increasing order.
@@ -779,43 +960,35 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
   else
     reached = reach_mask(rec, b, dx0);
   const int n_items = __popcll(reached);
-  if (wave_sum(n_items) > kDenseItems) {  // uniform per wave
+  // Whole bricks with 16-byte rows: a row is read as vectors.
+  const bool whole =
+      staged || (vec && ballot(b.ni < R || b.nj < R || b.nk < R) == 0);
+  if (whole && wave_sum(n_items) > kDenseItems) {  // uniform per wave
     T T0 = 0, T1 = 0, T2 = 0, Y0 = 0, Z0 = 0, Y1 = 0, Z1 = 0, YY = 0, YZ = 0, ZZ = 0;
-    if (ballot(rec.live) != 0)
-      voxel_brick_full<T, R, true>(rec, b, v_vol, static_cast<int64_t>(plane), D2, dx0, T0, T1,
-                                   T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ, reached);
-    if (!key_ok) return;
-    const T o = rec.o;
-    const T *qc = rec.q;
-    const T v[10] = {o * (qc[0] * T1 + qc[1] * Y0 + qc[2] * Z0),
-                     o * (qc[3] * Y0 + qc[4] * Z0 + qc[1] * T1),
-                     o * (qc[5] * Z0 + qc[4] * Y0 + qc[2] * T1),
-                     -half * o * T2,
-                     -o * Y1,
-                     -o * Z1,
-                     -half * o * YY,
-                     -o * YZ,
-                     -half * o * ZZ,
-                     T0};
-    store_row(rows, isect_src[r], v);
+    if (ballot(rec.live) != 0) {
+      if (staged)
+        voxel_brick_full<T, R, true>(rec, b, s_v + (key - key0) * kBrick, R * R, R, dx0, T0, T1,
+                                     T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ, reached);
+      else
+        voxel_brick_full<T, R, true>(rec, b,
+                                     v_vol + b.oi * plane + static_cast<int64_t>(b.oj) * D2 + b.ok,
+                                     plane, D2, dx0, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ,
+                                     reached);
+    }
+    if (apart)
+      voxel_sums_apart(means3d, conics, opac, g, N, b, v_vol, plane, D2, T0, T1, T2, Y0, Z0, Y1,
+                       Z1, YY, YZ, ZZ);
+    if (key_ok)
+      store_partials(rows, isect_src[r], rec, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
     return;
   }
-  {
-    ChunkRecord<T> cr;
-    cr.c[0] = dx0;
-    cr.c[1] = (static_cast<T>(b.oj) + half) - rec.m[1];
-    cr.c[2] = (static_cast<T>(b.oi) + half) - rec.m[2];
+  // The brick's first voxel centre minus the mean.
+  const T c1 = (static_cast<T>(b.oj) + half) - rec.m[1];
+  const T c2 = (static_cast<T>(b.oi) + half) - rec.m[2];
+  const typename Bits<T>::type my_lim = rec.live ? rec.lim : 0;
+  s_rows[w][lane] = reached;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) cr.h[c] = rec.h[c];
-    cr.lim = rec.live ? rec.lim : 0;
-    // Below 2^32: the caller checks D2 D1 D0 sizeof(T) <= 2^32.
-    cr.brick0 = (static_cast<uint32_t>(b.oi) * plane + static_cast<uint32_t>(b.oj) * D2 +
-                 static_cast<uint32_t>(b.ok)) * static_cast<uint32_t>(sizeof(T));
-    s_rec[w].store(static_cast<int>(lane), cr);
-    s_rows[w][lane] = reached;
-#pragma unroll
-    for (int c = 0; c < 10; ++c) s_acc[w][c][lane] = 0;
-  }
+  for (int c = 0; c < 10; ++c) s_acc[w][c][lane] = 0;
   // Chunk list: the full chunks in (chunk index, record) order, then each
   // record's short last chunk, longest first, so that the rounds of short
   // chunks take as many steps as their longest.  Each record's chunks keep
@@ -878,7 +1051,16 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
     const bool act = ci < n_list;
     const uint32_t ent = act ? static_cast<uint32_t>(s_chunk[w][ci]) : 0u;
     const uint32_t rl = ent & 63u, pos = (ent >> 6) & 63u, q = ent >> 12;
-    const ChunkRecord<T> cr = s_rec[w].load(static_cast<int>(rl));
+    // The record, from the registers of the lane that loaded it (every lane
+    // takes part); the conic scaled as scaled_conic does.
+    const int src = static_cast<int>(rl);
+    T qr[6], hr[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) qr[c] = __shfl(rec.q[c], src, 64);
+    scaled_conic(qr, hr);
+    const T cx = __shfl(dx0, src, 64), cy = __shfl(c1, src, 64), cz = __shfl(c2, src, 64);
+    const typename Bits<T>::type r_lim = shfl_bits(my_lim, src);
+    const uint32_t r_key = static_cast<uint32_t>(__shfl(static_cast<int>(key), src, 64));
     const uint64_t rows_m = s_rows[w][rl];
     const int n_here =
         act ? min(R, __popcll(rows_m) - static_cast<int>(q) * R) : 0;
@@ -888,9 +1070,17 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
     T dxk[R], wk[R];
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      dxk[k] = cr.c[0] + static_cast<T>(k);
+      dxk[k] = cx + static_cast<T>(k);
       wk[k] = 0;
     }
+    // The brick's gradient: staged, or in the volume.
+    Brick bb = {};
+    const T *__restrict__ vb = v_vol;
+    if (!staged) {
+      bb = brick_of(r_key + koff, n2, n1, R, D2, D1, D0);
+      vb += bb.oi * plane + static_cast<int64_t>(bb.oj) * D2 + bb.ok;
+    }
+    const uint32_t sv = staged ? (r_key - key0) * kBrick : 0u;
     T Y0 = 0, Z0 = 0, Y1 = 0, Z1 = 0, YY = 0, YZ = 0, ZZ = 0;
     // The round's longest chunk is its first (lane 0 is always active).
     const int steps = __builtin_amdgcn_readfirstlane(n_here);
@@ -898,40 +1088,53 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
     for (int st = 0; st < steps; ++st) {
       const bool item = st < n_here;
       // The next row (bit 63 when none is left: a step without an item
-      // still reads a row of the record's own brick, which lies inside the
-      // volume, and tests against a zero limit).
+      // still reads a row of the record's own brick and tests against a zero
+      // limit).
       const uint32_t p = static_cast<uint32_t>(__builtin_ctzll(rest | (1ull << 63)));
       rest &= rest - 1ull;
       const uint32_t li = p >> 3, lj = p & 7u;
       // The row centre's offsets from the mean as the columns' (dxk): the
       // brick corner's offset plus the row's index in the brick.
-      const T dz = static_cast<T>(li) + cr.c[2];
-      const T dy = static_cast<T>(lj) + cr.c[1];
-      const T B = fma(cr.h[1], dy, cr.h[2] * dz);
-      const T C = fma(fma(cr.h[3], dy, cr.h[4] * dz), dy, cr.h[5] * dz * dz);
-      const typename Bits<T>::type lim = item ? cr.lim : 0;
-      // 32-bit byte offsets: li, lj < 8 and plane_b = D1 D2 sizeof(T) < 2^24
-      // (the caller checks), so two full-rate 24-bit multiply-adds per row.
-      uint32_t off = __umul24(lj, row_b) + cr.brick0;
-      asm volatile("" : "+v"(off));  // two multiply-adds, not two products and a sum
-      off += __umul24(li, plane_b);
-      const T *__restrict__ vrow =
-          reinterpret_cast<const T *>(reinterpret_cast<const char *>(v_vol) + off);
+      const T dz = static_cast<T>(li) + cz;
+      const T dy = static_cast<T>(lj) + cy;
+      const T B = fma(hr[1], dy, hr[2] * dz);
+      const T C = fma(fma(hr[3], dy, hr[4] * dz), dy, hr[5] * dz * dz);
+      typename Bits<T>::type lim = item ? r_lim : 0;
+      asm volatile("" : "+v"(lim));  // one select, not a scalar AND per voxel
       T vv[R];
+      if (staged) {
+        const T *vrow = s_v + (sv + p * R);
 #pragma unroll
-      for (int c = 0; c < R / kq; ++c)
-        *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
+        for (int c = 0; c < R / kq; ++c)
+          *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
+      } else {
+        const T *__restrict__ vrow = vb + (li * plane + static_cast<int64_t>(lj) * D2);
+        if (whole) {
+#pragma unroll
+          for (int c = 0; c < R / kq; ++c)
+            *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
+        } else {
+          // Columns beyond the volume read zero; the rows and slices beyond
+          // it are reached by no record, only by a step without an item.
+          const int n = static_cast<int>(li) < bb.ni && static_cast<int>(lj) < bb.nj ? bb.nk : 0;
+#pragma unroll
+          for (int k = 0; k < R; ++k) vv[k] = k < n ? vrow[k] : static_cast<T>(0);
+        }
+      }
       T s0 = 0, s1 = 0;
+      T sl[R], e[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) sl[k] = fma(fma(hr[0], dxk[k], B), dxk[k], C);
+      neg_exp2_run(sl, e);
 #pragma unroll
       for (int k = 0; k < R; ++k) {
         const T dx = dxk[k];
-        const T slv = fma(fma(cr.h[0], dx, B), dx, C);
         // A failing voxel adds an exact zero whatever its upstream gradient
         // (a non-finite one included), as when the voxel is skipped.  The
         // product is formed unconditionally: as an operand of the
         // conditional it would become a branch around its load and exp.
-        const T p = vv[k] * neg_exp2(slv);
-        const T wv = alpha_pass(slv, lim) ? p : static_cast<T>(0);
+        const T p = vv[k] * e[k];
+        const T wv = alpha_pass(sl[k], lim) ? p : static_cast<T>(0);
         wk[k] += wv;
         s0 += wv;
         s1 = fma(wv, dx, s1);
@@ -976,23 +1179,12 @@ __global__ __launch_bounds__(64 * kChunkWaves) void voxel_bwd_chunk_kernel(
   T a[10];
 #pragma unroll
   for (int c = 0; c < 10; ++c) a[c] = s_acc[w][c][lane];
-  const T T0 = a[0], T1 = a[1], T2 = a[2], Y0 = a[3], Z0 = a[4], Y1 = a[5], Z1 = a[6],
-          YY = a[7], YZ = a[8], ZZ = a[9];
-  // Per-voxel terms of VoxelizeToVoxelsBwd.cu:409-421 summed over the brick,
-  // as in voxel_bwd_kernel.
-  const T o = rec.o;
-  const T *qc = rec.q;
-  const T v[10] = {o * (qc[0] * T1 + qc[1] * Y0 + qc[2] * Z0),
-                   o * (qc[3] * Y0 + qc[4] * Z0 + qc[1] * T1),
-                   o * (qc[5] * Z0 + qc[4] * Y0 + qc[2] * T1),
-                   -half * o * T2,
-                   -o * Y1,
-                   -o * Z1,
-                   -half * o * YY,
-                   -o * YZ,
-                   -half * o * ZZ,
-                   T0};
-  store_row(rows, isect_src[r], v);
+  if (apart)
+    voxel_sums_apart(means3d, conics, opac, static_cast<int64_t>(flatten_ids[r]), N,
+                     brick_of(key + koff, n2, n1, R, D2, D1, D0), v_vol, plane, D2, a[0], a[1],
+                     a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9]);
+  store_partials(rows, isect_src[r], rec, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8],
+                 a[9]);
 }
 
 // n0 brick layers of lists from layer z0 on (the whole grid: z0 = 0 and
@@ -1170,21 +1362,16 @@ int voxel_bwd_impl(const T *means3d, const T *conics, const T *opac,
   launch_voxel_bwd<T, RR, EXACT>(means3d, conics, opac, tile_offsets, isect_ids, flatten_ids,  \
                                  isect_src, n_isects, n_keys, koff, N, v_vol, D2, D1, D0, ts,  \
                                  n2, n1, vec, v_means, v_conics, v_opac, rows, stream)
-  // The chunked walk addresses the gradient with 32-bit byte offsets and
-  // 24-bit plane and row strides.
-  const int64_t elem = static_cast<int64_t>(sizeof(T));
-  if (ts == 8 && rows != nullptr && vec && D2 % 8 == 0 && D1 % 8 == 0 && D0 % 8 == 0 &&
-      n_vox * elem <= (int64_t{1} << 32) &&
-      static_cast<int64_t>(D1) * D2 * elem < (int64_t{1} << 24)) {
+  if (ts == 8 && rows != nullptr) {
     const dim3 grid(static_cast<uint32_t>(ceil_div(n_isects, 64 * kChunkWaves)));
     if (reach != nullptr)
       voxel_bwd_chunk_kernel<T, true><<<grid, dim3(64 * kChunkWaves), 0, stream>>>(
           means3d, conics, opac, tile_offsets, isect_ids, flatten_ids, isect_src, n_isects,
-          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, rows, reach);
+          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, vec, rows, reach);
     else
       voxel_bwd_chunk_kernel<T, false><<<grid, dim3(64 * kChunkWaves), 0, stream>>>(
           means3d, conics, opac, tile_offsets, isect_ids, flatten_ids, isect_src, n_isects,
-          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, rows, nullptr);
+          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, vec, rows, nullptr);
   } else if (ts == 8)
     R2S_VOXEL_BWD_R(8, true);
   else if (ts == 4)

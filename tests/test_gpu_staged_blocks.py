@@ -1,15 +1,17 @@
-"""The backward blocks that stage their tiles' upstream gradient in LDS, beside
-those whose records span too many tiles for it, on ragged and whole images:
-against the oracle at the usual bar (tests/helpers.py)."""
+"""The backward blocks that stage their tiles' (bricks') upstream gradient in
+LDS, beside those whose records span too many tiles for it, on ragged and
+whole images (volumes), and the voxel forward that walks every row of large
+footprints: against the oracle at the usual bar (tests/helpers.py)."""
 
 from __future__ import annotations
 
 import pytest
 import torch
 
-from helpers import check_raster, np32, raster_references
+from helpers import check_raster, check_voxel, np32, raster_references, voxel_references
+from r2splat.cuda import _ops
 from r2splat.cuda import _wrapper as W
-from test_gpu_ops import DEV, _raster_case
+from test_gpu_ops import DEV, _raster_case, _voxel_case
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +38,53 @@ def test_raster_backward_blocks(dtype, n, shape, views, staged):
                                                  H_img, 16, True)
     for name, r in check_raster(refs, grads=[np32(t) for t in got]).items():
         print(name, r)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,dims,log_mu,staged", [
+    (2500, (30, 20, 26), -3.2, True),   # ragged
+    (2500, (29, 21, 9), -1.6, True),    # ragged, waves that walk every row
+    (60, (90, 61, 77), -3.4, False),    # ragged, sparse bricks
+    (60, (96, 64, 80), -3.4, False),    # whole, sparse bricks
+    (5, (7, 3, 5), -3.2, True),         # one partial brick
+])
+def test_voxel_backward_blocks(dtype, n, dims, log_mu, staged):
+    d, m3, con, ids, fl, off = _voxel_case(n, 4, dims, 8, dtype, log_mu=log_mu)
+    blocks = [int(b.max() - b.min()) + 1 for b in ids.split(256)]
+    assert (min(blocks) <= 6) == staged, blocks
+    op = d["opac"]
+    vol = W.voxelize_to_voxels_fwd(m3, con, op, off, fl, *dims, 8)
+    v = torch.randn(vol.shape, generator=d["gen"], dtype=dtype)
+    refs = voxel_references(np32(m3), np32(con), np32(op), np32(off), np32(fl), *dims, 8,
+                            v_volume=v.numpy())
+    print("volume", check_voxel(refs, volume=np32(vol)))
+    vol_r, reach = _ops.voxelize_with_reach(m3, con, op, off, fl, *dims)
+    assert torch.equal(vol, vol_r)
+    plain = W.voxelize_to_voxels_bwd_per_gaussian(m3, con, op, off, ids, fl, v.to(DEV), *dims, 8)
+    for name, r in check_voxel(refs, grads=[np32(t) for t in plain]).items():
+        print(name, r)
+    n2, n1, n0 = (-(-x // 8) for x in dims)
+    lists = _ops.TileLists(None, ids, fl, *_ops.emission_order(fl, n2 * n1 * n0), off)
+    given = _ops.voxel_backward(m3, con, op, off, lists, v.to(DEV), *dims, 8, reach=reach)
+    for a, b in zip(plain, given):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dims", [(30, 20, 26), (32, 24, 32)])
+def test_non_finite_record_in_a_ragged_brick(dims):
+    """A record with a non-finite conic passes the alpha test wherever its sigma is NaN or
+    infinite: its own gradients are those of the one-pass kernel (NaN where they are), and
+    no other Gaussian's change."""
+    d, m3, con, ids, fl, off = _voxel_case(400, 6, dims, 8)
+    op, bad = d["opac"], int(fl[fl.numel() // 2])
+    v = torch.randn((dims[2], dims[1], dims[0]), generator=d["gen"]).to(DEV)
+    clean = W.voxelize_to_voxels_bwd_per_gaussian(m3, con, op, off, ids, fl, v, *dims, 8)
+    con2 = con.clone()
+    con2[bad, 3] = float("inf")
+    got = W.voxelize_to_voxels_bwd_per_gaussian(m3, con2, op, off, ids, fl, v, *dims, 8)
+    one_pass = W.voxelize_to_voxels_bwd_per_gaussian(m3, con2, op, off, ids, fl.clone(), v, *dims,
+                                                     8)
+    others = torch.arange(m3.shape[0], device=DEV) != bad
+    for a, b, c in zip(got, clean, one_pass):
+        assert torch.equal(a[others], b[others])
+        assert torch.equal(torch.isnan(a[bad]), torch.isnan(c[bad]))
