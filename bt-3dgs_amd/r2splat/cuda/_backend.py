@@ -17,7 +17,7 @@ import torch
 
 from ._lib import LIB_PATH, load
 
-__all__ = ["_C", "is_cuda_available", "library"]
+__all__ = ["_C", "is_cuda_available", "library", "operators"]
 
 
 class _LazyModule:
@@ -46,16 +46,22 @@ class _LazyModule:
             self._module = None
 
     def __getattr__(self, name: str):
-        self._try_load()
+        return getattr(self.module(), name)
+
+    def module(self):
         if self._module is None:
-            raise RuntimeError(f"r2splat HIP library is unavailable: {self._error}")
-        return getattr(self._module, name)
+            self._try_load()
+            if self._module is None:
+                raise RuntimeError(f"r2splat HIP library is unavailable: {self._error}")
+        return self._module
 
     def is_available(self) -> bool:
         self._try_load()
         return self._module is not None
 
     def library(self) -> ctypes.CDLL:
+        if self._lib is not None:
+            return self._lib
         self._try_load()
         if self._lib is None:
             raise RuntimeError(f"r2splat HIP library is unavailable: {self._error}")
@@ -78,6 +84,12 @@ _C = _CProxy()
 
 def is_cuda_available() -> bool:
     return _lazy_C.is_available()
+
+
+def operators():
+    """The tensor operators' module, as ``_C`` forwards to it (raises
+    RuntimeError if the library is unavailable)."""
+    return _lazy_C.module()
 
 
 def library() -> ctypes.CDLL:

@@ -10,8 +10,10 @@ no CPU fallback: without the library every call raises ``RuntimeError``.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
+import struct
 import threading
 import warnings
 from typing import NamedTuple, Optional, Tuple
@@ -29,6 +31,10 @@ def _lib():
     return _backend.library()
 
 
+def _is_input(t) -> bool:
+    return isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous()
+
+
 def _check_input(t: Tensor, name: str) -> None:
     # common.h:25-30 R2SPLAT_CHECK_INPUT
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
@@ -37,9 +43,16 @@ def _check_input(t: Tensor, name: str) -> None:
         raise RuntimeError(f"{name} must be contiguous")
 
 
+def _fail(*msg) -> None:
+    raise RuntimeError("".join(str(m) for m in msg))
+
+
+# For messages that are constants.  A message made from a tensor's shape or a
+# name is written under an `if`, so that a call that passes does not format it:
+# that text was a third of the host time of the smallest calls.
 def _check(cond: bool, *msg) -> None:
     if not cond:
-        raise RuntimeError("".join(str(m) for m in msg))
+        _fail(*msg)
 
 
 def _suffix(t: Tensor, op: str) -> str:
@@ -65,6 +78,17 @@ def _stream(device: torch.device):
         idx = device.index if device.index is not None else torch.cuda.current_device()
         return _RAW_STREAM(idx)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """torch.cuda.device(device), or nothing to switch when the calling thread
+    is on that device already (0.4 us instead of 3 us of host time)."""
+    if device.index == torch._C._cuda_getDevice():
+        return _HERE
+    return torch.cuda.device(device)
 
 
 _FUNCS = {}  # entry point name -> (library, its ctypes function)
@@ -111,6 +135,20 @@ _COUNT_HISTORY_LEN = 8
 _PINNED_COUNT = threading.local()  # per host thread: a count read back by one call at a time
 
 
+def _count_readback(dev: torch.device):
+    """This thread's (pinned 0-d int64 tensor, the same word as a ctypes
+    integer, event) for reading a count back from ``dev``."""
+    by_device = getattr(_PINNED_COUNT, "by_device", None)
+    if by_device is None:
+        by_device = _PINNED_COUNT.by_device = {}
+    entry = by_device.get(dev.index)
+    if entry is None:
+        host = torch.empty((), dtype=torch.int64, pin_memory=True)
+        entry = by_device[dev.index] = (host, ctypes.c_int64.from_address(host.data_ptr()),
+                                        torch.cuda.Event())
+    return entry
+
+
 def _note_count(key, n: int) -> None:
     hist = _COUNT_HISTORY.setdefault(key, [])
     hist.append(n)
@@ -149,18 +187,12 @@ def _emit_and_sort(launch, offsets: Tensor, n_items: int, n_keys: int, op: str,
             # caller's limit; a longer one falls through to the check below.
             cap = min(cap, max_records)
         outs, ws = alloc(cap)
-        pinned = getattr(_PINNED_COUNT, "by_device", None)
-        if pinned is None:
-            pinned = _PINNED_COUNT.by_device = {}
-        host = pinned.get(dev.index)
-        if host is None:
-            host = pinned[dev.index] = torch.empty(1, dtype=torch.int64, pin_memory=True)
-        host.copy_(offsets[n_items:n_items + 1], non_blocking=True)
-        ready = torch.cuda.Event()
+        host, value, ready = _count_readback(dev)
+        host.copy_(offsets[n_items], non_blocking=True)
         ready.record()
         launch(cap, end_bit, outs, ws)
         ready.synchronize()
-        n = int(host[0])
+        n = value.value
         _note_count(key, n)
         if n <= cap:
             return None if n == 0 else tuple(None if t is None else t[:n] for t in outs)
@@ -213,6 +245,12 @@ class TileLists(NamedTuple):
         if self.keys is not None:
             return self.keys
         return keys_from_offsets(self.tile_offsets, self.flatten_ids.numel())
+
+
+def _no_records(tiles_per_gauss: Tensor) -> TileLists:
+    dev = tiles_per_gauss.device
+    return TileLists(tiles_per_gauss, torch.empty((0,), dtype=torch.int64, device=dev),
+                     torch.empty((0,), dtype=torch.int32, device=dev), None, None)
 
 
 # The reference's operator signatures (isect_tiles -> rasterize_to_pixels_bwd*)
@@ -270,20 +308,20 @@ def parameter_transform_fwd(quats: Tensor, scale_ori: Tensor, scale_min: float,
     """ParameterTransform.cpp:34-84 -> (covars [N,6], max_scales [N])."""
     _check_input(quats, "quats")
     _check_input(scale_ori, "scale_ori")
-    _check(quats.dim() == 2 and quats.size(1) == 4,
-           "quats must be 2D [N, 4], got shape ", list(quats.shape))
-    _check(scale_ori.dim() == 2 and scale_ori.size(1) == 3,
-           "scale_ori must be 2D [N, 3], got shape ", list(scale_ori.shape))
+    if not (quats.dim() == 2 and quats.size(1) == 4):
+        _fail("quats must be 2D [N, 4], got shape ", list(quats.shape))
+    if not (scale_ori.dim() == 2 and scale_ori.size(1) == 3):
+        _fail("scale_ori must be 2D [N, 3], got shape ", list(scale_ori.shape))
     N = quats.size(0)
-    _check(scale_ori.size(0) == N, "scale_ori batch dim (", scale_ori.size(0),
-           ") doesn't match quats N=", N)
+    if scale_ori.size(0) != N:
+        _fail("scale_ori batch dim (", scale_ori.size(0), ") doesn't match quats N=", N)
     covars = torch.empty((N, 6), dtype=quats.dtype, device=quats.device)
     max_scales = torch.empty((N,), dtype=quats.dtype, device=quats.device)
     if N == 0:
         return covars, max_scales
     _check(scale_ori.dtype == quats.dtype, "quats and scale_ori must share a dtype")
     sfx = _suffix(quats, "parameter_transform_fwd")
-    with torch.cuda.device(quats.device):
+    with _on(quats.device):
         _call(f"r2s_parameter_transform_fwd_{sfx}", _ptr(quats), _ptr(scale_ori),
               float(scale_min), float(scale_max), _ptr(covars), _ptr(max_scales), N,
               _stream(quats.device))
@@ -307,7 +345,7 @@ def parameter_transform_bwd(quats: Tensor, scale_ori: Tensor, scale_min: float,
     _check(scale_ori.dtype == quats.dtype and v_covars.dtype == quats.dtype,
            "quats, scale_ori and v_covars must share a dtype")
     sfx = _suffix(quats, "parameter_transform_bwd")
-    with torch.cuda.device(quats.device):
+    with _on(quats.device):
         _call(f"r2s_parameter_transform_bwd_{sfx}", _ptr(quats), _ptr(scale_ori),
               float(scale_min), float(scale_max), _ptr(v_covars), _ptr(v_quats), _ptr(v_scale),
               N, _stream(quats.device))
@@ -319,13 +357,13 @@ def prepare_gaussians(quats: Tensor, raw_scales: Tensor, raw_opacities: Tensor,
     """Fused parameter_transform_fwd + softplus (r2splat/ops/direct.py:85-91)."""
     for t, n in ((quats, "quats"), (raw_scales, "scale_ori"), (raw_opacities, "raw_opacities")):
         _check_input(t, n)
-    _check(quats.dim() == 2 and quats.size(1) == 4,
-           "quats must be 2D [N, 4], got shape ", list(quats.shape))
-    _check(raw_scales.dim() == 2 and raw_scales.size(1) == 3,
-           "scale_ori must be 2D [N, 3], got shape ", list(raw_scales.shape))
+    if not (quats.dim() == 2 and quats.size(1) == 4):
+        _fail("quats must be 2D [N, 4], got shape ", list(quats.shape))
+    if not (raw_scales.dim() == 2 and raw_scales.size(1) == 3):
+        _fail("scale_ori must be 2D [N, 3], got shape ", list(raw_scales.shape))
     N = quats.size(0)
-    _check(raw_scales.size(0) == N, "scale_ori batch dim (", raw_scales.size(0),
-           ") doesn't match quats N=", N)
+    if raw_scales.size(0) != N:
+        _fail("scale_ori batch dim (", raw_scales.size(0), ") doesn't match quats N=", N)
     _check(raw_opacities.dim() == 1 and raw_opacities.size(0) == N,
            "raw_opacities must be 1D [N]")
     _check(raw_scales.dtype == quats.dtype and raw_opacities.dtype == quats.dtype,
@@ -337,7 +375,7 @@ def prepare_gaussians(quats: Tensor, raw_scales: Tensor, raw_opacities: Tensor,
     if N == 0:
         return covars, max_scales, opac
     sfx = _suffix(quats, "prepare_gaussians")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_prepare_gaussians_{sfx}", _ptr(quats), _ptr(raw_scales), _ptr(raw_opacities),
               float(scale_min), float(scale_max), _ptr(covars), _ptr(max_scales), _ptr(opac), N,
               _stream(dev))
@@ -361,7 +399,7 @@ def opacity_bwd(raw_opacities: Tensor, v_opacity_cn: Optional[Tensor],
     if N == 0:
         return out
     sfx = _suffix(raw_opacities, "opacity_bwd")
-    with torch.cuda.device(raw_opacities.device):
+    with _on(raw_opacities.device):
         _call(f"r2s_opacity_bwd_{sfx}", _ptr(raw_opacities), _ptr(v_opacity_cn),
               _ptr(v_opacity_3d), _ptr(out), C, N, _stream(raw_opacities.device))
     return out
@@ -370,17 +408,19 @@ def opacity_bwd(raw_opacities: Tensor, v_opacity_cn: Optional[Tensor],
 # ------------------------------------------------------------- projection --
 
 def _check_cameras(means, covars, viewmats, Ks):
-    _check(means.dim() == 2 and means.size(1) == 3,
-           "means must be 2D [N, 3], got shape ", list(means.shape))
-    _check(covars.dim() == 2 and covars.size(1) == 6,
-           "covars must be 2D [N, 6], got shape ", list(covars.shape))
-    _check(viewmats.dim() == 3 and viewmats.size(1) == 4 and viewmats.size(2) == 4,
-           "viewmats must be 3D [C, 4, 4], got shape ", list(viewmats.shape))
-    _check(Ks.dim() == 3 and Ks.size(1) == 3 and Ks.size(2) == 3,
-           "Ks must be 3D [C, 3, 3], got shape ", list(Ks.shape))
+    if not (means.dim() == 2 and means.size(1) == 3):
+        _fail("means must be 2D [N, 3], got shape ", list(means.shape))
+    if not (covars.dim() == 2 and covars.size(1) == 6):
+        _fail("covars must be 2D [N, 6], got shape ", list(covars.shape))
+    if not (viewmats.dim() == 3 and viewmats.size(1) == 4 and viewmats.size(2) == 4):
+        _fail("viewmats must be 3D [C, 4, 4], got shape ", list(viewmats.shape))
+    if not (Ks.dim() == 3 and Ks.size(1) == 3 and Ks.size(2) == 3):
+        _fail("Ks must be 3D [C, 3, 3], got shape ", list(Ks.shape))
     N, C = means.size(0), viewmats.size(0)
-    _check(covars.size(0) == N, "covars dim 0 (", covars.size(0), ") doesn't match N=", N)
-    _check(Ks.size(0) == C, "Ks batch dim (", Ks.size(0), ") doesn't match C=", C)
+    if covars.size(0) != N:
+        _fail("covars dim 0 (", covars.size(0), ") doesn't match N=", N)
+    if Ks.size(0) != C:
+        _fail("Ks batch dim (", Ks.size(0), ") doesn't match C=", C)
     return C, N
 
 
@@ -391,7 +431,8 @@ def world_to_image_projection_fwd(means: Tensor, covars: Tensor, viewmats: Tenso
     for t, n in ((means, "means"), (covars, "covars"), (viewmats, "viewmats"), (Ks, "Ks")):
         _check_input(t, n)
     C, N = _check_cameras(means, covars, viewmats, Ks)
-    _check(float(radius_clip) > 0.0, "radius_clip must be positive, got ", float(radius_clip))
+    if not (float(radius_clip) > 0.0):
+        _fail("radius_clip must be positive, got ", float(radius_clip))
     dev, dt = means.device, means.dtype
     means2d = torch.empty((C, N, 2), dtype=dt, device=dev)
     cov2d = torch.empty((C, N, 6), dtype=dt, device=dev)
@@ -399,7 +440,7 @@ def world_to_image_projection_fwd(means: Tensor, covars: Tensor, viewmats: Tenso
     if C * N == 0:
         return means2d, cov2d, radii
     sfx = _suffix(means, "world_to_image_projection_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_world_to_image_projection_fwd_{sfx}", _ptr(means), _ptr(covars),
               _ptr(viewmats), _ptr(Ks), int(dim1), int(dim0), float(eps_blur),
               float(radius_clip), _ptr(means2d), _ptr(cov2d), _ptr(radii), C, N, _stream(dev))
@@ -433,7 +474,7 @@ def world_to_image_projection_bwd(means: Tensor, covars: Tensor, viewmats: Tenso
         # over an empty camera set.
         return v_means.zero_(), v_covars.zero_()
     sfx = _suffix(means, "world_to_image_projection_bwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_world_to_image_projection_bwd_{sfx}", _ptr(means), _ptr(covars),
               _ptr(viewmats), _ptr(Ks), int(dim1), int(dim0), _ptr(v_means2d),
               _ptr(v_cov2d_3x3), _ptr(v_means), _ptr(v_covars), C, N, _stream(dev))
@@ -443,8 +484,10 @@ def world_to_image_projection_bwd(means: Tensor, covars: Tensor, viewmats: Tenso
 def conics_mu_fwd(cov2d_3x3: Tensor, eps: float) -> Tuple[Tensor, Tensor]:
     """ConicsMu.cpp:35-80 -> (conics [C,N,3], mus [C,N])."""
     _check_input(cov2d_3x3, "cov2d_3x3")
-    _check(cov2d_3x3.dim() == 3, "cov2d_3x3 must be 3D [C, N, 6], got dim=", cov2d_3x3.dim())
-    _check(cov2d_3x3.size(2) == 6, "cov2d_3x3 last dim must be 6, got ", cov2d_3x3.size(2))
+    if cov2d_3x3.dim() != 3:
+        _fail("cov2d_3x3 must be 3D [C, N, 6], got dim=", cov2d_3x3.dim())
+    if cov2d_3x3.size(2) != 6:
+        _fail("cov2d_3x3 last dim must be 6, got ", cov2d_3x3.size(2))
     C, N = cov2d_3x3.size(0), cov2d_3x3.size(1)
     dev, dt = cov2d_3x3.device, cov2d_3x3.dtype
     conics = torch.empty((C, N, 3), dtype=dt, device=dev)
@@ -452,7 +495,7 @@ def conics_mu_fwd(cov2d_3x3: Tensor, eps: float) -> Tuple[Tensor, Tensor]:
     if C * N == 0:
         return conics, mus
     sfx = _suffix(cov2d_3x3, "conics_mu_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_conics_mu_fwd_{sfx}", _ptr(cov2d_3x3), float(eps), _ptr(conics), _ptr(mus),
               C * N, _stream(dev))
     return conics, mus
@@ -479,7 +522,7 @@ def conics_mu_bwd(cov2d_3x3: Tensor, eps: float, conics: Tensor, mus: Tensor, v_
     if C * N == 0:
         return out
     sfx = _suffix(cov2d_3x3, "conics_mu_bwd")
-    with torch.cuda.device(cov2d_3x3.device):
+    with _on(cov2d_3x3.device):
         _call(f"r2s_conics_mu_bwd_{sfx}", _ptr(cov2d_3x3), float(eps), _ptr(conics), _ptr(mus),
               _ptr(v_conics), _ptr(v_mus), _ptr(out), C * N, _stream(cov2d_3x3.device))
     return out
@@ -494,7 +537,8 @@ def project_gaussians_fwd(means: Tensor, covars: Tensor, opacities: Tensor, view
         _check_input(t, n)
     C, N = _check_cameras(means, covars, viewmats, Ks)
     _check(opacities.dim() == 1 and opacities.size(0) == N, "opacities must be 1D [N]")
-    _check(float(radius_clip) > 0.0, "radius_clip must be positive, got ", float(radius_clip))
+    if not (float(radius_clip) > 0.0):
+        _fail("radius_clip must be positive, got ", float(radius_clip))
     dev, dt = means.device, means.dtype
     means2d = torch.empty((C, N, 2), dtype=dt, device=dev)
     cov2d = torch.empty((C, N, 6), dtype=dt, device=dev)
@@ -505,7 +549,7 @@ def project_gaussians_fwd(means: Tensor, covars: Tensor, opacities: Tensor, view
     if C * N == 0:
         return means2d, cov2d, radii, conics, mus, opac
     sfx = _suffix(means, "project_gaussians_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_project_gaussians_fwd_{sfx}", _ptr(means), _ptr(covars), _ptr(opacities),
               _ptr(viewmats), _ptr(Ks), int(img_w), int(img_h), float(eps2d),
               float(radius_clip), _ptr(means2d), _ptr(cov2d), _ptr(radii), _ptr(conics),
@@ -524,7 +568,8 @@ def project_pack_fwd(means: Tensor, covars: Tensor, opacities: Tensor, viewmats:
         _check_input(t, n)
     C, N = _check_cameras(means, covars, viewmats, Ks)
     _check(opacities.dim() == 1 and opacities.size(0) == N, "opacities must be 1D [N]")
-    _check(float(radius_clip) > 0.0, "radius_clip must be positive, got ", float(radius_clip))
+    if not (float(radius_clip) > 0.0):
+        _fail("radius_clip must be positive, got ", float(radius_clip))
     dev, dt = means.device, means.dtype
     means2d = torch.empty((C, N, 2), dtype=dt, device=dev)
     cov2d = torch.empty((C, N, 6), dtype=dt, device=dev)
@@ -541,7 +586,7 @@ def project_pack_fwd(means: Tensor, covars: Tensor, opacities: Tensor, viewmats:
         return means2d, cov2d, radii, conics, mus, opac, payload, outs
     sfx = _suffix(means, "project_pack_fwd")
     z = (None,) * 5 if outs is None else outs
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_project_pack_fwd_{sfx}", _ptr(means), _ptr(covars), _ptr(opacities),
               _ptr(viewmats), _ptr(Ks), int(img_w), int(img_h), float(eps2d),
               float(radius_clip), _ptr(means2d), _ptr(cov2d), _ptr(radii), _ptr(conics),
@@ -562,14 +607,15 @@ def project_gaussians_bwd(means: Tensor, covars: Tensor, viewmats: Tensor, Ks: T
     for t, shape, n in ((cov2d, (C, N, 6), "cov2d_3x3"), (conics, (C, N, 3), "conics"),
                         (mus, (C, N), "mus"), (v_means2d, (C, N, 2), "v_means2d"),
                         (v_conics, (C, N, 3), "v_conics"), (v_mus, (C, N), "v_mus")):
-        _check(tuple(t.shape) == shape, f"{n} shape must be {list(shape)}")
+        if t.shape != shape:
+            _fail(f"{n} shape must be {list(shape)}")
     dev, dt = means.device, means.dtype
     v_means = torch.empty((N, 3), dtype=dt, device=dev)
     v_covars = torch.empty((N, 6), dtype=dt, device=dev)
     if N == 0:
         return v_means, v_covars
     sfx = _suffix(means, "project_gaussians_bwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_project_gaussians_bwd_{sfx}", _ptr(means), _ptr(covars), _ptr(viewmats),
               _ptr(Ks), int(img_w), int(img_h), float(eps2d), _ptr(cov2d), _ptr(conics),
               _ptr(mus), _ptr(v_means2d), _ptr(v_conics), _ptr(v_mus), _ptr(v_means),
@@ -604,19 +650,21 @@ def explicit_backward_tail(means: Tensor, covars: Tensor, viewmats: Tensor, Ks: 
                         (quats, (N, 4), "quats"), (raw_scales, (N, 3), "raw_scales"),
                         (raw_opacities, (N,), "raw_opacities"),
                         (v_opacity_cn, (C, N), "v_opacity_cn")):
-        _check(tuple(t.shape) == shape, f"{n} shape must be {list(shape)}")
+        if t.shape != shape:
+            _fail(f"{n} shape must be {list(shape)}")
     _check((add_means is None) == (add_covars is None),
            "add_means and add_covars must be given together")
     for t, shape, n in ((add_means, (N, 3), "add_means"), (add_covars, (N, 6), "add_covars"),
                         (v_opacity_3d, (N,), "v_opacity_3d")):
         if t is not None:
             _check_input(t, n)
-            _check(tuple(t.shape) == shape, f"{n} shape must be {list(shape)}")
+            if t.shape != shape:
+                _fail(f"{n} shape must be {list(shape)}")
     dev, dt = means.device, means.dtype
     for t in (covars, viewmats, Ks, cov2d, conics, mus, v_means2d, v_conics, v_mus, add_means,
               add_covars, quats, raw_scales, raw_opacities, v_opacity_cn, v_opacity_3d):
-        _check(t is None or (t.dtype == dt and t.device == dev),
-               "explicit_backward_tail inputs must share one dtype and device")
+        if t is not None and (t.dtype != dt or t.device != dev):
+            _fail("explicit_backward_tail inputs must share one dtype and device")
     v_means = torch.empty((N, 3), dtype=dt, device=dev)
     v_quats = torch.empty((N, 4), dtype=dt, device=dev)
     v_raw_scales = torch.empty((N, 3), dtype=dt, device=dev)
@@ -624,7 +672,7 @@ def explicit_backward_tail(means: Tensor, covars: Tensor, viewmats: Tensor, Ks: 
     if N == 0:
         return v_means, v_quats, v_raw_scales, v_raw_opac
     sfx = _suffix(means, "explicit_backward_tail")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_explicit_backward_tail_{sfx}", _ptr(means), _ptr(covars), _ptr(viewmats),
               _ptr(Ks), int(img_w), int(img_h), float(eps2d), _ptr(cov2d), _ptr(conics),
               _ptr(mus), _ptr(v_means2d), _ptr(v_conics), _ptr(v_mus), _ptr(add_means),
@@ -656,14 +704,12 @@ def bin_tiles_2d(means2d: Tensor, radii: Tensor, tile_size: int, n_tiles_dim1: i
     dev = means2d.device
     tw, th, ts = int(n_tiles_dim1), int(n_tiles_dim0), int(tile_size)
     tiles_per_gauss = torch.empty((C, N), dtype=torch.int32, device=dev)
-    empty = TileLists(tiles_per_gauss, torch.empty((0,), dtype=torch.int64, device=dev),
-                      torch.empty((0,), dtype=torch.int32, device=dev), None, None)
     if C * N == 0:
-        return empty
+        return _no_records(tiles_per_gauss)
     lib = _lib()
     sfx = _suffix(means2d, "isect_tiles")
     rect = 1 if radii.dim() == 3 else 0
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _stream(dev)
         offsets = torch.empty((C * N + 1,), dtype=torch.int64, device=dev)
         ws = _workspace(lib.r2s_isect_workspace_bytes(C * N, 0, 0), dev)
@@ -680,7 +726,7 @@ def bin_tiles_2d(means2d: Tensor, radii: Tensor, tile_size: int, n_tiles_dim1: i
         res = _emit_and_sort(launch, offsets, C * N, C * tw * th, "isect_tiles", dev, "2d",
                              keep_ids=keep_ids)
     if res is None:
-        return empty
+        return _no_records(tiles_per_gauss)
     return TileLists(tiles_per_gauss, *res, tile_offsets)
 
 
@@ -701,7 +747,7 @@ def keys_from_offsets(tile_offsets: Tensor, n_isects: int) -> Tensor:
     dev = tile_offsets.device
     keys = torch.empty((int(n_isects),), dtype=torch.int64, device=dev)
     if keys.numel() > 0:
-        with torch.cuda.device(dev):
+        with _on(dev):
             _call("r2s_isect_keys_from_offsets", _ptr(tile_offsets), tile_offsets.numel(),
                   keys.numel(), _ptr(keys), _stream(dev))
     return keys
@@ -717,7 +763,7 @@ def isect_offset_encode(isect_ids: Tensor, C: int, n_tiles_dim1: int,
     offsets = torch.empty((C, th, tw), dtype=torch.int32, device=dev)
     if offsets.numel() == 0:
         return offsets
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call("r2s_isect_offset_encode", _ptr(isect_ids), isect_ids.numel(), C * tw * th,
               _ptr(offsets), _stream(dev))
     return offsets
@@ -743,13 +789,11 @@ def bin_tiles_3d(means3d: Tensor, radii: Tensor, tile_size: int, n_tiles_dim2: i
     dev = means3d.device
     n2, n1, n0, ts = int(n_tiles_dim2), int(n_tiles_dim1), int(n_tiles_dim0), int(tile_size)
     tiles_per_gauss = torch.empty((N,), dtype=torch.int32, device=dev)
-    empty = TileLists(tiles_per_gauss, torch.empty((0,), dtype=torch.int64, device=dev),
-                      torch.empty((0,), dtype=torch.int32, device=dev), None, None)
     if N == 0:
-        return empty
+        return _no_records(tiles_per_gauss)
     lib = _lib()
     sfx = _suffix(means3d, "isect_tiles_3d")
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _stream(dev)
         offsets = torch.empty((N + 1,), dtype=torch.int64, device=dev)
         ws = _workspace(lib.r2s_isect_workspace_bytes(N, 0, 0), dev)
@@ -769,7 +813,7 @@ def bin_tiles_3d(means3d: Tensor, radii: Tensor, tile_size: int, n_tiles_dim2: i
     if res is TOO_MANY:
         return None
     if res is None:
-        return empty
+        return _no_records(tiles_per_gauss)
     return TileLists(tiles_per_gauss, *res, tile_offsets)
 
 
@@ -791,7 +835,7 @@ def isect_offset_encode_3d(isect_ids: Tensor, n_tiles_dim2: int, n_tiles_dim1: i
     offsets = torch.empty((n0, n1, n2), dtype=torch.int32, device=dev)
     if offsets.numel() == 0:
         return offsets
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call("r2s_isect_offset_encode", _ptr(isect_ids), isect_ids.numel(), n0 * n1 * n2,
               _ptr(offsets), _stream(dev))
     return offsets
@@ -817,7 +861,7 @@ def layer_counts_3d(means3d: Tensor, radii: Tensor, tile_size: int, n_tiles_dim2
     dev = means3d.device
     counts = torch.empty((max(n0, 1),), dtype=torch.int64, device=dev)
     ws = _workspace(8 * (n0 + 1), dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_isect_layer_counts_3d_{_suffix(means3d, 'isect_tiles_3d')}", _ptr(means3d),
               _ptr(radii), N, int(tile_size), int(n_tiles_dim2), int(n_tiles_dim1), n0,
               _ptr(counts), _ptr(ws), ws.numel(), _stream(dev))
@@ -858,15 +902,14 @@ def bin_tiles_3d_slab(means3d: Tensor, radii: Tensor, tile_size: int, n_tiles_di
     dev = means3d.device
     n2, n1, n0, ts = int(n_tiles_dim2), int(n_tiles_dim1), int(n_tiles_dim0), int(tile_size)
     z0, z1 = int(z0), int(z1)
-    _check(0 <= z0 <= z1 <= n0, f"brick layers [{z0}, {z1}) outside [0, {n0})")
+    if not (0 <= z0 <= z1 <= n0):
+        _fail(f"brick layers [{z0}, {z1}) outside [0, {n0})")
     n_keys = (z1 - z0) * n1 * n2
     lib = _lib()
     sfx = _suffix(means3d, "isect_tiles_3d")
     tpg = torch.empty((N,), dtype=torch.int32, device=dev)
     offs = torch.empty((z1 - z0, n1, n2), dtype=torch.int32, device=dev)
-    empty = TileLists(tpg, torch.empty((0,), dtype=torch.int64, device=dev),
-                      torch.empty((0,), dtype=torch.int32, device=dev), None, None)
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _stream(dev)
         offsets = torch.empty((N + 1,), dtype=torch.int64, device=dev)
         ws = _workspace(lib.r2s_isect_workspace_bytes(N, 0, 0), dev)
@@ -876,7 +919,7 @@ def bin_tiles_3d_slab(means3d: Tensor, radii: Tensor, tile_size: int, n_tiles_di
         _check_record_count(n, "isect_tiles_3d (z-slab)")
         if n == 0 or n_keys == 0:
             offs.zero_()
-            return empty, offs
+            return _no_records(tpg), offs
         end_bit = _end_bit(n_keys)
         outs = (torch.empty((n,), dtype=torch.int64, device=dev) if keep_ids else None,
                 torch.empty((n,), dtype=torch.int32, device=dev),
@@ -900,7 +943,7 @@ def voxelize_slab(means3d: Tensor, conics: Tensor, opacities: Tensor, tile_offse
     d0, d1, d2 = volume.shape
     nz, n1, n2 = tile_offsets.shape
     dev = means3d.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_voxelize_fwd_slab_{_suffix(means3d, 'voxelize_to_voxels_fwd')}",
               _ptr(means3d), _ptr(conics), _ptr(opacities), _ptr(tile_offsets),
               _ptr(lists.flatten_ids) if lists.flatten_ids.numel() else None,
@@ -923,7 +966,7 @@ def voxel_backward_slab(means3d: Tensor, conics: Tensor, opacities: Tensor,
     n = lists.flatten_ids.numel()
     v_m, v_c, v_o = (torch.empty_like(t) for t in (means3d, conics, opacities))
     dev = means3d.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         if n == 0:
             for t in (v_m, v_c, v_o):
                 t.zero_()
@@ -977,7 +1020,7 @@ def rasterize_to_pixels_fwd(means2d: Tensor, conics: Tensor, opacities: Tensor, 
         return out.zero_()
     sfx = _suffix(means2d, "rasterize_to_pixels_fwd")
     lib = _lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         nbytes = lib.r2s_rasterize_workspace_bytes(C * tw * th, n_isects, ts,
                                                    means2d.element_size())
         ws = _workspace(nbytes, dev) if nbytes > 0 else None
@@ -996,9 +1039,9 @@ def _resolve_emission(emission, flatten_ids: Tensor, n_keys: int, op: str):
     else:
         emit = emission
         if emit is not None:
-            _check(emit[0].numel() == flatten_ids.numel() and
-                   emit[1].numel() == flatten_ids.numel(),
-                   f"{op}: emission arrays must have one entry per record")
+            if not (emit[0].numel() == flatten_ids.numel()
+                    and emit[1].numel() == flatten_ids.numel()):
+                _fail(f"{op}: emission arrays must have one entry per record")
     _note_path(emit is not None, op)
     return emit
 
@@ -1026,7 +1069,7 @@ def _raster_bwd(means2d, conics, opacities, mus, tile_offsets, isect_ids, flatte
         return v_abs, v_means2d, v_conics, v_opac, v_mus
     sfx = _suffix(means2d, op)
     dev = means2d.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         if emit is not None:
             ws = _workspace(_lib().r2s_rasterize_bwd_workspace_bytes(
                 n_isects, C * N, means2d.element_size()), dev)
@@ -1123,7 +1166,7 @@ def raster_pack(means2d: Tensor, conics: Tensor, opacities: Tensor, mus: Tensor,
         return payload, outs
     sfx = _suffix(means2d, "rasterize_pack")
     z = (None,) * 5 if outs is None else outs
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_rasterize_pack_{sfx}", _ptr(means2d), _ptr(conics), _ptr(opacities),
               _ptr(mus), C, N, _ptr(payload), *[_ptr(t) for t in z], _stream(dev))
     return payload, outs
@@ -1149,7 +1192,7 @@ def rasterize_packed(payload: Tensor, tile_offsets: Tensor, flatten_ids: Tensor,
         return out.zero_()
     sfx = _suffix(payload, "rasterize_packed")
     lib = _lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         nbytes = lib.r2s_rasterize_workspace_bytes(C * tw * th, n_isects, ts,
                                                    payload.element_size())
         ws = _workspace(nbytes, dev) if nbytes > 0 else None
@@ -1194,7 +1237,7 @@ def raster_backward_packed(payload: Tensor, opacities: Tensor, mus: Tensor,
         _note_path(True, "raster_backward_packed")
     emit, src = lists.emission if n_isects > 0 else (None, None)
     sfx = _suffix(payload, "raster_backward_packed")
-    with torch.cuda.device(dev):
+    with _on(dev):
         nbytes = _lib().r2s_rasterize_bwd_workspace_bytes(n_isects, 0, payload.element_size())
         ws = _workspace(nbytes, dev) if nbytes > 0 else None
         _call(f"r2s_rasterize_bwd_packed_{sfx}", _ptr(payload), _ptr(opacities), _ptr(mus),
@@ -1215,19 +1258,21 @@ def world_to_volume_mapping_fwd(means: Tensor, covars: Tensor, max_scales: Tenso
     for t, n in ((means, "means"), (covars, "covars"), (max_scales, "max_scales"),
                  (ranges, "ranges"), (centers, "centers")):
         _check_input(t, n)
-    _check(means.dim() == 2 and means.size(1) == 3,
-           "means must be 2D [N, 3], got shape ", list(means.shape))
-    _check(covars.dim() == 2 and covars.size(1) == 6,
-           "covars must be 2D [N, 6], got shape ", list(covars.shape))
-    _check(max_scales.dim() == 1, "max_scales must be 1D [N], got dim ", max_scales.dim())
-    _check(ranges.dim() == 1 and ranges.size(0) == 3,
-           "ranges must be 1D [3], got shape ", list(ranges.shape))
-    _check(centers.dim() == 1 and centers.size(0) == 3,
-           "centers must be 1D [3], got shape ", list(centers.shape))
+    if not (means.dim() == 2 and means.size(1) == 3):
+        _fail("means must be 2D [N, 3], got shape ", list(means.shape))
+    if not (covars.dim() == 2 and covars.size(1) == 6):
+        _fail("covars must be 2D [N, 6], got shape ", list(covars.shape))
+    if max_scales.dim() != 1:
+        _fail("max_scales must be 1D [N], got dim ", max_scales.dim())
+    if not (ranges.dim() == 1 and ranges.size(0) == 3):
+        _fail("ranges must be 1D [3], got shape ", list(ranges.shape))
+    if not (centers.dim() == 1 and centers.size(0) == 3):
+        _fail("centers must be 1D [3], got shape ", list(centers.shape))
     N = means.size(0)
-    _check(covars.size(0) == N, "covars batch dim (", covars.size(0), ") doesn't match N=", N)
-    _check(max_scales.size(0) == N, "max_scales batch dim (", max_scales.size(0),
-           ") doesn't match N=", N)
+    if covars.size(0) != N:
+        _fail("covars batch dim (", covars.size(0), ") doesn't match N=", N)
+    if max_scales.size(0) != N:
+        _fail("max_scales batch dim (", max_scales.size(0), ") doesn't match N=", N)
     dev, dt = means.device, means.dtype
     means3d = torch.empty((N, 3), dtype=dt, device=dev)
     conics = torch.empty((N, 6), dtype=dt, device=dev)
@@ -1237,7 +1282,7 @@ def world_to_volume_mapping_fwd(means: Tensor, covars: Tensor, max_scales: Tenso
     _check(covars.dtype == dt and ranges.dtype == dt and centers.dtype == dt,
            "means, covars, ranges and centers must share a dtype")
     sfx = _suffix(means, "world_to_volume_mapping_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_world_to_volume_mapping_fwd_{sfx}", _ptr(means), _ptr(covars),
               _ptr(ranges), _ptr(centers), int(dim2), int(dim1), int(dim0),
               float(eps3d), float(radius_clip), _ptr(means3d), _ptr(conics), _ptr(radii), N,
@@ -1270,7 +1315,7 @@ def world_to_volume_mapping_bwd(means: Tensor, covars: Tensor, ranges: Tensor, c
     _check(all(t.dtype == dt for t in (covars, ranges, centers, v_means3d_v, v_conics)),
            "world_to_volume_mapping_bwd inputs must share a dtype")
     sfx = _suffix(means, "world_to_volume_mapping_bwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_world_to_volume_mapping_bwd_{sfx}", _ptr(means), _ptr(covars),
               _ptr(ranges), _ptr(centers), int(dim2), int(dim1), int(dim0),
               float(eps3d), _ptr(v_means3d_v), _ptr(v_conics), _ptr(v_means), _ptr(v_covars), N,
@@ -1313,7 +1358,7 @@ def voxelize_to_voxels_fwd(means3d: Tensor, conics: Tensor, opacities: Tensor,
         return torch.zeros((d0, d1, d2), dtype=means3d.dtype, device=dev)
     out = torch.empty((d0, d1, d2), dtype=means3d.dtype, device=dev)
     sfx = _suffix(means3d, "voxelize_to_voxels_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_voxelize_fwd_{sfx}", _ptr(means3d), _ptr(conics), _ptr(opacities),
               _ptr(tile_offsets), _ptr(flatten_ids), n_isects, N, d2, d1, d0, ts, n2, n1, n0,
               _ptr(out), _stream(dev))
@@ -1340,7 +1385,7 @@ def voxelize_with_reach(means3d: Tensor, conics: Tensor, opacities: Tensor,
     out = torch.empty((d0, d1, d2), dtype=means3d.dtype, device=dev)
     reach = torch.empty(n_isects, dtype=torch.int64, device=dev)
     sfx = _suffix(means3d, "voxelize_to_voxels_fwd")
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call(f"r2s_voxelize_fwd_reach_{sfx}", _ptr(means3d), _ptr(conics), _ptr(opacities),
               _ptr(tile_offsets), _ptr(flatten_ids), n_isects, N, d2, d1, d0, 8, n2, n1, n0,
               _ptr(out), _ptr(reach), _stream(dev))
@@ -1366,7 +1411,7 @@ def _voxel_bwd(means3d, conics, opacities, tile_offsets, isect_ids, flatten_ids,
     _check(tuple(v_render.shape) == (d0, d1, d2), "v_render_output shape must be [dim0, dim1, dim2]")
     sfx = _suffix(means3d, op)
     dev = means3d.device
-    with torch.cuda.device(dev):
+    with _on(dev):
         if emit is not None and reach is not None:
             _check(ts == 8 and reach.dtype == torch.int64 and reach.numel() == n_isects
                    and reach.is_contiguous() and reach.device == dev,
@@ -1450,6 +1495,12 @@ def mask_split(mask: Tensor) -> Tuple[Tensor, int]:
     ``indices[n_true:]`` equals ``torch.where(~mask)[0]``
     (src/strategies/binary_tree.py:68,101-102,158).
     """
+    out, count = _mask_split_enqueue(mask)
+    return out, int(count.item())
+
+
+def _mask_split_enqueue(mask: Tensor) -> Tuple[Tensor, Tensor]:
+    """:func:`mask_split` with n_true still on the device, int64 [1]."""
     _check(isinstance(mask, torch.Tensor) and mask.is_cuda, "mask must be a CUDA tensor")
     m = mask.reshape(-1)
     if m.dtype != torch.bool and m.dtype != torch.uint8:
@@ -1460,12 +1511,11 @@ def mask_split(mask: Tensor) -> Tuple[Tensor, int]:
     out = torch.empty((n,), dtype=torch.int64, device=dev)
     count = torch.empty((1,), dtype=torch.int64, device=dev)
     lib = _lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws = _workspace(lib.r2s_mask_workspace_bytes(n), dev)
         _call("r2s_mask_split", _ptr(m) if n else None, n, _ptr(out) if n else None,
               _ptr(count), _ptr(ws), ws.numel(), _stream(dev))
-        n_true = int(count.item())
-    return out, n_true
+    return out, count
 
 
 # ------------------------------------------------------------- densify --
@@ -1478,58 +1528,83 @@ def mask_split(mask: Tensor) -> Tuple[Tensor, int]:
 # values; `extra` is the live column appended to a history archive
 # (role COL_HISTORY) and None otherwise.
 
-def _densify_table(columns, n_rows: int, main_rows: int, hist_rows: int, n_sel: int, what: str):
+_COLUMN = struct.Struct("@PPPqii")  # _lib.Column, packed in one call
+
+
+def _densify_columns(columns, n_rows: int, hist_rows: int, what: str) -> list:
+    """Check the columns; each one's values per row.  Nothing here depends on
+    how many rows are selected, so it runs while the device counts them."""
+    from . import _lib as L
+
+    widths = []
+    for i, col in enumerate(columns):
+        src, role, extra = col
+        if not _is_input(src):
+            _check_input(src, f"{what}: column {i}")
+        dtype, shape = src.dtype, src.shape
+        if dtype not in (torch.float32, torch.int32):
+            _fail(f"{what}: column {i} must be float32 or int32, got {dtype}")
+        if len(shape) < 1:
+            _fail(f"{what}: column {i} must have a row dimension")
+        width = math.prod(shape[1:])
+        if not (1 <= width <= L.DENSIFY_MAX_WIDTH):
+            _fail(f"{what}: column {i} has {width} values per row (1..{L.DENSIFY_MAX_WIDTH})")
+        if role in (L.COL_MEANS, L.COL_RAW_SCALES, L.COL_RAW_OPACITIES):
+            if dtype != torch.float32:
+                _fail(f"{what}: column {i} (role {role}) must be float32")
+        if role in (L.COL_PARENT, L.COL_LEVEL):
+            if not (dtype == torch.int32 and width == 1):
+                _fail(f"{what}: column {i} (parent / level) must be int32 [N]")
+        if role == L.COL_HISTORY:
+            if extra is None:
+                _fail(f"{what}: history column {i} needs its live column")
+            if not _is_input(extra):
+                _check_input(extra, f"{what}: live column of history column {i}")
+            if not (extra.dtype == dtype and extra.shape[1:] == shape[1:]):
+                _fail(f"{what}: history column {i} and its live column differ in dtype or shape")
+            if extra.size(0) != n_rows:
+                _fail(f"{what}: live column of history column {i} has {extra.size(0)} rows, "
+                      f"expected {n_rows}")
+            if shape[0] != hist_rows:
+                _fail(f"{what}: history column {i} has {shape[0]} rows, expected {hist_rows}")
+        else:
+            if extra is not None:
+                _fail(f"{what}: column {i}: only history columns take a live column")
+            if shape[0] != n_rows:
+                _fail(f"{what}: column {i} has {shape[0]} rows, expected {n_rows}")
+        widths.append(width)
+    return widths
+
+
+def _densify_table(columns, widths, main_rows: int, hist_rows: int, n_sel: int):
+    """The library's column table and the output tensors for columns that
+    :func:`_densify_columns` checked."""
     from . import _lib as L
 
     table = (L.Column * max(len(columns), 1))()
     outs, used = [], 0
-    for i, col in enumerate(columns):
-        src, role, extra = col
-        _check_input(src, f"{what}: column {i}")
-        _check(src.dtype in (torch.float32, torch.int32),
-               f"{what}: column {i} must be float32 or int32, got {src.dtype}")
-        _check(src.dim() >= 1, f"{what}: column {i} must have a row dimension")
-        width = int(math.prod(src.shape[1:]))
-        _check(1 <= width <= L.DENSIFY_MAX_WIDTH,
-               f"{what}: column {i} has {width} values per row (1..{L.DENSIFY_MAX_WIDTH})")
-        if role in (L.COL_MEANS, L.COL_RAW_SCALES, L.COL_RAW_OPACITIES):
-            _check(src.dtype == torch.float32, f"{what}: column {i} (role {role}) must be float32")
-        if role in (L.COL_PARENT, L.COL_LEVEL):
-            _check(src.dtype == torch.int32 and width == 1,
-                   f"{what}: column {i} (parent / level) must be int32 [N]")
+    for (src, role, extra), width in zip(columns, widths):
         if role == L.COL_HISTORY:
-            _check(extra is not None, f"{what}: history column {i} needs its live column")
-            _check_input(extra, f"{what}: live column of history column {i}")
-            _check(extra.dtype == src.dtype and tuple(extra.shape[1:]) == tuple(src.shape[1:]),
-                   f"{what}: history column {i} and its live column differ in dtype or shape")
-            _check(extra.size(0) == n_rows,
-                   f"{what}: live column of history column {i} has {extra.size(0)} rows, "
-                   f"expected {n_rows}")
-            _check(src.size(0) == hist_rows,
-                   f"{what}: history column {i} has {src.size(0)} rows, expected {hist_rows}")
             if n_sel == 0:
                 outs.append(src)  # nothing to archive: the archive is returned as is
                 continue
             rows = hist_rows + n_sel
         else:
-            _check(extra is None, f"{what}: column {i}: only history columns take a live column")
-            _check(src.size(0) == n_rows,
-                   f"{what}: column {i} has {src.size(0)} rows, expected {n_rows}")
             rows = main_rows
-        dst = torch.empty((rows,) + tuple(src.shape[1:]), dtype=src.dtype, device=src.device)
-        table[used] = L.Column(src.data_ptr() if src.numel() else None,
-                               dst.data_ptr() if dst.numel() else None,
-                               extra.data_ptr() if extra is not None and extra.numel() else None,
-                               rows, width, role)
+        dst = torch.empty((rows,) + src.shape[1:], dtype=src.dtype, device=src.device)
+        # An empty tensor's data_ptr() is 0, the null pointer.
+        _COLUMN.pack_into(table, used * _COLUMN.size, src.data_ptr(), dst.data_ptr(),
+                          0 if extra is None else extra.data_ptr(), rows, width, role)
         used += 1
         outs.append(dst)
     return table, used, outs
 
 
 def _densify_mask(mask: Tensor, n_rows: int, what: str):
-    _check(isinstance(mask, torch.Tensor) and mask.is_cuda, f"{what}: mask must be a CUDA tensor")
-    _check(mask.dim() == 1 and mask.size(0) == n_rows,
-           f"{what}: mask must be 1-D with {n_rows} entries")
+    if not (isinstance(mask, torch.Tensor) and mask.is_cuda):
+        _fail(f"{what}: mask must be a CUDA tensor")
+    if not (mask.dim() == 1 and mask.size(0) == n_rows):
+        _fail(f"{what}: mask must be 1-D with {n_rows} entries")
     m = mask if mask.dtype in (torch.bool, torch.uint8) else mask != 0
     return m.contiguous().view(torch.uint8)
 
@@ -1548,17 +1623,16 @@ def densify_split(mask: Tensor, columns, history_rows: int = 0, geometry=None):
 
     n = int(mask.shape[0]) if isinstance(mask, torch.Tensor) and mask.dim() == 1 else -1
     m = _densify_mask(mask, n, "densify_split")
-    idx, n_sel = mask_split(m)
-    n_rest = n - n_sel
+    idx, count = _mask_split_enqueue(m)
     dev = m.device
-    table, used, outs = _densify_table(columns, n, n_rest + 2 * n_sel, history_rows, n_sel,
-                                       "densify_split")
+    widths = _densify_columns(columns, n, history_rows, "densify_split")
     geo = None
     if geometry is not None:
         quats, raw_scales, smin, smax, eps, sigmoid = geometry
         for t, name in ((quats, "quats"), (raw_scales, "raw_scales")):
             _check_input(t, name)
-            _check(t.dtype == torch.float32, f"densify_split: {name} must be float32")
+            if t.dtype != torch.float32:
+                _fail(f"densify_split: {name} must be float32")
         _check(tuple(quats.shape) == (n, 4) and tuple(raw_scales.shape) == (n, 3),
                "densify_split: geometry must be quats [N,4] and raw_scales [N,3]")
         smin = [float(v) for v in smin]
@@ -1567,7 +1641,10 @@ def densify_split(mask: Tensor, columns, history_rows: int = 0, geometry=None):
         geo = L.SplitGeometry(quats.data_ptr() if n else None, raw_scales.data_ptr() if n else None,
                               (ctypes.c_float * 3)(*smin), (ctypes.c_float * 3)(*smax),
                               float(eps), int(bool(sigmoid)))
-    with torch.cuda.device(dev):
+    n_sel = int(count.item())
+    n_rest = n - n_sel
+    table, used, outs = _densify_table(columns, widths, n_rest + 2 * n_sel, history_rows, n_sel)
+    with _on(dev):
         _call("r2s_densify_split", idx.data_ptr() if n_sel else None, n_sel,
               idx[n_sel:].data_ptr() if n_rest else None, n_rest, int(history_rows),
               ctypes.byref(geo) if geo is not None else None, table, used, _stream(dev))
@@ -1584,11 +1661,12 @@ def densify_duplicate(mask: Tensor, columns, history_rows: int = 0):
     """
     n = int(mask.shape[0]) if isinstance(mask, torch.Tensor) and mask.dim() == 1 else -1
     m = _densify_mask(mask, n, "densify_duplicate")
-    idx, n_sel = mask_split(m)
+    idx, count = _mask_split_enqueue(m)
     dev = m.device
-    table, used, outs = _densify_table(columns, n, n + n_sel, history_rows, n_sel,
-                                       "densify_duplicate")
-    with torch.cuda.device(dev):
+    widths = _densify_columns(columns, n, history_rows, "densify_duplicate")
+    n_sel = int(count.item())
+    table, used, outs = _densify_table(columns, widths, n + n_sel, history_rows, n_sel)
+    with _on(dev):
         _call("r2s_densify_duplicate", m.data_ptr() if n else None, n,
               idx.data_ptr() if n_sel else None, n_sel, int(history_rows), table, used,
               _stream(dev))
@@ -1600,11 +1678,13 @@ def densify_remove(mask: Tensor, columns):
     Returns ``(outputs, n_removed)``."""
     n = int(mask.shape[0]) if isinstance(mask, torch.Tensor) and mask.dim() == 1 else -1
     m = _densify_mask(mask, n, "densify_remove")
-    idx, n_sel = mask_split(m)
-    n_keep = n - n_sel
+    idx, count = _mask_split_enqueue(m)
     dev = m.device
-    table, used, outs = _densify_table(columns, n, n_keep, 0, 0, "densify_remove")
-    with torch.cuda.device(dev):
+    widths = _densify_columns(columns, n, 0, "densify_remove")
+    n_sel = int(count.item())
+    n_keep = n - n_sel
+    table, used, outs = _densify_table(columns, widths, n_keep, 0, 0)
+    with _on(dev):
         _call("r2s_densify_remove", idx[n_sel:].data_ptr() if n_keep else None, n_keep, table,
               used, _stream(dev))
     return outs, n_sel
@@ -1613,8 +1693,10 @@ def densify_remove(mask: Tensor, columns):
 # ---------------------------------------------------------- projection loss --
 
 def _loss_images(t: Tensor, name: str) -> Tensor:
-    _check(isinstance(t, torch.Tensor) and t.is_cuda, f"{name} must be a CUDA tensor")
-    _check(t.dtype == torch.float32, f"{name} must be float32, got {t.dtype}")
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        _fail(f"{name} must be a CUDA tensor")
+    if t.dtype != torch.float32:
+        _fail(f"{name} must be float32, got {t.dtype}")
     return t.contiguous()
 
 
@@ -1639,7 +1721,7 @@ def projection_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Te
     dev = r.device
     lib = _lib()
     losses = torch.empty(3, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws = _workspace(lib.r2s_projection_loss_workspace_bytes(n, H, W), dev)
         _call("r2s_projection_loss_fwd_f32", _ptr(r), _ptr(t), _ptr(e), _ptr(m), n, H, W,
               int(window_size), _ptr(losses), _ptr(ws), ws.numel(), _stream(dev))
@@ -1659,7 +1741,7 @@ def projection_loss_bwd(render: Tensor, target: Tensor, edge_target: Optional[Te
     n, H, W = r.shape
     dev = r.device
     out = torch.empty_like(r)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call("r2s_projection_loss_bwd_f32", _ptr(r), _ptr(t), _ptr(e), _ptr(m), n, H, W,
               int(window_size), _ptr(g), _ptr(workspace), workspace.numel(), _ptr(out),
               _stream(dev))
@@ -1681,7 +1763,7 @@ def tv_fwd(volume: Tensor, mean: bool = True) -> Tensor:
     dev = v.device
     lib = _lib()
     out = torch.empty((), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws = _workspace(lib.r2s_tv_workspace_bytes(), dev)
         _call("r2s_tv_fwd_f32", _ptr(v), *v.shape, int(bool(mean)), _ptr(out), _ptr(ws),
               ws.numel(), _stream(dev))
@@ -1695,7 +1777,7 @@ def tv_bwd(volume: Tensor, grad_out: Tensor, mean: bool = True) -> Tensor:
     _check(g.numel() == 1, "grad_out must be a scalar")
     dev = v.device
     out = torch.empty_like(v)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call("r2s_tv_bwd_f32", _ptr(v), *v.shape, int(bool(mean)), _ptr(g), _ptr(out),
               _stream(dev))
     return out
@@ -1722,7 +1804,7 @@ def hierarchy_loss_fwd(child_means: Tensor, parent: Tensor, history_means: Tenso
     dev = c.device
     lib = _lib()
     out = torch.empty(2, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws = _workspace(lib.r2s_hierarchy_workspace_bytes(n), dev)
         _call("r2s_hierarchy_loss_fwd_f32", _ptr(c), _ptr(par), n, _ptr(hm), _ptr(hs), _ptr(hq),
               int(history_count), float(max_parent_distance_factor), _ptr(out), _ptr(ws),
@@ -1735,7 +1817,7 @@ def hierarchy_loss_bwd(n: int, grad_out: Tensor, out: Tensor, workspace: Tensor)
     g = _loss_images(grad_out, "grad_out")
     dev = out.device
     v = torch.empty((n, 3), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _call("r2s_hierarchy_loss_bwd_f32", n, _ptr(g), _ptr(out), _ptr(workspace),
               workspace.numel(), _ptr(v), _stream(dev))
     return v

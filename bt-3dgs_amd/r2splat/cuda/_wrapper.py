@@ -8,12 +8,12 @@ from __future__ import annotations
 
 from typing import Callable
 
+from ._backend import operators as _operators
+
 
 def _make_cuda_func(name: str) -> Callable:
     def call_cuda(*args, **kwargs):
-        from ._backend import _C
-
-        return getattr(_C, name)(*args, **kwargs)
+        return getattr(_operators(), name)(*args, **kwargs)
 
     call_cuda.__name__ = name
     return call_cuda

@@ -28,18 +28,15 @@ from typing import NamedTuple, Optional, Tuple
 
 import torch
 
+# The operators' module, loaded at the first call: importing r2splat.ops must
+# not load the HIP library.
+from ..cuda._backend import operators as _ops
+
 Tensor = torch.Tensor
 
 CUDA_REQUIRED = "Direct r2splat operators require CUDA tensors."
 TILE_2D = "2D tile_size must be positive with tile_size**2 <= 1024."
 TILE_3D = "3D tile_size must be positive with tile_size**3 <= 1024."
-
-
-def _ops():
-    # Deferred: importing r2splat.ops must not load the HIP library.
-    from ..cuda._backend import _C
-
-    return _C
 
 
 def activate(quats: Tensor, raw_scales: Tensor, raw_opacities: Tensor, scale_min: float,

@@ -25,6 +25,7 @@ from typing import Optional
 
 import torch
 
+from ..cuda._backend import operators
 from ._passes import ImagePass, VolumePass, activate
 from .direct import MappingVoxelizationResult, ProjectionRasterizationResult
 
@@ -173,8 +174,6 @@ def explicit_backward(
     image_pass = state.projection
     if image_pass is None:
         raise RuntimeError("Explicit backward requires a projection forward pass.")
-    from ..cuda._backend import _C
-
     volume_pass = state.voxel
     g3 = None
     if volume_pass is not None and volume_pass.volume.grad is not None:
@@ -205,10 +204,10 @@ def explicit_backward(
             volume_weights = g3.v_weights
         # Covariance -> (quaternion, raw scale) VJP; opacity: the volume's
         # gradient times softplus' = sigmoid.
-        v_quats, v_raw_scales = _C.parameter_transform_bwd(
+        v_quats, v_raw_scales = operators().parameter_transform_bwd(
             quats.contiguous(), raw_scales.contiguous(), state.scale_min, state.scale_max,
             world_covars.get().contiguous())
-        v_raw_opacities = _C.opacity_bwd(raw_opacities.contiguous(), None, volume_weights)
+        v_raw_opacities = operators().opacity_bwd(raw_opacities.contiguous(), None, volume_weights)
         v_means = world_means.get()
 
     _add_to_grad(means, v_means)
