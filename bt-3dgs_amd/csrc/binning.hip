@@ -121,51 +121,81 @@ __device__ __forceinline__ uint32_t box_3d(const T *__restrict__ means3d,
 constexpr int kCountThreads = 1024;
 constexpr int kCountItems = kScanTile / kCountThreads;
 
+// The whole scan when one block counts every item (at most kScanTile of
+// them): offsets[0 .. M] from the block's own counts, one launch fewer.
+// So few items are bound by their launches: 4k Gaussians of a 64 x 64 view,
+// projected, rasterized and back, take 176 us with the separate scans here
+// and in the sort (kDirectTiles) and 165 us without.
+__device__ __forceinline__ void scan_counts(const uint32_t (&c)[kCountItems], int64_t M,
+                                            int64_t *lds, int64_t *__restrict__ offsets) {
+  int64_t run = 0;
+#pragma unroll
+  for (int k = 0; k < kCountItems; ++k) {
+    int64_t total;
+    const int64_t before = block_exclusive_scan(static_cast<int64_t>(c[k]), lds, total);
+    const int64_t idx = static_cast<int64_t>(k) * kCountThreads + threadIdx.x;
+    if (idx < M) offsets[idx] = run + before;
+    run += total;
+  }
+  if (threadIdx.x == 0) offsets[M] = run;
+}
+
+// Ends a count kernel: the offsets themselves where one block counts every
+// item (`offsets` given), else the block's sum for the downsweep.
+__device__ __forceinline__ void finish_counts(const uint32_t (&c)[kCountItems], int64_t M,
+                                              int64_t *lds, int64_t *__restrict__ block_sums,
+                                              int64_t *__restrict__ offsets) {
+  if (offsets != nullptr) {
+    scan_counts(c, M, lds, offsets);
+    return;
+  }
+  int64_t s = 0, total;
+#pragma unroll
+  for (int k = 0; k < kCountItems; ++k) s += c[k];
+  block_exclusive_scan(s, lds, total);
+  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kCountThreads) void count_2d_kernel(
     const T *__restrict__ means2d, const int32_t *__restrict__ radii, int rect, int64_t M,
     uint32_t ts, uint32_t tw, uint32_t th, int32_t *__restrict__ counts,
-    int64_t *__restrict__ block_sums) {
+    int64_t *__restrict__ block_sums, int64_t *__restrict__ offsets) {
   __shared__ int64_t lds[kCountThreads / 64];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x;
-  int64_t s = 0;
+  uint32_t c[kCountItems] = {};
 #pragma unroll
   for (int k = 0; k < kCountItems; ++k) {
     const int64_t idx = base + k * kCountThreads;
     if (idx < M) {
       Rect r;
-      const uint32_t c = rect_2d(means2d, radii, rect, idx, ts, tw, th, r);
-      counts[idx] = static_cast<int32_t>(c);
-      s += c;
+      c[k] = rect_2d(means2d, radii, rect, idx, ts, tw, th, r);
+      counts[idx] = static_cast<int32_t>(c[k]);
     }
   }
-  int64_t total;
-  block_exclusive_scan(s, lds, total);
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
+  finish_counts(c, M, lds, block_sums, offsets);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kCountThreads) void count_3d_kernel(
     const T *__restrict__ means3d, const int32_t *__restrict__ radii, int64_t N, uint32_t ts,
     uint32_t n2, uint32_t n1, uint32_t n0, uint32_t z0, uint32_t z1,
-    int32_t *__restrict__ counts, int64_t *__restrict__ block_sums) {
+    int32_t *__restrict__ counts, int64_t *__restrict__ block_sums,
+    int64_t *__restrict__ offsets) {
   __shared__ int64_t lds[kCountThreads / 64];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x;
   const uint32_t n[3] = {n2, n1, n0};
-  int64_t s = 0;
+  uint32_t c[kCountItems] = {};
 #pragma unroll
   for (int k = 0; k < kCountItems; ++k) {
     const int64_t idx = base + k * kCountThreads;
     if (idx < N) {
       Box b;
-      const uint32_t c = box_3d(means3d, radii, idx, ts, n, z0, z1, b);
-      counts[idx] = static_cast<int32_t>(c);
-      s += c;
+      c[k] = box_3d(means3d, radii, idx, ts, n, z0, z1, b);
+      counts[idx] = static_cast<int32_t>(c[k]);
     }
   }
-  int64_t total;
-  block_exclusive_scan(s, lds, total);
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
+  finish_counts(c, N, lds, block_sums, offsets);
 }
 
 // Records per brick layer: each Gaussian's box adds its (dim2, dim1) area to
@@ -417,8 +447,21 @@ constexpr int kMaxDigits = 1 << kMaxPassBits;
 // from the device (the emission scan's total); with n > cap they write
 // nothing, so a caller may launch them before it knows n.
 
-// Digit histogram of one 4096-item tile, written digit-major:
-// hist[d * nblocks + tile] (zero rows for tiles past n).  Tiles are
+// For a short list each scatter block adds up the tiles' histograms itself;
+// above, a device-wide scan of the digit-major histogram gives every (digit,
+// tile) its start.  A short list is bound by its launches, and the scan is
+// two of them in every pass; the sums cost each block the whole histogram
+// out of L2, eight tiles at a time in a serial chain.  Binning a view, host
+// and device together, with the scan and with the sums: 57 -> 47 us at 256
+// keys and up to 178 tiles (643k records) but 57 -> 64 us at 354; at 1024
+// keys 57 -> 45 us at 25 tiles, 57 -> 49-56 us at 48, 58 -> 60 us at 92.
+// So: at most kDirectTiles tiles and kDirectWords histogram words.
+constexpr int64_t kDirectTiles = 128;
+constexpr int64_t kDirectWords = 65536;
+
+// Digit histogram of one 4096-item tile (zero rows for tiles past n) at
+// hist[d * digit_stride + tile * tile_stride]: digit-major (nblocks, 1) for
+// the device-wide scan, tile-major (1, digits) for the scatter's own sums.  Tiles are
 // XCD-contiguous (xcd_swizzle), so the blocks writing neighbouring words of
 // a digit's row share an L2.
 __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t *__restrict__ keys,
@@ -426,7 +469,9 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
                                                                   int64_t cap, uint32_t shift,
                                                                   uint32_t digits,
                                                                   uint32_t *__restrict__ hist,
-                                                                  uint32_t nblocks) {
+                                                                  uint32_t nblocks,
+                                                                  uint32_t digit_stride,
+                                                                  uint32_t tile_stride) {
   __shared__ uint32_t h[kMaxDigits];
   const int64_t n = *n_dev;
   if (n <= 0 || n > cap) return;
@@ -444,7 +489,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
     if (base + r * kSortThreads < n) atomicAdd(&h[(key[r] >> shift) & mask], 1u);
   __syncthreads();
   for (uint32_t d = threadIdx.x; d < digits; d += kSortThreads)
-    hist[static_cast<int64_t>(d) * nblocks + tile] = h[d];
+    hist[static_cast<int64_t>(d) * digit_stride + static_cast<int64_t>(tile) * tile_stride] = h[d];
 }
 
 // One block sorts its kSortTile items by digit in LDS (stable: waves in
@@ -466,7 +511,8 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ e_in,
     const uint32_t *__restrict__ gid_in, const int64_t *__restrict__ n_dev, int64_t cap,
     uint32_t shift, uint32_t bits,
-    const uint32_t *__restrict__ digit_offsets, uint32_t nblocks, uint32_t *__restrict__ keys_out,
+    const uint32_t *__restrict__ digit_offsets, uint32_t direct, uint32_t nblocks,
+    uint32_t *__restrict__ keys_out,
     uint32_t *__restrict__ e_out, uint32_t *__restrict__ gid_out,
     int64_t *__restrict__ keys_out64, int32_t *__restrict__ vals_out32,
     int32_t *__restrict__ src_out, int32_t *__restrict__ tile_offsets, uint32_t n_keys) {
@@ -511,10 +557,44 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   const uint32_t dk = (digits + kSortThreads - 1) / kSortThreads;
   const uint32_t d0 = threadIdx.x * dk;
   uint32_t gb[kDPT];
+  if (direct) {
+    // digit_offsets holds the tiles' histograms, tile-major: a digit's run of
+    // this tile starts after every record of the smaller digits and the
+    // digit's records in the tiles before.
+    uint32_t all[kDPT], mine = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < kDPT; ++j) {
-    const uint32_t d = min(d0 + j, digits - 1u);
-    gb[j] = digit_offsets[static_cast<int64_t>(d) * nblocks + tile];
+    for (uint32_t j = 0; j < kDPT; ++j) all[j] = gb[j] = 0;
+    for (uint32_t t0 = 0; t0 < nblocks; t0 += 8) {
+#pragma unroll
+      for (uint32_t j = 0; j < kDPT; ++j) {
+        const uint32_t d = d0 + j;
+        uint32_t v[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+          v[k] = digit_offsets[min(t0 + k, nblocks - 1u) * digits + min(d, digits - 1u)];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+          const uint32_t x = j < dk && d < digits && t0 + k < nblocks ? v[k] : 0u;
+          all[j] += x;
+          gb[j] += t0 + k < tile ? x : 0u;
+        }
+      }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kDPT; ++j) mine += all[j];
+    uint32_t records;
+    uint32_t run = block_exclusive_scan(mine, wsum, records);
+#pragma unroll
+    for (uint32_t j = 0; j < kDPT; ++j) {
+      gb[j] += run;
+      run += all[j];
+    }
+  } else {
+#pragma unroll
+    for (uint32_t j = 0; j < kDPT; ++j) {
+      const uint32_t d = min(d0 + j, digits - 1u);
+      gb[j] = digit_offsets[static_cast<int64_t>(d) * nblocks + tile];
+    }
   }
   // A single pass over the whole key (the caller passes tile_offsets only
   // then): block 0's run starts are the numbers of records with a smaller
@@ -741,15 +821,15 @@ inline uint32_t key_bits_for(int64_t n_keys) {
 template <bool kFirst, bool kFinal, bool kTwo>
 int launch_scatter_sized(uint32_t bits, bool key16, const uint32_t *kin, const uint32_t *ein,
                          const uint32_t *gin, const int64_t *n_dev, int64_t cap, uint32_t shift,
-                         const uint32_t *digit_offsets, uint32_t nb, uint32_t *kout,
+                         const uint32_t *digit_offsets, bool direct, uint32_t nb, uint32_t *kout,
                          uint32_t *eout, uint32_t *gout, int64_t *keys64, int32_t *vals32,
                          int32_t *src, int32_t *tile_offsets, uint32_t n_keys,
                          hipStream_t stream) {
 #define R2S_SCATTER_SIZED(DB, K16)                                                              \
   radix_scatter_kernel<kFirst, kFinal, kTwo, DB, K16><<<dim3(nb), dim3(kSortThreads), 0,      \
                                                        stream>>>(                             \
-      kin, ein, gin, n_dev, cap, shift, bits, digit_offsets, nb, kout, eout, gout, keys64,     \
-      vals32, src, tile_offsets, n_keys)
+      kin, ein, gin, n_dev, cap, shift, bits, digit_offsets, direct ? 1u : 0u, nb, kout, eout, \
+      gout, keys64, vals32, src, tile_offsets, n_keys)
   if (bits <= 8 && key16)
     R2S_SCATTER_SIZED(8, true);
   else if (kFirst && kFinal && bits <= 10 && key16)
@@ -763,13 +843,13 @@ int launch_scatter_sized(uint32_t bits, bool key16, const uint32_t *kin, const u
 int launch_scatter(bool first, bool last, bool two, uint32_t bits, bool key16,
                    const uint32_t *kin, const uint32_t *ein, const uint32_t *gin,
                    const int64_t *n_dev, int64_t cap, uint32_t shift,
-                   const uint32_t *digit_offsets, uint32_t nb, uint32_t *kout, uint32_t *eout,
-                   uint32_t *gout, int64_t *keys64, int32_t *vals32, int32_t *src,
+                   const uint32_t *digit_offsets, bool direct, uint32_t nb, uint32_t *kout,
+                   uint32_t *eout, uint32_t *gout, int64_t *keys64, int32_t *vals32, int32_t *src,
                    int32_t *tile_offsets, uint32_t n_keys, hipStream_t stream) {
 #define R2S_SCATTER_PASS(F, L, T)                                                                \
   return launch_scatter_sized<F, L, T>(bits, key16, kin, ein, gin, n_dev, cap, shift,           \
-                                       digit_offsets, nb, kout, eout, gout, keys64, vals32, src, \
-                                       tile_offsets, n_keys, stream)
+                                       digit_offsets, direct, nb, kout, eout, gout, keys64,      \
+                                       vals32, src, tile_offsets, n_keys, stream)
   if (first && last) {
     if (two) R2S_SCATTER_PASS(true, true, true);
     R2S_SCATTER_PASS(true, true, false);
@@ -808,19 +888,23 @@ int radix_sort(SortSpace &s, const int64_t *n_dev, int64_t cap, uint32_t key_bit
     const uint32_t bits = key_bits == 0 ? 1u : min(pbits, key_bits - shift);
     const uint32_t digits = 1u << bits;
     const int64_t n_hist = static_cast<int64_t>(nb) * digits;
-    radix_hist_kernel<<<dim3(nb), dim3(kSortThreads), 0, stream>>>(kin, n_dev, cap, shift,
-                                                                   digits, s.hist, nb);
-    R2S_RETURN_IF(device_exclusive_scan<uint32_t, uint32_t>(s.hist, n_hist, s.hist_scan, nullptr,
-                                                            s.partials, stream,
-                                                            "isect sort scan"));
+    const bool direct = s.nblocks <= kDirectTiles && n_hist <= kDirectWords;
+    radix_hist_kernel<<<dim3(nb), dim3(kSortThreads), 0, stream>>>(
+        kin, n_dev, cap, shift, digits, s.hist, nb, direct ? 1u : nb, direct ? digits : 1u);
+    if (direct)
+      R2S_RETURN_IF(check_launch("isect sort histogram"));
+    else
+      R2S_RETURN_IF(device_exclusive_scan<uint32_t, uint32_t>(s.hist, n_hist, s.hist_scan,
+                                                              nullptr, s.partials, stream,
+                                                              "isect sort scan"));
     const bool first = p == 0, last = p == passes - 1;
     uint32_t *kout = (p % 2 == 0) ? s.k1 : s.k0;
     if (last && keys64 == nullptr && passes == 1) kout = nullptr;
     uint32_t *eout = (p % 2 == 0) ? s.e1 : s.e0;
     uint32_t *gout = (p % 2 == 0) ? s.g1 : s.g0;
     R2S_RETURN_IF(launch_scatter(first, last, two, bits, key_bits <= 16, kin, ein, gin, n_dev,
-                                 cap, shift, s.hist_scan, nb, kout, eout, gout, keys64, vals32,
-                                 src, passes == 1 ? tile_offsets : nullptr,
+                                 cap, shift, direct ? s.hist : s.hist_scan, direct, nb, kout,
+                                 eout, gout, keys64, vals32, src, passes == 1 ? tile_offsets : nullptr,
                                  static_cast<uint32_t>(n_keys), stream));
     kin = kout;
     ein = eout;
@@ -868,9 +952,12 @@ int count_2d_impl(const T *means2d, const int32_t *radii, int rect, int64_t C, i
   R2S_RETURN_IF(check_workspace(ws, ws_bytes, count_space_bytes(M), name));
   Carver cv(ws);
   int64_t *partials = cv.take<int64_t>(scan_partials_count(M));
-  count_2d_kernel<T><<<dim3(static_cast<uint32_t>(ceil_div(M, kScanTile))), dim3(kCountThreads),
-                      0, stream>>>(means2d, radii, rect, M, ts, tw, th, counts, partials);
+  const int64_t blocks = ceil_div(M, kScanTile);
+  count_2d_kernel<T><<<dim3(static_cast<uint32_t>(blocks)), dim3(kCountThreads), 0, stream>>>(
+      means2d, radii, rect, M, ts, tw, th, counts, partials,
+      blocks == 1 ? offsets : nullptr);
   R2S_RETURN_IF(check_launch(name));
+  if (blocks == 1) return R2S_OK;
   return device_exclusive_scan_from_sums<int32_t, int64_t>(counts, M, offsets, offsets + M,
                                                            partials, stream, name);
 }
@@ -894,9 +981,12 @@ int count_3d_impl(const T *means3d, const int32_t *radii, int64_t N, uint32_t ts
   R2S_RETURN_IF(check_workspace(ws, ws_bytes, count_space_bytes(N), name));
   Carver cv(ws);
   int64_t *partials = cv.take<int64_t>(scan_partials_count(N));
-  count_3d_kernel<T><<<dim3(static_cast<uint32_t>(ceil_div(N, kScanTile))), dim3(kCountThreads),
-                      0, stream>>>(means3d, radii, N, ts, n2, n1, n0, z0, z1, counts, partials);
+  const int64_t blocks = ceil_div(N, kScanTile);
+  count_3d_kernel<T><<<dim3(static_cast<uint32_t>(blocks)), dim3(kCountThreads), 0, stream>>>(
+      means3d, radii, N, ts, n2, n1, n0, z0, z1, counts, partials,
+      blocks == 1 ? offsets : nullptr);
   R2S_RETURN_IF(check_launch(name));
+  if (blocks == 1) return R2S_OK;
   return device_exclusive_scan_from_sums<int32_t, int64_t>(counts, N, offsets, offsets + N,
                                                            partials, stream, name);
 }
