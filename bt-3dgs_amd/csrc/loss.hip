@@ -15,6 +15,8 @@
 //                     (w.r.t. mu_x, E[x^2], E[xy]) written for the backward,
 //                     and per-block sums of S, |x - y| and m |x - e|;
 //   loss_reduce_kernel the block sums in a fixed order (deterministic);
+//                     trainer_reduce_kernel the same beside the volume TV's,
+//                     the hierarchy term and the weighted total;
 //   ssim_bwd_kernel   the adjoint: separable passes over A, B, C and the
 //                     gradient  d/dx = s_l1 sgn(x - y) / n
 //                              - s_ssim (G*A + 2 x G*B + y G*C) / n
@@ -151,39 +153,81 @@ __global__ __launch_bounds__(kLossThreads) void ssim_fwd_kernel(
   }
 }
 
-// losses = {mean |x - y|, 1 - mean S, mean m |x - e|} from the block sums,
-// summed in double in a fixed order.
-__global__ __launch_bounds__(kLossThreads) void loss_reduce_kernel(const float *__restrict__ partials,
-                                                                   int64_t n_blocks, double inv_n,
-                                                                   float *__restrict__ losses) {
-  __shared__ double s_red[3][kLossThreads / 64];
-  double t[3] = {0, 0, 0};
-  for (int64_t b = threadIdx.x; b < n_blocks; b += kLossThreads) {
+// Sums of N interleaved columns of n block sums in double, in a fixed order;
+// valid in thread 0.
+template <int N>
+__device__ __forceinline__ void sum_partials(const float *__restrict__ partials, int64_t n,
+                                             double (&s)[N]) {
+  __shared__ double s_red[N][kLossThreads / 64];
+  double t[N] = {};
+  for (int64_t b = threadIdx.x; b < n; b += kLossThreads) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) t[k] += partials[3 * b + k];
+    for (int k = 0; k < N; ++k) t[k] += partials[N * b + k];
   }
-  const int w = static_cast<int>(threadIdx.x) / 64;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double s = wave_sum(t[k]);
-    if (lane_id() == 0) s_red[k][w] = s;
+  for (int k = 0; k < N; ++k) {
+    const double v = wave_sum(t[k]);
+    if (lane_id() == 0) s_red[k][threadIdx.x / 64] = v;
   }
   __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) s[k] = 0;
   if (threadIdx.x == 0) {
-    double s[3] = {0, 0, 0};
-    for (int k = 0; k < 3; ++k)
+    for (int k = 0; k < N; ++k)
       for (int j = 0; j < kLossThreads / 64; ++j) s[k] += s_red[k][j];
-    losses[0] = static_cast<float>(s[1] * inv_n);
-    losses[1] = static_cast<float>(1.0 - s[0] * inv_n);
-    losses[2] = static_cast<float>(s[2] * inv_n);
   }
 }
 
+// losses = {mean |x - y|, 1 - mean S, mean m |x - e|} from the block sums.
+__device__ __forceinline__ void projection_losses(const double (&s)[3], double inv_n, float *l) {
+  l[0] = static_cast<float>(s[1] * inv_n);
+  l[1] = static_cast<float>(1.0 - s[0] * inv_n);
+  l[2] = static_cast<float>(s[2] * inv_n);
+}
+
+__global__ __launch_bounds__(kLossThreads) void loss_reduce_kernel(const float *__restrict__ partials,
+                                                                   int64_t n_blocks, double inv_n,
+                                                                   float *__restrict__ losses) {
+  double s[3];
+  sum_partials<3>(partials, n_blocks, s);
+  if (threadIdx.x == 0) projection_losses(s, inv_n, losses);
+}
+
+// Every term of the trainer's loss and their weighted sum in one launch:
+// terms = {l1, 1 - ssim, edge, tv, hierarchy}, total = weights . terms
+// (summed in double).  A few microseconds of kernel; bound by its launch, as
+// were the two reductions, the concatenation and the dot product that it
+// replaces: the loss of 512^2 projections and a 64^3 volume, forward and
+// backward, 194 -> 162 us with the backward's scales formed in its kernels.
+__global__ __launch_bounds__(kLossThreads) void trainer_reduce_kernel(
+    const float *__restrict__ partials, int64_t n_blocks, double inv_n,
+    const float *__restrict__ tv_partials, int64_t n_tv, double tv_scale,
+    const float *__restrict__ hierarchy, const float *__restrict__ weights,
+    float *__restrict__ terms, float *__restrict__ total) {
+  double s[3], tv[1];
+  sum_partials<3>(partials, n_blocks, s);
+  sum_partials<1>(tv_partials, n_tv, tv);
+  if (threadIdx.x == 0) {
+    float l[5];
+    projection_losses(s, inv_n, l);
+    l[3] = static_cast<float>(tv[0] * tv_scale);
+    l[4] = hierarchy[0];
+    double t = 0;
+    for (int k = 0; k < 5; ++k) {
+      terms[k] = l[k];
+      t += static_cast<double>(weights[k]) * static_cast<double>(l[k]);
+    }
+    total[0] = static_cast<float>(t);
+  }
+}
+
+// upstream (optional): one factor for all three scales.
 __global__ __launch_bounds__(kLossThreads) void ssim_bwd_kernel(
     const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ e,
     const float *__restrict__ m, const float *__restrict__ A, const float *__restrict__ B,
     const float *__restrict__ C, int H, int W, Window win, float inv_n,
-    const float *__restrict__ scales, float *__restrict__ grad) {
+    const float *__restrict__ scales, const float *__restrict__ upstream,
+    float *__restrict__ grad) {
   __shared__ float s_in[3][kSpan * kSpan];
   __shared__ float s_h[3][kSpan * kTile];
   const int tiles_x = (W + kTile - 1) / kTile;
@@ -206,7 +250,9 @@ __global__ __launch_bounds__(kLossThreads) void ssim_bwd_kernel(
     for (int q = 0; q < 3; ++q) s_h[q][idx] = h[q];
   }
   __syncthreads();
-  const float s_l1 = scales[0] * inv_n, s_ssim = scales[1] * inv_n, s_edge = scales[2] * inv_n;
+  const float up = upstream != nullptr ? upstream[0] : 1.0f;
+  const float s_l1 = scales[0] * up * inv_n, s_ssim = scales[1] * up * inv_n,
+              s_edge = scales[2] * up * inv_n;
 #pragma unroll
   for (int k = 0; k < kPerThread; ++k) {
     const int o = threadIdx.x + k * kLossThreads;
@@ -272,23 +318,16 @@ __global__ __launch_bounds__(kLossThreads) void tv_fwd_kernel(const float *__res
 __global__ __launch_bounds__(kLossThreads) void sum_reduce_kernel(const float *__restrict__ partials,
                                                                   int64_t n, double scale,
                                                                   float *__restrict__ out) {
-  __shared__ double s_red[kLossThreads / 64];
-  double t = 0;
-  for (int64_t b = threadIdx.x; b < n; b += kLossThreads) t += partials[b];
-  t = wave_sum(t);
-  if (lane_id() == 0) s_red[threadIdx.x / 64] = t;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0;
-    for (int k = 0; k < kLossThreads / 64; ++k) s += s_red[k];
-    out[0] = static_cast<float>(s * scale);
-  }
+  double s[1];
+  sum_partials<1>(partials, n, s);
+  if (threadIdx.x == 0) out[0] = static_cast<float>(s[0] * scale);
 }
 
 // d tv / d v = scale * sum over axes of sgn(v - v_prev) - sgn(v_next - v).
 __global__ __launch_bounds__(kLossThreads) void tv_bwd_kernel(const float *__restrict__ v, int D0,
                                                               int D1, int D2,
                                                               const float *__restrict__ grad_out,
+                                                              const float *__restrict__ upstream,
                                                               float scale,
                                                               float *__restrict__ grad) {
   const int64_t n = static_cast<int64_t>(D0) * D1 * D2, plane = static_cast<int64_t>(D1) * D2;
@@ -304,7 +343,7 @@ __global__ __launch_bounds__(kLossThreads) void tv_bwd_kernel(const float *__res
   if (b + 1 < D1) g -= sgn(v[i + D2] - x);
   if (c > 0) g += sgn(x - v[i - 1]);
   if (c + 1 < D2) g -= sgn(v[i + 1] - x);
-  grad[i] = g * (grad_out[0] * scale);
+  grad[i] = g * (grad_out[0] * (upstream != nullptr ? upstream[0] : 1.0f) * scale);
 }
 
 int64_t tv_terms(int D0, int D1, int D2) {
@@ -459,6 +498,87 @@ int check_tv_args(int D0, int D1, int D2, const char *what) {
   return R2S_OK;
 }
 
+// The projection loss' images, as its entry points take them.
+struct Images {
+  const float *render, *target, *edge_target, *edge_mask;
+  int64_t n;
+  int H, W;
+  int64_t pixels() const { return n * H * W; }
+  int tiles() const { return static_cast<int>(ceil_div(H, kTile) * ceil_div(W, kTile)); }
+};
+
+int launch_ssim_fwd(const Images &im, const Window &win, const LossSpace &s, hipStream_t stream,
+                    const char *what) {
+  ssim_fwd_kernel<<<dim3(im.tiles(), static_cast<uint32_t>(im.n)), dim3(kLossThreads), 0,
+                    stream>>>(im.render, im.target, im.edge_target, im.edge_mask, im.H, im.W, win,
+                              s.A, s.B, s.C, s.partials);
+  return check_launch(what);
+}
+
+int launch_ssim_bwd(const Images &im, const Window &win, const LossSpace &s, const float *scales,
+                    const float *upstream, float *v_render, hipStream_t stream,
+                    const char *what) {
+  ssim_bwd_kernel<<<dim3(im.tiles(), static_cast<uint32_t>(im.n)), dim3(kLossThreads), 0,
+                    stream>>>(im.render, im.target, im.edge_target, im.edge_mask, s.A, s.B, s.C,
+                              im.H, im.W, win,
+                              static_cast<float>(1.0 / static_cast<double>(im.pixels())), scales,
+                              upstream, v_render);
+  return check_launch(what);
+}
+
+// Blocks (and block sums) of the TV forward over n > 0 voxels.
+int64_t tv_blocks(int64_t n) { return std::min<int64_t>(kTvBlocks, ceil_div(n, kLossThreads)); }
+
+int launch_tv_fwd(const float *volume, int D0, int D1, int D2, float *partials,
+                  hipStream_t stream, const char *what) {
+  const int64_t n = static_cast<int64_t>(D0) * D1 * D2;
+  tv_fwd_kernel<<<dim3(static_cast<uint32_t>(tv_blocks(n))), dim3(kLossThreads), 0, stream>>>(
+      volume, D0, D1, D2, partials);
+  return check_launch(what);
+}
+
+// loss.py:19-20: mean divides by max(1, number of differences).
+double tv_scale(int D0, int D1, int D2, int mean) {
+  const int64_t terms = tv_terms(D0, D1, D2);
+  return mean ? 1.0 / static_cast<double>(terms > 1 ? terms : 1) : 1.0;
+}
+
+int launch_tv_bwd(const float *volume, int D0, int D1, int D2, int mean, const float *grad_out,
+                  const float *upstream, float *v_volume, hipStream_t stream, const char *what) {
+  const int64_t n = static_cast<int64_t>(D0) * D1 * D2;
+  tv_bwd_kernel<<<dim3(static_cast<uint32_t>(ceil_div(n, kLossThreads))), dim3(kLossThreads), 0,
+                  stream>>>(volume, D0, D1, D2, grad_out, upstream,
+                            static_cast<float>(tv_scale(D0, D1, D2, mean)), v_volume);
+  return check_launch(what);
+}
+
+struct TrainerSpace {
+  LossSpace loss;
+  float *tv;
+};
+
+TrainerSpace carve_trainer(Carver &cv, int64_t n_images, int H, int W) {
+  TrainerSpace s;
+  s.loss = carve_loss(cv, n_images, H, W);
+  s.tv = cv.take<float>(kTvBlocks);
+  return s;
+}
+
+int check_images(const Images &im, const char *what) {
+  R2S_RETURN_IF(check_loss_args(im.n, im.H, im.W, what));
+  R2S_REQUIRE((im.edge_target == nullptr) == (im.edge_mask == nullptr),
+              "%s: edge_target and edge_mask go together", what);
+  return R2S_OK;
+}
+
+int check_loss_workspace(const void *ws, size_t have, int64_t need, const char *what) {
+  if (ws == nullptr || static_cast<int64_t>(have) < need) {
+    set_error("%s: workspace of %zu bytes, %lld required", what, have, (long long)need);
+    return R2S_EWORKSPACE;
+  }
+  return R2S_OK;
+}
+
 }  // namespace
 }  // namespace r2s
 
@@ -549,14 +669,9 @@ int r2s_tv_fwd_f32(const float *volume, int32_t D0, int32_t D1, int32_t D2, int3
     return R2S_EWORKSPACE;
   }
   float *partials = static_cast<float *>(workspace);
-  const int64_t blocks = std::min<int64_t>(r2s::kTvBlocks, r2s::ceil_div(n, r2s::kLossThreads));
-  r2s::tv_fwd_kernel<<<dim3(static_cast<uint32_t>(blocks)), dim3(r2s::kLossThreads), 0,
-                       stream>>>(volume, D0, D1, D2, partials);
-  R2S_RETURN_IF(r2s::check_launch(what));
-  // loss.py:19-20: mean divides by max(1, number of differences).
-  const int64_t terms = r2s::tv_terms(D0, D1, D2);
-  const double scale = mean ? 1.0 / static_cast<double>(terms > 1 ? terms : 1) : 1.0;
-  r2s::sum_reduce_kernel<<<1, r2s::kLossThreads, 0, stream>>>(partials, blocks, scale, out);
+  R2S_RETURN_IF(r2s::launch_tv_fwd(volume, D0, D1, D2, partials, stream, what));
+  r2s::sum_reduce_kernel<<<1, r2s::kLossThreads, 0, stream>>>(
+      partials, r2s::tv_blocks(n), r2s::tv_scale(D0, D1, D2, mean), out);
   return r2s::check_launch(what);
 }
 
@@ -568,14 +683,8 @@ int r2s_tv_bwd_f32(const float *volume, int32_t D0, int32_t D1, int32_t D2, int3
   const int64_t n = static_cast<int64_t>(D0) * D1 * D2;
   if (n == 0) return R2S_OK;
   R2S_REQUIRE(volume && grad_out && v_volume, "%s: null pointer", what);
-  const int64_t terms = r2s::tv_terms(D0, D1, D2);
-  const float scale =
-      mean ? static_cast<float>(1.0 / static_cast<double>(terms > 1 ? terms : 1)) : 1.0f;
-  r2s::tv_bwd_kernel<<<dim3(static_cast<uint32_t>(r2s::ceil_div(n, r2s::kLossThreads))),
-                       dim3(r2s::kLossThreads), 0, r2s::as_stream(st)>>>(volume, D0, D1, D2,
-                                                                         grad_out, scale,
-                                                                         v_volume);
-  return r2s::check_launch(what);
+  return r2s::launch_tv_bwd(volume, D0, D1, D2, mean, grad_out, nullptr, v_volume,
+                            r2s::as_stream(st), what);
 }
 
 int64_t r2s_projection_loss_workspace_bytes(int64_t n_images, int32_t H, int32_t W) {
@@ -591,31 +700,21 @@ int r2s_projection_loss_fwd_f32(const float *render, const float *target,
                                 r2s_stream_t st) {
   r2s::clear_error();
   const char *what = "projection_loss_fwd";
-  R2S_RETURN_IF(r2s::check_loss_args(n_images, H, W, what));
+  const r2s::Images im{render, target, edge_target, edge_mask, n_images, H, W};
+  R2S_RETURN_IF(r2s::check_images(im, what));
   r2s::Window win;
   R2S_RETURN_IF(r2s::make_window(window_size, win, what));
   R2S_REQUIRE(losses != nullptr, "%s: null losses", what);
-  R2S_REQUIRE((edge_target == nullptr) == (edge_mask == nullptr),
-              "%s: edge_target and edge_mask go together", what);
-  const int64_t npix = n_images * H * W;
-  R2S_REQUIRE(npix > 0, "%s: empty images (the reference's mean is NaN)", what);
+  R2S_REQUIRE(im.pixels() > 0, "%s: empty images (the reference's mean is NaN)", what);
   R2S_REQUIRE(render && target, "%s: null image", what);
-  const int64_t need = r2s_projection_loss_workspace_bytes(n_images, H, W);
-  if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need) {
-    r2s::set_error("%s: workspace of %zu bytes, %lld required", what, workspace_bytes,
-                   (long long)need);
-    return R2S_EWORKSPACE;
-  }
+  R2S_RETURN_IF(r2s::check_loss_workspace(
+      workspace, workspace_bytes, r2s_projection_loss_workspace_bytes(n_images, H, W), what));
   r2s::Carver cv(workspace);
   const r2s::LossSpace s = r2s::carve_loss(cv, n_images, H, W);
-  const int tiles = static_cast<int>(r2s::ceil_div(H, r2s::kTile) * r2s::ceil_div(W, r2s::kTile));
   hipStream_t stream = r2s::as_stream(st);
-  r2s::ssim_fwd_kernel<<<dim3(tiles, static_cast<uint32_t>(n_images)), dim3(r2s::kLossThreads), 0,
-                         stream>>>(render, target, edge_target, edge_mask, H, W, win, s.A, s.B,
-                                   s.C, s.partials);
-  R2S_RETURN_IF(r2s::check_launch(what));
+  R2S_RETURN_IF(r2s::launch_ssim_fwd(im, win, s, stream, what));
   r2s::loss_reduce_kernel<<<1, r2s::kLossThreads, 0, stream>>>(
-      s.partials, n_images * tiles, 1.0 / static_cast<double>(npix), losses);
+      s.partials, n_images * im.tiles(), 1.0 / static_cast<double>(im.pixels()), losses);
   return r2s::check_launch(what);
 }
 
@@ -626,29 +725,86 @@ int r2s_projection_loss_bwd_f32(const float *render, const float *target,
                                 size_t workspace_bytes, float *v_render, r2s_stream_t st) {
   r2s::clear_error();
   const char *what = "projection_loss_bwd";
-  R2S_RETURN_IF(r2s::check_loss_args(n_images, H, W, what));
+  const r2s::Images im{render, target, edge_target, edge_mask, n_images, H, W};
+  R2S_RETURN_IF(r2s::check_images(im, what));
   r2s::Window win;
   R2S_RETURN_IF(r2s::make_window(window_size, win, what));
-  R2S_REQUIRE((edge_target == nullptr) == (edge_mask == nullptr),
-              "%s: edge_target and edge_mask go together", what);
-  const int64_t npix = n_images * H * W;
-  if (npix == 0) return R2S_OK;
+  if (im.pixels() == 0) return R2S_OK;
   R2S_REQUIRE(render && target && grad_scales && v_render, "%s: null pointer", what);
-  const int64_t need = r2s_projection_loss_workspace_bytes(n_images, H, W);
-  if (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need) {
-    r2s::set_error("%s: workspace of %zu bytes, %lld required", what, workspace_bytes,
-                   (long long)need);
-    return R2S_EWORKSPACE;
-  }
+  R2S_RETURN_IF(r2s::check_loss_workspace(
+      workspace, workspace_bytes, r2s_projection_loss_workspace_bytes(n_images, H, W), what));
   r2s::Carver cv(const_cast<void *>(workspace));
-  const r2s::LossSpace s = r2s::carve_loss(cv, n_images, H, W);
-  const int tiles = static_cast<int>(r2s::ceil_div(H, r2s::kTile) * r2s::ceil_div(W, r2s::kTile));
-  r2s::ssim_bwd_kernel<<<dim3(tiles, static_cast<uint32_t>(n_images)), dim3(r2s::kLossThreads), 0,
-                         r2s::as_stream(st)>>>(render, target, edge_target, edge_mask, s.A, s.B,
-                                               s.C, H, W, win,
-                                               static_cast<float>(1.0 / static_cast<double>(npix)),
-                                               grad_scales, v_render);
+  return r2s::launch_ssim_bwd(im, win, r2s::carve_loss(cv, n_images, H, W), grad_scales, nullptr,
+                              v_render, r2s::as_stream(st), what);
+}
+
+int64_t r2s_trainer_loss_workspace_bytes(int64_t n_images, int32_t H, int32_t W) {
+  r2s::Carver cv(nullptr);
+  r2s::carve_trainer(cv, n_images > 0 ? n_images : 0, H > 0 ? H : 0, W > 0 ? W : 0);
+  return static_cast<int64_t>(cv.used);
+}
+
+int r2s_trainer_loss_fwd_f32(const float *render, const float *target, const float *edge_target,
+                             const float *edge_mask, int64_t n_images, int32_t H, int32_t W,
+                             int32_t window_size, const float *volume, int32_t D0, int32_t D1,
+                             int32_t D2, int32_t tv_mean, const float *hierarchy,
+                             const float *weights, float *terms, float *total, void *workspace,
+                             size_t workspace_bytes, r2s_stream_t st) {
+  r2s::clear_error();
+  const char *what = "trainer_loss_fwd";
+  const r2s::Images im{render, target, edge_target, edge_mask, n_images, H, W};
+  R2S_RETURN_IF(r2s::check_images(im, what));
+  R2S_RETURN_IF(r2s::check_tv_args(D0, D1, D2, what));
+  r2s::Window win;
+  R2S_RETURN_IF(r2s::make_window(window_size, win, what));
+  R2S_REQUIRE(hierarchy && weights && terms && total, "%s: null pointer", what);
+  R2S_REQUIRE(im.pixels() > 0, "%s: empty images (the reference's mean is NaN)", what);
+  R2S_REQUIRE(render && target, "%s: null image", what);
+  R2S_RETURN_IF(r2s::check_loss_workspace(workspace, workspace_bytes,
+                                          r2s_trainer_loss_workspace_bytes(n_images, H, W), what));
+  r2s::Carver cv(workspace);
+  const r2s::TrainerSpace s = r2s::carve_trainer(cv, n_images, H, W);
+  hipStream_t stream = r2s::as_stream(st);
+  R2S_RETURN_IF(r2s::launch_ssim_fwd(im, win, s.loss, stream, what));
+  const int64_t n_tv = volume == nullptr ? 0 : static_cast<int64_t>(D0) * D1 * D2;
+  if (n_tv > 0) R2S_RETURN_IF(r2s::launch_tv_fwd(volume, D0, D1, D2, s.tv, stream, what));
+  r2s::trainer_reduce_kernel<<<1, r2s::kLossThreads, 0, stream>>>(
+      s.loss.partials, n_images * im.tiles(), 1.0 / static_cast<double>(im.pixels()), s.tv,
+      r2s::tv_blocks(n_tv), n_tv > 0 ? r2s::tv_scale(D0, D1, D2, tv_mean) : 0.0, hierarchy,
+      weights, terms, total);
   return r2s::check_launch(what);
+}
+
+int r2s_trainer_loss_bwd_f32(const float *render, const float *target, const float *edge_target,
+                             const float *edge_mask, int64_t n_images, int32_t H, int32_t W,
+                             int32_t window_size, const float *volume, int32_t D0, int32_t D1,
+                             int32_t D2, int32_t tv_mean, const float *weights,
+                             const float *grad_total, const void *workspace,
+                             size_t workspace_bytes, float *v_render, float *v_volume,
+                             r2s_stream_t st) {
+  r2s::clear_error();
+  const char *what = "trainer_loss_bwd";
+  const r2s::Images im{render, target, edge_target, edge_mask, n_images, H, W};
+  R2S_RETURN_IF(r2s::check_images(im, what));
+  R2S_RETURN_IF(r2s::check_tv_args(D0, D1, D2, what));
+  r2s::Window win;
+  R2S_RETURN_IF(r2s::make_window(window_size, win, what));
+  R2S_REQUIRE(weights && grad_total, "%s: null pointer", what);
+  hipStream_t stream = r2s::as_stream(st);
+  if (v_render != nullptr && im.pixels() > 0) {
+    R2S_REQUIRE(render && target, "%s: null image", what);
+    R2S_RETURN_IF(r2s::check_loss_workspace(
+        workspace, workspace_bytes, r2s_trainer_loss_workspace_bytes(n_images, H, W), what));
+    r2s::Carver cv(const_cast<void *>(workspace));
+    R2S_RETURN_IF(r2s::launch_ssim_bwd(im, win, r2s::carve_trainer(cv, n_images, H, W).loss,
+                                       weights, grad_total, v_render, stream, what));
+  }
+  if (v_volume != nullptr && static_cast<int64_t>(D0) * D1 * D2 > 0) {
+    R2S_REQUIRE(volume != nullptr, "%s: null volume", what);
+    R2S_RETURN_IF(r2s::launch_tv_bwd(volume, D0, D1, D2, tv_mean, weights + 3, grad_total,
+                                     v_volume, stream, what));
+  }
+  return R2S_OK;
 }
 
 }  // extern "C"

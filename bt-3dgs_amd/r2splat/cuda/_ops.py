@@ -1700,11 +1700,7 @@ def _loss_images(t: Tensor, name: str) -> Tensor:
     return t.contiguous()
 
 
-def projection_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Tensor],
-                        edge_mask: Optional[Tensor], window_size: int = 11):
-    """Losses [3] = (mean |r - t|, 1 - mean SSIM(r, t), mean m |r - e|) over
-    images [n, H, W] (loss.py:135-172, metric.py:36-54), and the workspace the
-    backward needs."""
+def _loss_inputs(render, target, edge_target, edge_mask):
     r = _loss_images(render, "render")
     _check(r.dim() == 3, "render must be [n, H, W]")
     t = _loss_images(target, "target")
@@ -1717,6 +1713,15 @@ def projection_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Te
         m = _loss_images(edge_mask, "edge_mask")
         _check(e.shape == r.shape and m.shape == r.shape,
                "edge_target and edge_mask must have the render's shape")
+    return r, t, e, m
+
+
+def projection_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Tensor],
+                        edge_mask: Optional[Tensor], window_size: int = 11):
+    """Losses [3] = (mean |r - t|, 1 - mean SSIM(r, t), mean m |r - e|) over
+    images [n, H, W] (loss.py:135-172, metric.py:36-54), and the workspace the
+    backward needs."""
+    r, t, e, m = _loss_inputs(render, target, edge_target, edge_mask)
     n, H, W = r.shape
     dev = r.device
     lib = _lib()
@@ -1781,6 +1786,59 @@ def tv_bwd(volume: Tensor, grad_out: Tensor, mean: bool = True) -> Tensor:
         _call("r2s_tv_bwd_f32", _ptr(v), *v.shape, int(bool(mean)), _ptr(g), _ptr(out),
               _stream(dev))
     return out
+
+
+# ----------------------------------------------------------- trainer loss --
+
+def trainer_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Tensor],
+                     edge_mask: Optional[Tensor], volume: Optional[Tensor], hierarchy: Tensor,
+                     weights: Tensor, window_size: int = 11, tv_mean: bool = True):
+    """projection_loss_fwd, tv_fwd (zero without a volume), the one-element
+    hierarchy term and their weighted sum: (terms [5] = (l1, 1 - ssim, edge,
+    tv, hierarchy), total, workspace for trainer_loss_bwd)."""
+    r, t, e, m = _loss_inputs(render, target, edge_target, edge_mask)
+    v = None if volume is None else _tv_volume(volume)
+    _check(isinstance(hierarchy, torch.Tensor) and hierarchy.is_cuda,
+           "hierarchy must be a CUDA tensor")
+    _check(hierarchy.numel() == 1, "hierarchy must hold one value")
+    h = _loss_images(hierarchy.to(torch.float32), "hierarchy")
+    w = _loss_images(weights, "weights")
+    _check(w.numel() == 5, "weights must hold five values")
+    dev = r.device
+    _check(h.device == dev, "hierarchy must be on the render's device")
+    n, H, W = r.shape
+    terms = torch.empty(5, dtype=torch.float32, device=dev)
+    total = torch.empty((), dtype=torch.float32, device=dev)
+    with _on(dev):
+        ws = _workspace(_lib().r2s_trainer_loss_workspace_bytes(n, H, W), dev)
+        _call("r2s_trainer_loss_fwd_f32", _ptr(r), _ptr(t), _ptr(e), _ptr(m), n, H, W,
+              int(window_size), _ptr(v), *((0, 0, 0) if v is None else v.shape),
+              int(bool(tv_mean)), _ptr(h), _ptr(w), _ptr(terms), _ptr(total), _ptr(ws),
+              ws.numel(), _stream(dev))
+    return terms, total, ws
+
+
+def trainer_loss_bwd(render: Tensor, target: Tensor, edge_target: Optional[Tensor],
+                     edge_mask: Optional[Tensor], volume: Optional[Tensor], weights: Tensor,
+                     grad_total: Tensor, workspace: Tensor, window_size: int = 11,
+                     tv_mean: bool = True, want_render: bool = True, want_volume: bool = True):
+    """(v_render or None, v_volume or None) of trainer_loss_fwd's total for
+    its upstream gradient."""
+    r, t, e, m = _loss_inputs(render, target, edge_target, edge_mask)
+    v = None if volume is None else _tv_volume(volume)
+    w = _loss_images(weights, "weights")
+    g = _loss_images(grad_total, "grad_total")
+    _check(w.numel() == 5 and g.numel() == 1, "weights must hold five values, grad_total one")
+    n, H, W = r.shape
+    dev = r.device
+    v_r = torch.empty_like(r) if want_render else None
+    v_v = torch.empty_like(v) if want_volume and v is not None else None
+    with _on(dev):
+        _call("r2s_trainer_loss_bwd_f32", _ptr(r), _ptr(t), _ptr(e), _ptr(m), n, H, W,
+              int(window_size), _ptr(v), *((0, 0, 0) if v is None else v.shape),
+              int(bool(tv_mean)), _ptr(w), _ptr(g), _ptr(workspace), workspace.numel(),
+              _ptr(v_r), _ptr(v_v), _stream(dev))
+    return v_r, v_v
 
 
 # --------------------------------------------------------- hierarchy loss --

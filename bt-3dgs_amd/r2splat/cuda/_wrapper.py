@@ -49,6 +49,8 @@ densify_duplicate = _make_cuda_func("densify_duplicate")
 densify_remove = _make_cuda_func("densify_remove")
 projection_loss_fwd = _make_cuda_func("projection_loss_fwd")
 projection_loss_bwd = _make_cuda_func("projection_loss_bwd")
+trainer_loss_fwd = _make_cuda_func("trainer_loss_fwd")
+trainer_loss_bwd = _make_cuda_func("trainer_loss_bwd")
 tv_fwd = _make_cuda_func("tv_fwd")
 tv_bwd = _make_cuda_func("tv_bwd")
 hierarchy_loss_fwd = _make_cuda_func("hierarchy_loss_fwd")

@@ -84,10 +84,11 @@ _WEIGHTS = {}
 
 class _TrainerLoss(torch.autograd.Function):
     """The loss computers' terms and weighted total as outputs of one graph
-    node: forward = the projection-loss launch, the TV launch and one
-    weighted sum; backward = the effective scale of each term (its own
-    upstream gradient plus its weight times the total's), then one
-    projection-loss launch and one TV launch.  Terms are ordered (l1, ssim,
+    node: forward = the projection-loss launch, the TV launch and one launch
+    for every reduction, the terms and their weighted sum; backward = one
+    projection-loss launch and one TV launch, which form each term's scale
+    from its weight and the total's upstream gradient (a term's own upstream
+    gradient, where it has one, is added to it first).  Terms are ordered (l1, ssim,
     edge, tv, hierarchy); the hierarchy term is an input (computed by the
     caller), so its gradient is passed back."""
 
@@ -96,11 +97,8 @@ class _TrainerLoss(torch.autograd.Function):
         # Outputs that receive no gradient (the terms, in a trainer's
         # total.backward()) pass None instead of a zero tensor each.
         ctx.set_materialize_grads(False)
-        losses, ws = W.projection_loss_fwd(r, t, e, m, window_size)
-        z = _zero(r.device).reshape(1)
-        tv = z if vol is None else W.tv_fwd(vol, tv_mean).reshape(1)
-        terms = torch.cat((losses, tv, hier.detach().reshape(1).to(torch.float32)))
-        total = torch.dot(terms, weights)
+        terms, total, ws = W.trainer_loss_fwd(r, t, e, m, vol, hier.detach(), weights,
+                                              window_size, tv_mean)
         ctx.save_for_backward(weights, r, t, e, m, ws, vol)
         ctx.window_size, ctx.tv_mean = window_size, tv_mean
         ctx.hier_dtype, ctx.hier_shape = hier.dtype, hier.shape
@@ -116,10 +114,17 @@ class _TrainerLoss(torch.autograd.Function):
         if g_total is None:
             g_total = _zero(dev)
         if g_l1 is None and g_ssim is None and g_edge is None and g_tv is None:
-            eff = weights * g_total.to(torch.float32)
-        else:
-            own = _grad_vector((g_l1, g_ssim, g_edge, g_tv, None), dev)
-            eff = torch.addcmul(own, weights, g_total.to(torch.float32))
+            # The total alone, a trainer's case: the kernels form the scales.
+            g = g_total.to(torch.float32)
+            v_r, v_vol = W.trainer_loss_bwd(r, t, e, m, vol, weights, g, ws, ctx.window_size,
+                                            ctx.tv_mean, ctx.needs_input_grad[1],
+                                            ctx.needs_input_grad[5])
+            v_hier = None
+            if ctx.needs_input_grad[6]:
+                v_hier = (weights[4] * g).reshape(ctx.hier_shape).to(ctx.hier_dtype)
+            return None, v_r, None, None, None, v_vol, v_hier, None, None
+        own = _grad_vector((g_l1, g_ssim, g_edge, g_tv, None), dev)
+        eff = torch.addcmul(own, weights, g_total.to(torch.float32))
         v_r = None
         if ctx.needs_input_grad[1]:
             v_r = W.projection_loss_bwd(r, t, e, m, eff[:3], ws, ctx.window_size)

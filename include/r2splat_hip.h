@@ -1036,6 +1036,37 @@ int r2s_tv_bwd_f32(const float *volume, int32_t D0, int32_t D1, int32_t D2,
                    r2s_stream_t stream);
 
 /* ---------------------------------------------------------------------- */
+/* The trainer's whole loss                                                */
+/* ---------------------------------------------------------------------- */
+
+/* Workspace of r2s_trainer_loss_fwd/bwd; keep it between the two calls. */
+int64_t r2s_trainer_loss_workspace_bytes(int64_t n_images, int32_t H, int32_t W);
+
+/* src/utils/loss.py:105-172: the projection losses of
+ * r2s_projection_loss_fwd_f32, the TV of r2s_tv_fwd_f32 (0 for a NULL or
+ * empty volume) and the caller's hierarchy term hierarchy[0] (device) ->
+ * terms[5] = {l1, 1 - ssim, edge, tv, hierarchy} and total[0] =
+ * weights[5] . terms, all on the device. */
+int r2s_trainer_loss_fwd_f32(const float *render, const float *target,
+                             const float *edge_target, const float *edge_mask,
+                             int64_t n_images, int32_t H, int32_t W, int32_t window_size,
+                             const float *volume, int32_t D0, int32_t D1, int32_t D2,
+                             int32_t tv_mean, const float *hierarchy, const float *weights,
+                             float *terms, float *total, void *workspace,
+                             size_t workspace_bytes, r2s_stream_t stream);
+
+/* Its VJP for the total's upstream gradient grad_total[0] (device): each
+ * term's scale is weights[k] * grad_total[0].  v_render and v_volume may be
+ * NULL (not wanted).  Reads the workspace the forward filled. */
+int r2s_trainer_loss_bwd_f32(const float *render, const float *target,
+                             const float *edge_target, const float *edge_mask,
+                             int64_t n_images, int32_t H, int32_t W, int32_t window_size,
+                             const float *volume, int32_t D0, int32_t D1, int32_t D2,
+                             int32_t tv_mean, const float *weights, const float *grad_total,
+                             const void *workspace, size_t workspace_bytes, float *v_render,
+                             float *v_volume, r2s_stream_t stream);
+
+/* ---------------------------------------------------------------------- */
 /* Hierarchy loss                                                          */
 /* ---------------------------------------------------------------------- */
 
