@@ -502,10 +502,16 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
 // keys_out64 null (a caller keeping only the tile offsets) the keys go to
 // keys_out when it is given (for a later offset search) and nowhere else.
 // The LDS footprint follows the sort: digit tables for 2^kDBits digits,
-// keys staged as 16 bits when every key fits (kKey16), and in a single-pass
-// sort the emission index staged as its 16-bit block-local position.  At
-// config 4 (one 10-bit pass) and config 3 (two passes of 8 and 7 bits over
-// 15-bit keys) that leaves room for three blocks per CU instead of two.
+// keys staged as 16 bits when every key fits (kKey16), and in the first pass
+// the emission index staged as its 16-bit block-local position.  At config 4
+// (one 10-bit pass) and config 3 (two passes of 8 and 7 bits over 15-bit
+// keys) that leaves room for three blocks per CU instead of two, and in the
+// first of two 9-bit passes too (18-bit keys, a 512^3 volume's bricks): with
+// the nine ballots a digit needs instead of the 2048-digit table's eleven,
+// that pass took 348 -> 297 us for 39 M records and the second 421 -> 409 us,
+// which stays at two blocks (a third, with the emission index staged after
+// the ids in the same words, left it at 411 us: its runs of a few records
+// per digit bound it at the stores).
 template <bool kFirst, bool kFinal, bool kTwo, int kDBits, bool kKey16>
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ e_in,
@@ -519,7 +525,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   static_assert(kDBits >= 8 && kDBits <= kMaxPassBits, "digit tables of 256 to 2048");
   constexpr int kD = 1 << kDBits;
   constexpr int kDPT = kD / kSortThreads;  // digits per thread in the scan
-  constexpr bool kLocalE = kFirst && kFinal;
+  constexpr bool kLocalE = kFirst;  // e is the input index
   using KeyS = typename std::conditional<kKey16, uint16_t, uint32_t>::type;
   using ES = typename std::conditional<kLocalE, uint16_t, uint32_t>::type;
   // Per-wave digit counters, then (in place) each wave's start within the
@@ -704,7 +710,8 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
     } else {
       keys_out[dest] = k;
       gid_out[dest] = s_gid[lp];
-      if (kTwo) e_out[dest] = s_e[lp];
+      if (kTwo)
+        e_out[dest] = kLocalE ? static_cast<uint32_t>(block_first) + s_e[lp] : s_e[lp];
     }
   }
 }
@@ -816,8 +823,8 @@ inline uint32_t key_bits_for(int64_t n_keys) {
   return b;
 }
 
-// Launches the scatter instantiation for one pass: digit tables of 256,
-// 1024 (a single pass) or 2048 digits, 16-bit key staging when the keys fit.
+// Launches the scatter instantiation for one pass: digit tables of 256, 512
+// (one of several passes), 1024 (a single pass) or 2048 digits, 16-bit key staging when the keys fit.
 template <bool kFirst, bool kFinal, bool kTwo>
 int launch_scatter_sized(uint32_t bits, bool key16, const uint32_t *kin, const uint32_t *ein,
                          const uint32_t *gin, const int64_t *n_dev, int64_t cap, uint32_t shift,
@@ -834,6 +841,8 @@ int launch_scatter_sized(uint32_t bits, bool key16, const uint32_t *kin, const u
     R2S_SCATTER_SIZED(8, true);
   else if (kFirst && kFinal && bits <= 10 && key16)
     R2S_SCATTER_SIZED(10, true);
+  else if (!(kFirst && kFinal) && bits <= 9)
+    R2S_SCATTER_SIZED(9, false);
   else
     R2S_SCATTER_SIZED(kMaxPassBits, false);
 #undef R2S_SCATTER_SIZED

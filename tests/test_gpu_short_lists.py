@@ -1,7 +1,8 @@
 """Binning of lists short enough for the forms with fewer launches: one count
 block storing the offsets itself (at most 4096 items), and sort tiles of 4096
 records (up to 128 of them, and 65536 digit counts) whose histograms the
-scatter adds up itself.  Whole numbers: every list equals the oracle's."""
+scatter adds up itself; and the sort's 9-bit passes.  Whole numbers: every
+list equals the oracle's."""
 
 import numpy as np
 import pytest
@@ -66,4 +67,20 @@ def test_bricks(bricks, n):
     offsets = binning.isect_offset_encode_3d(ids, n2, n1, n0)
     for _ in range(2):
         lists = _ops.bin_tiles_3d(m3.to(DEV), r.to(DEV), 8, n2, n1, n0)
+        _compare(lists, tpg, ids, flat, offsets)
+
+
+# 18-bit keys (two passes of 9 bits) and 25-bit keys (three passes of 9, 9 and
+# 7 bits): the 512-digit form of the first, a middle and the last pass.
+@pytest.mark.parametrize("bricks", [(64, 64, 40), (512, 256, 160)])
+def test_nine_bit_passes(bricks):
+    n2, n1, n0 = bricks
+    n = 3000
+    g = torch.Generator().manual_seed(n0)
+    m3 = (torch.rand(n, 3, generator=g) * torch.tensor([8.0 * n2, 8.0 * n1, 8.0 * n0])).float()
+    r = torch.randint(0, 20, (n, 3), generator=g).int()
+    tpg, ids, flat = binning.isect_tiles_3d(m3.numpy(), r.numpy(), 8, n2, n1, n0)
+    offsets = binning.isect_offset_encode_3d(ids, n2, n1, n0)
+    for keep in (True, False):
+        lists = _ops.bin_tiles_3d(m3.to(DEV), r.to(DEV), 8, n2, n1, n0, keep_ids=keep)
         _compare(lists, tpg, ids, flat, offsets)
