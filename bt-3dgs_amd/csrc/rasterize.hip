@@ -517,15 +517,19 @@ __device__ __forceinline__ uint32_t wave_row_mask(const RasterRecord<T> &rec, in
   return readlane_u32(m, 63);
 }
 
-// The whole tile of one record when every tile of the wave lies inside the
-// image (no column guard), kChunk columns at a time.  The column offsets
-// dx_k are the same on every row, so they are kept in registers, and the
-// column sums W_k = sum over rows of w accumulate per column: T0, T1, T2 then
-// follow from W_k once per record, which leaves three accumulations per pixel
-// (W_k, s0, s1) instead of four.  A row outside the record's reach fails the
-// alpha test at every pixel (the reach is conservative) and a dead record's
-// limit is zero, so the upstream gradient is loaded without masks; rows that
-// no lane reaches are skipped.
+// The whole tile of one record, kChunk columns at a time, for a wave whose
+// tiles all have R rows of R columns to read: tiles inside the image, or
+// staged ones (zero beyond it).  The column offsets dx_k are the same on
+// every row, so they are kept in registers, and the column sums
+// W_k = sum over rows of w accumulate per column: T0, T1, T2 then follow from
+// W_k once per record, which leaves three accumulations per pixel (W_k, s0,
+// s1) instead of four.  Every lane walks the rows that any lane of the wave
+// reaches: a row of the image outside a record's own reach fails its alpha
+// test at every pixel (the reach, clamped to the image, is conservative), and
+// a pixel beyond the image, which a footprint crossing the edge may pass,
+// adds w = 0 of its staged zero (sigma is finite there: staged waves with a
+// record that is not positive definite take the masked rows instead).  So the
+// gradient is loaded without masks.
 // kAbsSigned: per row a0 = sum |w|, a1 = sum |w| dx; then PX = |a A1 + b AY|,
 // PY = |b A1 + c AY| with A1 = sum |w| dx and AY = sum |w| dy over the tile.
 // v: the tile's upstream gradient, `stride` values from row to row, every
@@ -612,13 +616,13 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
   return s;
 }
 
-// The sums of one record (one lane) over its tile: the whole-tile form when
-// every tile of the wave lies inside the image, else row by row with masked
-// loads.  Wave-uniform branches only.
+// The sums of one record (one lane) over its tile (nx x ny pixels of it in
+// the image): the whole-tile form when every lane's tile lies inside the
+// image, else row by row with masked loads.  Wave-uniform branches only.
 template <typename T, int R, bool kExact, bool kAbs>
 __device__ __forceinline__ TileSums<T> raster_record_sums(const RasterRecord<T> &rec,
                                                           const T *__restrict__ vimg, uint32_t W,
-                                                          int ox, int oy, int nx, int nts,
+                                                          int ox, int oy, int nx, int ny, int nts,
                                                           bool vec, T dx0) {
   const T half = static_cast<T>(0.5);
   TileSums<T> s = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -626,7 +630,8 @@ __device__ __forceinline__ TileSums<T> raster_record_sums(const RasterRecord<T> 
   // non-finite (uniform over the wave).
   const bool guard = ballot(rec.live && !rec.pd && nx < nts) != 0;
   bool full = false;
-  if constexpr (kExact && R <= 16 && R % kChunk == 0) full = vec && ballot(nx < nts) == 0;
+  if constexpr (kExact && R <= 16 && R % kChunk == 0)
+    full = vec && ballot(nx < nts || ny < nts) == 0;
   if (full && ballot(rec.live) != 0) {
     s = raster_tile_walk<T, R, kAbs ? kAbsTerms : kAbsNone>(
         rec, vimg + static_cast<int64_t>(oy) * W + ox, W, oy, dx0);
@@ -743,7 +748,7 @@ __global__ __launch_bounds__(kBwdThreads) void raster_bwd_kernel(
     load_raster_record(means2d, conics, opac, mus, g, n_items, key_ok, oy, oy + ny - 1, rec);
   const T dx0 = (static_cast<T>(ox) + static_cast<T>(0.5)) - rec.mx;
   const TileSums<T> s =
-      raster_record_sums<T, R, kExact, kAbs>(rec, vimg, W, ox, oy, nx, nts, vec, dx0);
+      raster_record_sums<T, R, kExact, kAbs>(rec, vimg, W, ox, oy, nx, ny, nts, vec, dx0);
   if (!key_ok) return;
   T v[9];
   raster_partials<T, kAbs>(rec, s, v);
@@ -983,6 +988,7 @@ __global__ __launch_bounds__(kSplitThreads) void raster_bwd_split_kernel(
   const uint32_t ty = t / tw, tx = t - ty * tw;
   const int ox = static_cast<int>(tx) * R, oy = static_cast<int>(ty) * R;
   const int nx = min(R, static_cast<int>(W) - ox);
+  const int ny = min(R, static_cast<int>(H) - oy);
   const T *__restrict__ vimg = v_image + static_cast<int64_t>(cam) * H * W;
   const T dx0 = (static_cast<T>(ox) + half) - rec.mx;
   TileSums<T> s;
@@ -994,7 +1000,7 @@ __global__ __launch_bounds__(kSplitThreads) void raster_bwd_split_kernel(
     s = raster_tile_walk<T, R, kAbsSigned>(rec, vimg + static_cast<int64_t>(oy) * W + ox, W, oy,
                                            dx0);
   } else {
-    s = raster_record_sums<T, R, true, true>(rec, vimg, W, ox, oy, nx, R, vec, dx0);
+    s = raster_record_sums<T, R, true, true>(rec, vimg, W, ox, oy, nx, ny, R, vec, dx0);
   }
   if (!valid) return;
   T v[9];

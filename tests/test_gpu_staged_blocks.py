@@ -41,6 +41,37 @@ def test_raster_backward_blocks(dtype, n, shape, views, staged):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("two_pass", [True, False])
+@pytest.mark.parametrize("ts", [8, 16])
+@pytest.mark.parametrize("n,shape,views", [(40, (64, 44), 1), (40, (64, 44), 2),
+                                           (60, (336, 204), 1), (60, (336, 204), 2)])
+def test_raster_backward_ragged_bottom(n, shape, views, ts, two_pass, dtype):
+    """Rows that a 16-byte load fits, no ragged column, a ragged last tile row, and lists too
+    sparse to stage: waves of whole and ragged tiles side by side, with footprints that cross
+    the image's bottom edge."""
+    W_img, H_img = shape
+    d, m2, con, mu, op, ids, fl, off = _raster_case(n, 5, W_img, H_img, ts, views, dtype,
+                                                    log_mu=-2.6 if W_img == 64 else -3.0)
+    tw, th = W_img // ts, -(-H_img // ts)
+    assert W_img % ts == 0 and H_img % ts != 0
+    bottom = ids % (tw * th) // tw == th - 1
+    assert any(b.any() and not b.all() for b in bottom.split(64))
+    assert int(ids[:256].max() - ids[:256].min()) >= 4
+    if not two_pass:
+        fl = fl.clone()
+    assert (_ops.emission_order(fl, off.numel()) is not None) == two_pass
+    v = torch.randn((views, H_img, W_img), generator=d["gen"], dtype=dtype)
+    for absgrad in (True, False):
+        refs = raster_references(np32(m2), np32(con), np32(op), np32(mu), np32(off), np32(fl),
+                                 W_img, H_img, ts, v_image=v.numpy(), absgrad=absgrad)
+        got = W.rasterize_to_pixels_bwd_per_gaussian(m2, con, op, mu, off, ids, fl, v.to(DEV),
+                                                     W_img, H_img, ts, absgrad)
+        for name, r in check_raster(refs, grads=[None if t is None else np32(t)
+                                                 for t in got]).items():
+            print(absgrad, name, r)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("n,dims,log_mu,staged", [
     (2500, (30, 20, 26), -3.2, True),   # ragged
     (2500, (29, 21, 9), -1.6, True),    # ragged, waves that walk every row
