@@ -858,9 +858,10 @@ __device__ __forceinline__ uint64_t shfl_bits(uint64_t v, int src) {
   return static_cast<uint64_t>(__shfl(static_cast<long long>(v), src, 64));
 }
 
-// Chunks of one chunked wave: its records reach at most kDenseItems rows, in
-// chunks of up to kChunkRows, at most one short chunk per record.
-constexpr int kMaxChunks = kDenseItems / kChunkRows + 64;
+// Chunks of one wave: 64 records of at most 64 rows, in chunks of up to
+// kChunkRows.  A wave over kDenseItems takes the dense walk only where its
+// bricks can be read whole, so no smaller bound holds.
+constexpr int kMaxChunks = 64 * (64 / kChunkRows);
 
 // kGiven: each record's reach mask comes from `reach` (stored by the forward
 // over the same lists, voxel_fwd_reach_kernel) instead of the culling

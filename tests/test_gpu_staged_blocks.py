@@ -5,6 +5,7 @@ footprints: against the oracle at the usual bar (tests/helpers.py)."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -96,6 +97,35 @@ def test_voxel_backward_blocks(dtype, n, dims, log_mu, staged):
         print(name, r)
     n2, n1, n0 = (-(-x // 8) for x in dims)
     lists = _ops.TileLists(None, ids, fl, *_ops.emission_order(fl, n2 * n1 * n0), off)
+    given = _ops.voxel_backward(m3, con, op, off, lists, v.to(DEV), *dims, 8, reach=reach)
+    for a, b in zip(plain, given):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("dims", [(90, 61, 77), (92, 61, 77), (96, 61, 80)])
+def test_voxel_backward_full_chunk_lists(dims, dtype):
+    """A few Gaussians that cover the whole volume: blocks over too many bricks to stage, whose
+    records reach every row, in bricks that cannot be read whole (ragged, or rows that no
+    16-byte load fits): the longest chunk lists."""
+    d, m3, con, ids, fl, off = _voxel_case(5, 8, dims, 8, dtype, log_mu=-0.7)
+    assert min(int(b.max() - b.min()) + 1 for b in ids.split(256)[:-1]) > 6
+    op = d["opac"]
+    _, reach = _ops.voxelize_with_reach(m3, con, op, off, fl, *dims)
+    rows = np.array([bin(int(x)).count("1") for x in reach.cpu().numpy().view(np.uint64)])
+    chunks = np.add.reduceat(-(-rows // 8), np.arange(0, rows.size, 64))
+    n2, n1, _ = (-(-x // 8) for x in dims)
+    at = np.stack([np32(ids) % n2, np32(ids) // n2 % n1, np32(ids) // (n2 * n1)], 1)
+    ragged = ((at + 1) * 8 > np.array(dims)).any(1) | (dims[0] % 4 != 0)
+    split = np.add.reduceat(ragged, np.arange(0, rows.size, 64)) > 0
+    assert chunks[split].max() > 448, chunks
+    v = torch.randn((dims[2], dims[1], dims[0]), generator=d["gen"], dtype=dtype)
+    refs = voxel_references(np32(m3), np32(con), np32(op), np32(off), np32(fl), *dims, 8,
+                            v_volume=v.numpy())
+    plain = W.voxelize_to_voxels_bwd_per_gaussian(m3, con, op, off, ids, fl, v.to(DEV), *dims, 8)
+    for name, r in check_voxel(refs, grads=[np32(t) for t in plain]).items():
+        print(name, r)
+    lists = _ops.TileLists(None, ids, fl, *_ops.emission_order(fl, off.numel()), off)
     given = _ops.voxel_backward(m3, con, op, off, lists, v.to(DEV), *dims, 8, reach=reach)
     for a, b in zip(plain, given):
         assert torch.equal(a, b)
