@@ -130,8 +130,9 @@ __device__ __forceinline__ double limit_as_value(uint64_t b) {
 }
 
 // Keys of the records of a wave: `rb` is the wave's first record (uniform),
-// `r` the lane's; the key of record r is the last k with offsets[k] <= r
-// (offsets[0] = 0, non-decreasing).  One uniform search for rb, then a
+// `r` the lane's; the key of record r is the last k with offsets[k] <= r, or
+// 0 where there is none (offsets non-decreasing; any others give some key
+// below n_keys).  One uniform search for rb, then a
 // uniform walk over the next few keys' first indices; a window holding more
 // boundaries than that (empty keys share their successor's first index, so
 // a run of them is many boundaries at one index) finishes with a per-lane
@@ -148,7 +149,8 @@ __device__ __forceinline__ uint32_t wave_record_key(const int32_t *__restrict__ 
     const uint32_t step = (hi - lo + 63) / 64;
     const uint32_t at = lo + lane_id() * step;
     const bool below = at < hi && static_cast<int64_t>(offsets[at]) <= rb;
-    lo += (static_cast<uint32_t>(__popcll(ballot(below))) - 1) * step;  // lane 0 is below
+    // No lane is below where a caller's offsets start after rb: key 0 then.
+    lo += static_cast<uint32_t>(max(static_cast<int>(__popcll(ballot(below))), 1) - 1) * step;
     hi = min(lo + step, hi);
   }
   const int64_t r_last = min(rb + 63, n_isects - 1);

@@ -131,6 +131,33 @@ def test_voxel_backward_full_chunk_lists(dims, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("first", [1, 100, 700])
+def test_offsets_that_start_after_the_first_record(first):
+    """Records before a caller's first tile (brick) offset have no key to be found: they count
+    to key 0, as when the keys are given."""
+    d, m2, con, mu, op, ids, fl, off = _raster_case(4000, 9, 160, 144, 16)
+    assert off.numel() > 64 and fl.numel() > 1000
+    off, ids = off.clamp(min=first), torch.where(torch.arange(ids.numel(), device=DEV) < first, 0,
+                                                 ids)
+    v = torch.randn((1, 144, 160), generator=d["gen"]).to(DEV)
+    for absgrad in (True, False):
+        got = W.rasterize_to_pixels_bwd(m2, con, op, mu, off, fl, v, 160, 144, 16, absgrad)
+        want = W.rasterize_to_pixels_bwd_per_gaussian(m2, con, op, mu, off, ids, fl, v, 160, 144,
+                                                      16, absgrad)
+        for a, b in zip(got[not absgrad:], want[not absgrad:]):
+            assert torch.equal(a, b)
+    dims = (40, 36, 32)
+    d, m3, con, ids, fl, off = _voxel_case(3000, 10, dims, 8)
+    assert off.numel() > 64 and fl.numel() > 1000
+    off, ids = off.clamp(min=first), torch.where(torch.arange(ids.numel(), device=DEV) < first, 0,
+                                                 ids)
+    v = torch.randn(dims[::-1], generator=d["gen"]).to(DEV)
+    got = W.voxelize_to_voxels_bwd(m3, con, d["opac"], off, fl, v, *dims, 8)
+    want = W.voxelize_to_voxels_bwd_per_gaussian(m3, con, d["opac"], off, ids, fl, v, *dims, 8)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dims", [(30, 20, 26), (32, 24, 32)])
 def test_non_finite_record_in_a_ragged_brick(dims):
     """A record with a non-finite conic passes the alpha test wherever its sigma is NaN or
