@@ -54,7 +54,7 @@ struct Vec<double> {
 
 struct Brick {
   int oi, oj, ok;  // origin (dim0, dim1, dim2)
-  int ni, nj, nk;  // extent inside the volume
+  int ni, nj, nk;  // extent inside the volume (0 in bricks of a larger grid)
 };
 
 __device__ __forceinline__ Brick brick_of(uint32_t key, uint32_t n2, uint32_t n1, uint32_t ts,
@@ -65,9 +65,10 @@ __device__ __forceinline__ Brick brick_of(uint32_t key, uint32_t n2, uint32_t n1
   b.oi = static_cast<int>(b0 * ts);
   b.oj = static_cast<int>(b1 * ts);
   b.ok = static_cast<int>(b2 * ts);
-  b.ni = static_cast<int>(min(ts, D0 - b0 * ts));
-  b.nj = static_cast<int>(min(ts, D1 - b1 * ts));
-  b.nk = static_cast<int>(min(ts, D2 - b2 * ts));
+  // The grid may be larger than the volume: no wrap below zero.
+  b.ni = static_cast<int>(min(ts, D0 - min(D0, b0 * ts)));
+  b.nj = static_cast<int>(min(ts, D1 - min(D1, b1 * ts)));
+  b.nk = static_cast<int>(min(ts, D2 - min(D2, b2 * ts)));
   return b;
 }
 

@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import check_raster, check_voxel, np32, raster_references, voxel_references
+from helpers import (assert_close, check_raster, check_voxel, np32, raster_references,
+                     voxel_references)
 from r2splat.cuda import _ops
 from r2splat.cuda import _wrapper as W
 from test_gpu_ops import DEV, _raster_case, _voxel_case
@@ -156,6 +157,31 @@ def test_offsets_that_start_after_the_first_record(first):
     want = W.voxelize_to_voxels_bwd_per_gaussian(m3, con, d["opac"], off, ids, fl, v, *dims, 8)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("ts", [4, 8, 10])
+def test_brick_grid_larger_than_the_volume(ts):
+    """Bricks of a caller's grid that lie beyond the volume hold no voxel: the volume and the
+    gradients are those of the exact grid."""
+    dims = (30, 20, 26)
+    n2, n1, n0 = (-(-x // ts) for x in dims)
+    d, m3, con, _, _, _ = _voxel_case(1500, 12, dims, ts)
+    v = torch.randn(dims[::-1], generator=d["gen"]).to(DEV)
+    # Radii that take in every brick.
+    r3 = torch.full((m3.shape[0], 3), 200, dtype=torch.int32, device=DEV)
+    outs = []
+    for e2, e1, e0 in ((0, 0, 0), (2, 1, 2)):
+        grid = (n2 + e2, n1 + e1, n0 + e0)
+        _, ids, fl = W.isect_tiles_3d(m3, r3, ts, *grid)
+        off = W.isect_offset_encode_3d(ids, *grid)
+        assert off[-1, -1, -1] < fl.numel()
+        outs.append([W.voxelize_to_voxels_fwd(m3, con, d["opac"], off, fl, *dims, ts),
+                     *W.voxelize_to_voxels_bwd_per_gaussian(m3, con, d["opac"], off, ids, fl, v,
+                                                            *dims, ts)])
+    want, got = outs
+    # Sums of the same terms: in other waves and orders, 1e-5 of the largest is their rounding.
+    for name, a, b in zip(("volume", "v_means3d", "v_conics", "v_opacities"), got, want):
+        assert_close(np32(a), np32(b), name, rtol=1e-5, atol=1e-5 * float(b.abs().max()))
 
 
 @pytest.mark.parametrize("dims", [(30, 20, 26), (32, 24, 32)])
