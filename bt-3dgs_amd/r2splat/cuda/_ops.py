@@ -1806,6 +1806,8 @@ def trainer_loss_fwd(render: Tensor, target: Tensor, edge_target: Optional[Tenso
     _check(w.numel() == 5, "weights must hold five values")
     dev = r.device
     _check(h.device == dev, "hierarchy must be on the render's device")
+    _check(w.device == dev, "weights must be on the render's device")
+    _check(v is None or v.device == dev, "volume must be on the render's device")
     n, H, W = r.shape
     terms = torch.empty(5, dtype=torch.float32, device=dev)
     total = torch.empty((), dtype=torch.float32, device=dev)
@@ -1831,6 +1833,9 @@ def trainer_loss_bwd(render: Tensor, target: Tensor, edge_target: Optional[Tenso
     _check(w.numel() == 5 and g.numel() == 1, "weights must hold five values, grad_total one")
     n, H, W = r.shape
     dev = r.device
+    _check(w.device == dev and g.device == dev,
+           "weights and grad_total must be on the render's device")
+    _check(v is None or v.device == dev, "volume must be on the render's device")
     v_r = torch.empty_like(r) if want_render else None
     v_v = torch.empty_like(v) if want_volume and v is not None else None
     with _on(dev):

@@ -71,3 +71,25 @@ def test_no_cpu_fallback():
     with pytest.raises(ValueError, match="backward_mode"):
         explicit.prepare_explicit_gaussians(q, s, o, scale_min=5e-4, scale_max=1.0,
                                             backward_mode="x")
+
+
+@pytest.mark.parametrize("other", ["volume", "weights", "hierarchy", "grad_total"])
+def test_trainer_loss_refuses_inputs_of_another_gpu(other):
+    """Tensors without memory stand in for two GPUs: the kernels must not be handed a pointer
+    of another one."""
+    from torch._subclasses import FakeTensorMode
+
+    from r2splat.cuda import _ops
+
+    with FakeTensorMode():
+        at = lambda name: f"cuda:{int(name == other)}"  # noqa: E731
+        r, t = (torch.empty(1, 8, 8, device="cuda:0") for _ in range(2))
+        vol, w = torch.empty(4, 4, 4, device=at("volume")), torch.empty(5, device=at("weights"))
+        if other != "grad_total":
+            h = torch.empty((), device=at("hierarchy"))
+            with pytest.raises(RuntimeError, match="must be on the render's device"):
+                _ops.trainer_loss_fwd(r, t, None, None, vol, h, w)
+        if other != "hierarchy":
+            g, ws = torch.empty((), device=at("grad_total")), torch.empty(16, device="cuda:0")
+            with pytest.raises(RuntimeError, match="must be on the render's device"):
+                _ops.trainer_loss_bwd(r, t, None, None, vol, w, g, ws)
