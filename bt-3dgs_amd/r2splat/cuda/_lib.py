@@ -159,12 +159,16 @@ DENSIFY_MAX_WIDTH = 16
 
 SYMBOLS = sorted(list(_PLAIN) + [f"r2s_{n}_{s}" for n in _FLOAT_OPS for s in ("f32", "f64")])
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """dlopen the library and attach the C signatures of every exported symbol."""
     lib = ctypes.CDLL(path)
+    # Before the entries: a library of another revision may lack some.
+    lib.r2s_abi_version.restype, lib.r2s_abi_version.argtypes = _PLAIN["r2s_abi_version"]
+    if lib.r2s_abi_version() != ABI_VERSION:
+        raise RuntimeError(f"{path}: ABI version {lib.r2s_abi_version()} != {ABI_VERSION}")
     for name, (res, args) in _PLAIN.items():
         fn = getattr(lib, name)
         fn.restype, fn.argtypes = res, args
@@ -172,6 +176,4 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         for suffix in ("f32", "f64"):
             fn = getattr(lib, f"r2s_{name}_{suffix}")
             fn.restype, fn.argtypes = _i32, args
-    if lib.r2s_abi_version() != ABI_VERSION:
-        raise RuntimeError(f"{path}: ABI version {lib.r2s_abi_version()} != {ABI_VERSION}")
     return lib

@@ -4,6 +4,7 @@ and rejects invalid arguments before touching any device."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -31,6 +32,15 @@ def test_exports_every_declared_symbol(lib):
         assert hasattr(lib, name), f"{name} missing from {_lib.LIB_PATH}"
     assert sorted(_lib.SYMBOLS) == declared, "ctypes table and header disagree"
     assert lib.r2s_abi_version() == _lib.ABI_VERSION
+
+
+def test_library_of_an_earlier_revision_is_named(tmp_path):
+    """A library built before the newest entries: the version is reported, not a symbol."""
+    src, so = tmp_path / "old.c", str(tmp_path / "old.so")
+    src.write_text("int r2s_abi_version(void) { return 10; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(src)], check=True)
+    with pytest.raises(RuntimeError, match="ABI version 10 != "):
+        _lib.load(so)
 
 
 def test_invalid_arguments_are_rejected_without_a_device(lib):
