@@ -101,6 +101,18 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, uint32_t src) {
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// A value that every lane holds alike, in scalar registers (the asm statement
+// emits no code; a value known to be uniform would stay in vector ones).
+template <typename T>
+__device__ __forceinline__ T uniform_value(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit values");
+  asm volatile("" : "+v"(v));
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(T, readlane_u32(__builtin_bit_cast(uint32_t, v), 0));
+  else
+    return __builtin_bit_cast(T, readlane_i64(__builtin_bit_cast(int64_t, v), 0));
+}
+
 // One DPP lane move of a 32- or 64-bit value (the halves moved
 // separately): lanes the move does not write (no source lane in the row, or
 // a row outside kRowMask) read `fill`.

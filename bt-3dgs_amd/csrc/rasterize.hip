@@ -132,10 +132,11 @@ __global__ __launch_bounds__(1024) void raster_fwd_kernel(
 // staged per record (alpha_limit), so a pixel costs an add, two FMAs, one
 // v_exp_f32, the compare (which masks) and the accumulating FMA.  Vector
 // issue bounds it: the exps run in groups of eight at raised priority
-// (neg_exp2_run), and the columns' offsets dx_0 + k are formed in the loop,
-// which keeps the kernel at 53 VGPRs and 25 KB of LDS (eight waves per SIMD)
-// where a staged table of them took 64 and 37: 0.208 -> 0.203 ms for 4.7 M
-// records on 512^2, 89 -> 85 us for 1.7 M records of nine 333 x 217 views.
+// (neg_exp2_run), and the columns' offsets from the mean are formed in the
+// loop from pixel centres in scalar registers, which keeps the kernel at 52
+// VGPRs and 25 KB of LDS (eight waves per SIMD) where a staged table of them
+// took 64 and 37: 0.210 -> 0.203 ms for 4.7 M records on 512^2, 86 -> 82 us
+// for 1.7 M records of nine 333 x 217 views.
 // At the end each wave adds its groups' partial tiles across lanes and the
 // block adds its waves' in order: a fixed order, so the result is
 // deterministic (the per-pixel order differs from a plain list-order sum
@@ -208,9 +209,15 @@ __global__ __launch_bounds__(kFwdBatch) void raster_fwd_rows_kernel(
   const int64_t t1 = (key == n_keys - 1) ? n_isects : static_cast<int64_t>(tile_offsets[key + 1]);
   const int64_t start = t0 + (t1 - t0) * split / splits;
   const int64_t end = t0 + (t1 - t0) * (split + 1) / splits;
-  T acc[R];
+  // The pixel centres of the lane's columns, exact.  A lane that covers a whole
+  // tile row has the tile's, kept in scalar registers.
+  T acc[R], pxk[R];
 #pragma unroll
-  for (int q = 0; q < R; ++q) acc[q] = 0;
+  for (int q = 0; q < R; ++q) {
+    acc[q] = 0;
+    const T centre = px0 + static_cast<T>(q);
+    pxk[q] = LPR == 1 ? uniform_value(centre) : centre;
+  }
   const int wave_first = wave * G;  // uniform: the record loop below is a scalar loop
   const int group = lane / NL;
   if (tid < G) {
@@ -274,10 +281,10 @@ __global__ __launch_bounds__(kFwdBatch) void raster_fwd_rows_kernel(
       const V4 p = s_rec[jb + group].p;
       const V4 q = s_rec[jb + group].q;
       const typename Bits<T>::type lim = bits_of(q.z);
-      const T dx0 = px0 - p.x, dy = py - p.y;
+      const T dy = py - p.y;
       const T B = p.w * dy, C = q.x * dy * dy;
-      // sigma from the pixel's offset from the mean, as the reference forms
-      // it: a quadratic in the column offset instead would cancel badly where
+      // dx as the reference forms it (pixel centre minus mean, one rounding):
+      // a quadratic in the column offset instead would cancel badly where
       // sigma is small but the offset's terms are large (sub-pixel
       // footprints far along the row).
 #pragma unroll
@@ -285,7 +292,7 @@ __global__ __launch_bounds__(kFwdBatch) void raster_fwd_rows_kernel(
         T sl[kRun], e[kRun];
 #pragma unroll
         for (int k = 0; k < kRun; ++k) {
-          const T dx = dx0 + static_cast<T>(h + k);
+          const T dx = pxk[h + k] - p.x;
           sl[k] = fma(fma(p.z, dx, B), dx, C);
         }
         neg_exp2_run(sl, e);

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
       const V4 h0 = s_rec[3 * t + 1];
       const V4 h1 = s_rec[3 * t + 2];
       const typename Bits<T>::type lim = bits_of(h1.z);
-      const T dx0 = px0 - mo.x, dy = py - mo.y, dz = pz - mo.z;
+      const T dy = py - mo.y, dz = pz - mo.z;
       const T B = h0.y * dy + h0.z * dz;
       const T C = (h0.w * dy + h1.x * dz) * dy + h1.y * dz * dz;
       constexpr int kRun = R < 8 ? R : 8;  // voxels per run of exps
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
         T sl[kRun], e[kRun];
 #pragma unroll
         for (int k = 0; k < kRun; ++k) {
-          const T dx = dx0 + static_cast<T>(r + k);
+          const T dx = (px0 + static_cast<T>(r + k)) - mo.x;
           sl[k] = fma(fma(h0.x, dx, B), dx, C);
         }
         neg_exp2_run(sl, e);

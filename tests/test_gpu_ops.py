@@ -1181,3 +1181,32 @@ def _raster_radii(m2, d):
     Ks[:, 1, 2] = 32
     return W.project_gaussians_fwd(d["means"], d["covars"], d["opac"], d["viewmats"], Ks, 64, 64,
                                    1e-8, 3.0)[2]
+
+
+@pytest.mark.parametrize("ts", [8, 16, 32])
+def test_rasterize_fwd_pixel_offset_is_rounded_once(ts):
+    """dx is the pixel centre minus the mean with one rounding.  Means near a tile's left edge
+    for which the offset of the row's first pixel plus the column rounds differently there,
+    each beside another mean of the same dx: the same pixel value, bit for bit."""
+    f = np.float32
+    x = np.random.default_rng(0).uniform(-0.25, 0.25, 200_000).astype(f)
+    k = 15 if ts > 8 else 7
+    once, twice = f(k + 0.5) - x, (f(0.5) - x) + f(k)
+    same = {d: v for d, v in zip(once[once == twice], x[once == twice])}
+    pairs = [(a, same[d]) for a, d in zip(x[once != twice], once[once != twice]) if d in same][:64]
+    assert len(pairs) >= 16
+    n = len(pairs)
+    # One Gaussian a view; sigma of about 10 at the pixel, where a rounding of dx shows most.
+    m2 = torch.tensor(np.array(pairs)).reshape(2 * n, 1)
+    m2 = torch.stack([m2, torch.full_like(m2, 4.5)], -1).to(DEV)
+    con = torch.tensor([20.0 / (k + 0.5) ** 2, 0.0, 0.1]).expand(2 * n, 1, 3).contiguous().to(DEV)
+    one = torch.ones(2 * n, 1, device=DEV)
+    r = torch.full((2 * n, 1, 2), 64, dtype=torch.int32, device=DEV)
+    _, ids, fl = W.isect_tiles(m2, r, ts, 1, 1)
+    off = W.isect_offset_encode(ids, 2 * n, 1, 1)
+    img = W.rasterize_to_pixels_fwd(m2, con, one, one, off, fl, ts, ts, ts)
+    payload, _ = _ops.raster_pack(m2, con, one, one)
+    for image in (img, _ops.rasterize_packed(payload, off, fl, 2 * n, 1, ts, ts, ts)):
+        at = image[:, 4, k].reshape(n, 2)
+        assert float(at.min()) > 1e-5
+        assert torch.equal(at[:, 0], at[:, 1])
