@@ -530,7 +530,10 @@ __device__ __forceinline__ uint32_t wave_row_mask(const RasterRecord<T> &rec, in
 // every row, so they are kept in registers, and the column sums
 // W_k = sum over rows of w accumulate per column: T0, T1, T2 then follow from
 // W_k once per record, which leaves three accumulations per pixel (W_k, s0,
-// s1) instead of four.  Every lane walks the rows that any lane of the wave
+// s1) instead of four.  Each chunk's sums over the rows are kept apart and
+// added at the end: in one chain over both halves of a row the rounding error
+// of the absolute sums was 1.06-1.08 times that of full rows, of the conic's
+// 1.02-1.03, and apart it is 0.98 times each.  Every lane walks the rows that any lane of the wave
 // reaches: a row of the image outside a record's own reach fails its alpha
 // test at every pixel (the reach, clamped to the image, is conservative), and
 // a pixel beyond the image, which a footprint crossing the edge may pass,
@@ -559,6 +562,7 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
       dxk[k] = dx0 + static_cast<T>(h + k);
       wk[k] = 0;
     }
+    T y0 = 0, yy = 0, y1 = 0, ax = 0, ay = 0;  // of these columns
 #pragma unroll 1
     for (uint32_t m = rows; m != 0; m &= m - 1) {
       const int ly = __builtin_ctz(m);
@@ -597,15 +601,15 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
         }
       }
       const T t = dy * s0;
-      s.Y0 += t;
-      s.YY = fma(dy, t, s.YY);
-      s.Y1 = fma(dy, s1, s.Y1);
+      y0 += t;
+      yy = fma(dy, t, yy);
+      y1 = fma(dy, s1, y1);
       if (kAbs == kAbsTerms) {
-        s.PX += px;
-        s.PY += py;
+        ax += px;
+        ay += py;
       } else if (kAbs == kAbsSigned) {
-        AY = fma(dy, px, AY);
-        A1 += py;
+        ay = fma(dy, px, ay);
+        ax += py;
       }
     }
 #pragma unroll
@@ -614,6 +618,16 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
       s.T0 += wk[k];
       s.T1 += wx;
       s.T2 += wx * dxk[k];
+    }
+    s.Y0 += y0;
+    s.YY += yy;
+    s.Y1 += y1;
+    if (kAbs == kAbsTerms) {
+      s.PX += ax;
+      s.PY += ay;
+    } else if (kAbs == kAbsSigned) {
+      A1 += ax;
+      AY += ay;
     }
   }
   if (kAbs == kAbsSigned) {
@@ -876,7 +890,9 @@ constexpr uint32_t kStageStride = 16 * 16 + 16;
 
 // The two-pass (rows) backward with absolute gradients at tile size 16.
 // Vector issue bounds it (1.5 vector instructions in flight per SIMD).  Half
-// a tile row at a time (raster_tile_walk) it takes 75 VGPRs instead of 89,
+// a tile row at a time (raster_tile_walk) it takes 80 VGPRs instead of 89 (the
+// bound on waves keeps it there: at 81, five waves per SIMD, it took 0.432 ms
+// where it takes 0.411 for 4.3 M records on 512^2),
 // and with the gradients staged it reads LDS, where 64 lanes times 16 bytes
 // per load kept the vector cache's return path busy for 86 % of the kernel's
 // time: 0.357 -> 0.345 ms for 4.7 M records on 512^2, 0.876 -> 0.818 ms for
@@ -884,7 +900,7 @@ constexpr uint32_t kStageStride = 16 * 16 + 16;
 // take the same walk: a 333 x 217 projection of 200k Gaussians, forward and
 // backward, went from 269 to 238 us.
 template <typename T>
-__global__ __launch_bounds__(kSplitThreads) void raster_bwd_split_kernel(
+__global__ __launch_bounds__(kSplitThreads, sizeof(T) == 4 ? 6 : 1) void raster_bwd_split_kernel(
     const T *__restrict__ payload, const int32_t *__restrict__ tile_offsets,
     const int64_t *__restrict__ isect_ids, const int32_t *__restrict__ flatten_ids,
     const int32_t *__restrict__ isect_src, int64_t n_isects, uint32_t n_keys, int64_t n_items,
