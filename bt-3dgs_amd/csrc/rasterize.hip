@@ -533,21 +533,25 @@ __device__ __forceinline__ uint32_t wave_row_mask(const RasterRecord<T> &rec, in
 // s1) instead of four.  Each chunk's sums over the rows are kept apart and
 // added at the end: in one chain over both halves of a row the rounding error
 // of the absolute sums was 1.06-1.08 times that of full rows, of the conic's
-// 1.02-1.03, and apart it is 0.98 times each.  Every lane walks the rows that any lane of the wave
-// reaches: a row of the image outside a record's own reach fails its alpha
-// test at every pixel (the reach, clamped to the image, is conservative), and
-// a pixel beyond the image, which a footprint crossing the edge may pass,
-// adds w = 0 of its staged zero (sigma is finite there: staged waves with a
-// record that is not positive definite take the masked rows instead).  So the
-// gradient is loaded without masks.
+// 1.02-1.03, and apart it is 0.98 times each.
+// Every lane walks the rows that any lane of the wave reaches: a row of the
+// image outside a record's own reach fails its alpha test at every pixel (the
+// reach, clamped to the image, is conservative), and a pixel beyond the
+// image, which a footprint crossing the edge may pass, adds w = 0 of its
+// staged zero (sigma is finite there: staged waves with a record that is not
+// positive definite take the masked rows instead).  So the gradient is loaded
+// without masks.
+// kRagged: of the `ragged` lanes' tiles only the first ny >= 1 rows are in the
+// image; for the others they read the first and test against a zero limit.
 // kAbsSigned: per row a0 = sum |w|, a1 = sum |w| dx; then PX = |a A1 + b AY|,
 // PY = |b A1 + c AY| with A1 = sum |w| dx and AY = sum |w| dy over the tile.
 // v: the tile's upstream gradient, `stride` values from row to row, every
 // row's chunks 16-byte aligned.
-template <typename T, int R, AbsForm kAbs>
+template <typename T, int R, AbsForm kAbs, bool kRagged = false>
 __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &rec,
                                                         const T *__restrict__ v, uint32_t stride,
-                                                        int oy, T dx0) {
+                                                        int oy, T dx0, bool ragged = false,
+                                                        int ny = R) {
   using Q = typename Quad<T>::type;
   constexpr int kq = Quad<T>::n;
   TileSums<T> s = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -566,7 +570,9 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
 #pragma unroll 1
     for (uint32_t m = rows; m != 0; m &= m - 1) {
       const int ly = __builtin_ctz(m);
-      const T *__restrict__ vrow = v + (static_cast<size_t>(ly) * stride + h);
+      const bool row_ok = !kRagged || !ragged || ly < ny;
+      const T *__restrict__ vrow = (row_ok ? v + static_cast<size_t>(ly) * stride : v) + h;
+      const typename Bits<T>::type lim = row_ok ? rec.lim : 0;
       T vv[kChunk];
 #pragma unroll
       for (int q = 0; q < kChunk / kq; ++q)
@@ -588,7 +594,7 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
         // The product is formed unconditionally: as an operand of the
         // conditional it would become a branch around its load and exp.
         const T p = vv[k] * e[k];
-        const T w = alpha_pass(sl[k], rec.lim) ? p : static_cast<T>(0);
+        const T w = alpha_pass(sl[k], lim) ? p : static_cast<T>(0);
         wk[k] += w;
         s0 += w;
         s1 = fma(w, dx, s1);
@@ -637,10 +643,86 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
   return s;
 }
 
+// The whole tile of one record by full rows, read from memory, for tiles with
+// a row in the image at least.  As raster_tile_walk, but each lane tests the
+// rows outside its own reach (and so those beyond the image) against a zero
+// limit and reads its tile's first row there.  It takes 90 to 95 registers
+// where the half rows take 73 to 80 and is the better form where the atomics
+// after it bound the kernel: the one-pass backward took 68 us for 45k records
+// of 512^2 over half rows and 60 us over full ones (27k: 65 and 56), the same
+// from 260k on.  The two-pass form without absolute gradients takes 15.2 us
+// for 86k records by full rows and 14.0 by half rows, 308 and 304 for 4.3 M.
+template <typename T, int R, bool kAbs>
+__device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &rec,
+                                                        const T *__restrict__ vimg, uint32_t W,
+                                                        int ox, int oy, T dx0) {
+  using Q = typename Quad<T>::type;
+  constexpr int kq = Quad<T>::n;
+  TileSums<T> s = {0, 0, 0, 0, 0, 0, 0, 0};
+  T dxk[R], wk[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    dxk[k] = dx0 + static_cast<T>(k);
+    wk[k] = 0;
+  }
+  const T half = static_cast<T>(0.5);
+#pragma unroll 1
+  for (int ly = 0; ly < R; ++ly) {
+    const int i = oy + ly;
+    const bool in_row = rec.live && i >= rec.i0 && i <= rec.i1;
+    if (ballot(in_row) == 0) continue;
+    const T dy = (static_cast<T>(i) + half) - rec.my;
+    const T B = rec.hb * dy, C = rec.hc * dy * dy;
+    const T bdy = rec.b * dy, cdy = rec.c * dy;
+    const typename Bits<T>::type lim = in_row ? rec.lim : 0;
+    const T *__restrict__ vrow = vimg + static_cast<int64_t>(in_row ? i : oy) * W + ox;
+    T s0 = 0, s1 = 0, px = 0, py = 0;
+#pragma unroll
+    for (int h = 0; h < R; h += kChunk) {
+      T vv[kChunk];
+#pragma unroll
+      for (int q = 0; q < kChunk / kq; ++q)
+        *reinterpret_cast<Q *>(vv + q * kq) = *reinterpret_cast<const Q *>(vrow + h + q * kq);
+#pragma unroll
+      for (int kk = 0; kk < kChunk; ++kk) {
+        const T dx = dxk[h + kk];
+        const T sl = fma(fma(rec.ha, dx, B), dx, C);
+        const T p = vv[kk] * neg_exp2(sl);  // unconditional, as in raster_tile_walk
+        const T w = alpha_pass(sl, lim) ? p : static_cast<T>(0);
+        wk[h + kk] += w;
+        s0 += w;
+        s1 = fma(w, dx, s1);
+        if (kAbs) {
+          px = fma(fabs(w), fabs(fma(rec.a, dx, bdy)), px);
+          py = fma(fabs(w), fabs(fma(rec.b, dx, cdy)), py);
+        }
+      }
+    }
+    s.Y0 += dy * s0;
+    s.YY += dy * (dy * s0);
+    s.Y1 += dy * s1;
+    if (kAbs) {
+      s.PX += px;
+      s.PY += py;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const T wx = wk[k] * dxk[k];
+    s.T0 += wk[k];
+    s.T1 += wx;
+    s.T2 += wx * dxk[k];
+  }
+  return s;
+}
+
 // The sums of one record (one lane) over its tile (nx x ny pixels of it in
-// the image): the whole-tile form when every lane's tile lies inside the
-// image, else row by row with masked loads.  Wave-uniform branches only.
-template <typename T, int R, bool kExact, bool kAbs>
+// the image): a whole-tile form when every lane's tile has all its columns in
+// the image, else row by row with masked loads.  Wave-uniform branches only.
+// Waves with ragged bottom tiles take a whole-tile form too: by masked rows
+// they were the last to end beside whole ones (a two-pass backward of 27k
+// records of 512 x 500: 35 us, 29 so).
+template <typename T, int R, bool kExact, bool kAbs, bool kHalves>
 __device__ __forceinline__ TileSums<T> raster_record_sums(const RasterRecord<T> &rec,
                                                           const T *__restrict__ vimg, uint32_t W,
                                                           int ox, int oy, int nx, int ny, int nts,
@@ -652,10 +734,18 @@ __device__ __forceinline__ TileSums<T> raster_record_sums(const RasterRecord<T> 
   const bool guard = ballot(rec.live && !rec.pd && nx < nts) != 0;
   bool full = false;
   if constexpr (kExact && R <= 16 && R % kChunk == 0)
-    full = vec && ballot(nx < nts || ny < nts) == 0;
+    full = vec && ballot(nx < nts || ny < 1) == 0;
   if (full && ballot(rec.live) != 0) {
-    s = raster_tile_walk<T, R, kAbs ? kAbsTerms : kAbsNone>(
-        rec, vimg + static_cast<int64_t>(oy) * W + ox, W, oy, dx0);
+    const T *__restrict__ v = vimg + static_cast<int64_t>(oy) * W + ox;
+    constexpr AbsForm kForm = kAbs ? kAbsTerms : kAbsNone;
+    if constexpr (!kHalves)
+      s = raster_tile_full<T, R, kAbs>(rec, vimg, W, ox, oy, dx0);
+    else if (const uint64_t ragged = ballot(ny < nts); ragged == 0)
+      s = raster_tile_walk<T, R, kForm>(rec, v, W, oy, dx0);
+    else
+      s = raster_tile_walk<T, R, kForm, true>(
+          rec, v, W, oy, dx0, ny < nts,
+          static_cast<int>(readlane_u32(static_cast<uint32_t>(ny), __builtin_ctzll(ragged))));
   } else if (ballot(rec.live) != 0) {
     for (int ly = 0; ly < R; ++ly) {
       if (!kExact && ly >= nts) break;
@@ -769,7 +859,7 @@ __global__ __launch_bounds__(kBwdThreads) void raster_bwd_kernel(
     load_raster_record(means2d, conics, opac, mus, g, n_items, key_ok, oy, oy + ny - 1, rec);
   const T dx0 = (static_cast<T>(ox) + static_cast<T>(0.5)) - rec.mx;
   const TileSums<T> s =
-      raster_record_sums<T, R, kExact, kAbs>(rec, vimg, W, ox, oy, nx, ny, nts, vec, dx0);
+      raster_record_sums<T, R, kExact, kAbs, kRows>(rec, vimg, W, ox, oy, nx, ny, nts, vec, dx0);
   if (!key_ok) return;
   T v[9];
   raster_partials<T, kAbs>(rec, s, v);
@@ -890,9 +980,7 @@ constexpr uint32_t kStageStride = 16 * 16 + 16;
 
 // The two-pass (rows) backward with absolute gradients at tile size 16.
 // Vector issue bounds it (1.5 vector instructions in flight per SIMD).  Half
-// a tile row at a time (raster_tile_walk) it takes 80 VGPRs instead of 89 (the
-// bound on waves keeps it there: at 81, five waves per SIMD, it took 0.432 ms
-// where it takes 0.411 for 4.3 M records on 512^2),
+// a tile row at a time (raster_tile_walk) it takes 75 VGPRs instead of 89,
 // and with the gradients staged it reads LDS, where 64 lanes times 16 bytes
 // per load kept the vector cache's return path busy for 86 % of the kernel's
 // time: 0.357 -> 0.345 ms for 4.7 M records on 512^2, 0.876 -> 0.818 ms for
@@ -1001,9 +1089,7 @@ __global__ __launch_bounds__(kSplitThreads, sizeof(T) == 4 ? 6 : 1) void raster_
   s_key[slot] = in_list ? key : key0;
   s_rec.store(static_cast<int>(slot), split_record(rec));
   __syncthreads();
-  const int32_t rr = s_r[threadIdx.x];
-  const bool valid = rr >= 0;
-  if (ballot(valid) == 0) return;  // uniform per wave; no barrier follows
+  if (ballot(s_r[threadIdx.x] >= 0) == 0) return;  // uniform per wave; no barrier follows
   key = s_key[threadIdx.x];
   rec = raster_record(s_rec.load(static_cast<int>(threadIdx.x)));
   const bool wave_fast = (wave + 1) * 64 <= n_fast;
@@ -1023,9 +1109,11 @@ __global__ __launch_bounds__(kSplitThreads, sizeof(T) == 4 ? 6 : 1) void raster_
     s = raster_tile_walk<T, R, kAbsSigned>(rec, vimg + static_cast<int64_t>(oy) * W + ox, W, oy,
                                            dx0);
   } else {
-    s = raster_record_sums<T, R, true, true>(rec, vimg, W, ox, oy, nx, ny, R, vec, dx0);
+    s = raster_record_sums<T, R, true, true, true>(rec, vimg, W, ox, oy, nx, ny, R, vec, dx0);
   }
-  if (!valid) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // s_r read again, not kept in a register
+  const int32_t rr = s_r[threadIdx.x];
+  if (rr < 0) return;
   T v[9];
   raster_partials<T, true>(rec, s, v);
   const T r8[8] = {v[0], v[1], v[2], v[3], v[4], s.T0, v[7], v[8]};
