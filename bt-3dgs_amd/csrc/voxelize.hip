@@ -753,13 +753,24 @@ __global__ __launch_bounds__(kBwdThreads) void voxel_bwd_kernel(
 }
 
 // The row of a record's ten partials: the per-voxel terms of
-// VoxelizeToVoxelsBwd.cu:409-421 summed over the brick.
+// VoxelizeToVoxelsBwd.cu:409-421 summed over the brick.  The record's opacity
+// and conic are loaded again, so that they need not stay in registers; `used`:
+// the record has sums (a skipped one's row is zero whatever its conic holds).
 template <typename T>
 __device__ __forceinline__ void store_partials(T *__restrict__ rows, int64_t e,
-                                               const BwdRecord<T> &rec, T T0, T T1, T T2, T Y0,
-                                               T Z0, T Y1, T Z1, T YY, T YZ, T ZZ) {
-  const T half = static_cast<T>(0.5), o = rec.o;
-  const T *q = rec.q;
+                                               const T *__restrict__ conics,
+                                               const T *__restrict__ opac, int64_t g, bool used,
+                                               T T0, T T1, T T2, T Y0, T Z0, T Y1, T Z1, T YY,
+                                               T YZ, T ZZ) {
+  T q[6], o = 0;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) q[c] = 0;
+  if (used) {
+    o = opac[g];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) q[c] = conics[6 * g + c];
+  }
+  const T half = static_cast<T>(0.5);
   const T v[10] = {o * (q[0] * T1 + q[1] * Y0 + q[2] * Z0),
                    o * (q[3] * Y0 + q[4] * Z0 + q[1] * T1),
                    o * (q[5] * Z0 + q[4] * Y0 + q[2] * T1),
@@ -868,7 +879,7 @@ constexpr int kMaxChunks = 64 * (64 / kChunkRows);
 // over the same lists, voxel_fwd_reach_kernel) instead of the culling
 // setup and the per-slice row ranges.
 template <typename T, bool kGiven>
-__global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
+__global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxel_bwd_chunk_kernel(
     const T *__restrict__ means3d, const T *__restrict__ conics, const T *__restrict__ opac,
     const int32_t *__restrict__ tile_offsets, const int64_t *__restrict__ isect_ids,
     const int32_t *__restrict__ flatten_ids, const int32_t *__restrict__ isect_src,
@@ -886,9 +897,9 @@ __global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
   __shared__ uint32_t s_key_min[kChunkWaves], s_key_max[kChunkWaves];
   __shared__ __align__(16) T s_v[kStageBricks * kBrick];
   const uint32_t w = wave_index(), lane = lane_id();
-  const int64_t rb = static_cast<int64_t>(xcd_swizzle(blockIdx.x, gridDim.x)) *
-                         (64 * kChunkWaves) + 64 * static_cast<int64_t>(w);
-  const int64_t r = rb + lane;
+  // Positions in the list fit 32 bits: n_isects < 2^31 (the caller checks).
+  const uint32_t rb = xcd_swizzle(blockIdx.x, gridDim.x) * (64 * kChunkWaves) + 64 * w;
+  const uint32_t r = rb + lane;
   const bool in_list = r < n_isects;
   uint32_t key;
   bool key_ok = in_list;
@@ -951,9 +962,24 @@ __global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
   // beyond the volume, it is summed apart, voxel by voxel.
   const bool apart = rec.live && rec.lim == Bits<T>::kSign &&
                      (b.ni < R || b.nj < R || b.nk < R);
+  const bool used = rec.live;
   if (apart) rec.live = false;
   const T half = static_cast<T>(0.5);
   const T dx0 = (static_cast<T>(b.ok) + half) - rec.m[0];
+
+  // The row of the lane's record from its sums over the walked rows.
+  const auto finish = [&](T T0, T T1, T T2, T Y0, T Z0, T Y1, T Z1, T YY, T YZ, T ZZ) {
+    if (!key_ok) return;
+    uint32_t at = r, of = key;
+    asm volatile("" : "+v"(at), "+v"(of));  // what they give is formed here, not kept till here
+    const int64_t gauss = flatten_ids[at];
+    if (apart)
+      voxel_sums_apart(means3d, conics, opac, gauss, N,
+                       brick_of(of + koff, n2, n1, R, D2, D1, D0), v_vol, plane, D2, T0, T1, T2,
+                       Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+    store_partials(rows, isect_src[at], conics, opac, gauss, used, T0, T1, T2, Y0, Z0, Y1, Z1, YY,
+                   YZ, ZZ);
+  };
 
   // The record's reached rows; the items are its set bits in increasing order.
   uint64_t reached;
@@ -977,11 +1003,7 @@ __global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
                                      plane, D2, dx0, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ,
                                      reached);
     }
-    if (apart)
-      voxel_sums_apart(means3d, conics, opac, g, N, b, v_vol, plane, D2, T0, T1, T2, Y0, Z0, Y1,
-                       Z1, YY, YZ, ZZ);
-    if (key_ok)
-      store_partials(rows, isect_src[r], rec, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+    finish(T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
     return;
   }
   // The brick's first voxel centre minus the mean.
@@ -1047,146 +1069,154 @@ __global__ __launch_bounds__(64 * kChunkWaves, 5) void voxel_bwd_chunk_kernel(
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
+  // The two forms apart: the registers of one are not held through the other.
+  const auto walk = [&](auto staged_tag) {
+    constexpr bool kStaged = decltype(staged_tag)::value;
 #pragma unroll 1
-  for (uint32_t cb = 0; cb < n_list; cb += 64) {
-    const uint32_t ci = cb + lane;
-    const bool act = ci < n_list;
-    const uint32_t ent = act ? static_cast<uint32_t>(s_chunk[w][ci]) : 0u;
-    const uint32_t rl = ent & 63u, pos = (ent >> 6) & 63u, q = ent >> 12;
-    // The record, from the registers of the lane that loaded it (every lane
-    // takes part); the conic scaled as scaled_conic does.
-    const int src = static_cast<int>(rl);
-    T qr[6], hr[6];
+    for (uint32_t cb = 0; cb < n_list; cb += 64) {
+      const uint32_t ci = cb + lane;
+      const bool act = ci < n_list;
+      const uint32_t ent = act ? static_cast<uint32_t>(s_chunk[w][ci]) : 0u;
+      const uint32_t rl = ent & 63u, pos = (ent >> 6) & 63u, q = ent >> 12;
+      // The record, from the registers of the lane that loaded it (every lane
+      // takes part); the conic scaled as scaled_conic does.
+      const int src = static_cast<int>(rl);
+      T qr[6], hr[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) qr[c] = __shfl(rec.q[c], src, 64);
-    scaled_conic(qr, hr);
-    const T cx = __shfl(dx0, src, 64), cy = __shfl(c1, src, 64), cz = __shfl(c2, src, 64);
-    const typename Bits<T>::type r_lim = shfl_bits(my_lim, src);
-    const uint32_t r_key = static_cast<uint32_t>(__shfl(static_cast<int>(key), src, 64));
-    const uint64_t rows_m = s_rows[w][rl];
-    const int n_here =
-        act ? min(R, __popcll(rows_m) - static_cast<int>(q) * R) : 0;
-    // The record's rows from the chunk's first on: the chunk's items are
-    // its n_here lowest set bits.
-    uint64_t rest = act ? rows_m & (~0ull << pos) : 0ull;
-    T dxk[R], wk[R];
+      for (int c = 0; c < 6; ++c) qr[c] = __shfl(rec.q[c], src, 64);
+      scaled_conic(qr, hr);
+      const T cx = __shfl(dx0, src, 64), cy = __shfl(c1, src, 64), cz = __shfl(c2, src, 64);
+      const typename Bits<T>::type r_lim = shfl_bits(my_lim, src);
+      const uint32_t r_key = static_cast<uint32_t>(__shfl(static_cast<int>(key), src, 64));
+      const uint64_t rows_m = s_rows[w][rl];
+      const int n_here =
+          act ? min(R, __popcll(rows_m) - static_cast<int>(q) * R) : 0;
+      // The record's rows from the chunk's first on: the chunk's items are
+      // its n_here lowest set bits.
+      uint64_t rest = act ? rows_m & (~0ull << pos) : 0ull;
+      T dxk[R], wk[R];
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-      dxk[k] = cx + static_cast<T>(k);
-      wk[k] = 0;
-    }
-    // The brick's gradient: staged, or in the volume.
-    Brick bb = {};
-    const T *__restrict__ vb = v_vol;
-    if (!staged) {
-      bb = brick_of(r_key + koff, n2, n1, R, D2, D1, D0);
-      vb += bb.oi * plane + static_cast<int64_t>(bb.oj) * D2 + bb.ok;
-    }
-    const uint32_t sv = staged ? (r_key - key0) * kBrick : 0u;
-    T Y0 = 0, Z0 = 0, Y1 = 0, Z1 = 0, YY = 0, YZ = 0, ZZ = 0;
-    // The round's longest chunk is its first (lane 0 is always active).
-    const int steps = __builtin_amdgcn_readfirstlane(n_here);
-#pragma unroll 1
-    for (int st = 0; st < steps; ++st) {
-      const bool item = st < n_here;
-      // The next row (bit 63 when none is left: a step without an item
-      // still reads a row of the record's own brick and tests against a zero
-      // limit).
-      const uint32_t p = static_cast<uint32_t>(__builtin_ctzll(rest | (1ull << 63)));
-      rest &= rest - 1ull;
-      const uint32_t li = p >> 3, lj = p & 7u;
-      // The row centre's offsets from the mean as the columns' (dxk): the
-      // brick corner's offset plus the row's index in the brick.
-      const T dz = static_cast<T>(li) + cz;
-      const T dy = static_cast<T>(lj) + cy;
-      const T B = fma(hr[1], dy, hr[2] * dz);
-      const T C = fma(fma(hr[3], dy, hr[4] * dz), dy, hr[5] * dz * dz);
-      typename Bits<T>::type lim = item ? r_lim : 0;
-      asm volatile("" : "+v"(lim));  // one select, not a scalar AND per voxel
-      T vv[R];
-      if (staged) {
-        const T *vrow = s_v + (sv + p * R);
-#pragma unroll
-        for (int c = 0; c < R / kq; ++c)
-          *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
+      for (int k = 0; k < R; ++k) {
+        dxk[k] = cx + static_cast<T>(k);
+        wk[k] = 0;
+      }
+      // The brick's gradient: staged, or in the volume.
+      const T *__restrict__ vb = v_vol;
+      uint32_t sv = 0;
+      int nk = R;
+      if constexpr (kStaged) {
+        sv = (r_key - key0) * kBrick;
       } else {
-        const T *__restrict__ vrow = vb + (li * plane + static_cast<int64_t>(lj) * D2);
-        if (whole) {
+        const Brick bb = brick_of(r_key + koff, n2, n1, R, D2, D1, D0);
+        vb += bb.oi * plane + static_cast<int64_t>(bb.oj) * D2 + bb.ok;
+        nk = bb.nk;
+      }
+      T Y0 = 0, Z0 = 0, Y1 = 0, Z1 = 0, YY = 0, YZ = 0, ZZ = 0;
+      // The round's longest chunk is its first (lane 0 is always active).
+      const int steps = __builtin_amdgcn_readfirstlane(n_here);
+#pragma unroll 1
+      for (int st = 0; st < steps; ++st) {
+        const bool item = st < n_here;
+        // The next row (bit 63 when none is left: a step without an item
+        // still reads a row of the record's own brick and tests against a zero
+        // limit).
+        const uint32_t p = static_cast<uint32_t>(__builtin_ctzll(rest | (1ull << 63)));
+        rest &= rest - 1ull;
+        const uint32_t li = p >> 3, lj = p & 7u;
+        // The row centre's offsets from the mean as the columns' (dxk): the
+        // brick corner's offset plus the row's index in the brick.
+        const T dz = static_cast<T>(li) + cz;
+        const T dy = static_cast<T>(lj) + cy;
+        const T B = fma(hr[1], dy, hr[2] * dz);
+        const T C = fma(fma(hr[3], dy, hr[4] * dz), dy, hr[5] * dz * dz);
+        typename Bits<T>::type lim = item ? r_lim : 0;
+        asm volatile("" : "+v"(lim));  // one select, not a scalar AND per voxel
+        T vv[R];
+        if constexpr (kStaged) {
+          const T *vrow = s_v + (sv + p * R);
 #pragma unroll
           for (int c = 0; c < R / kq; ++c)
             *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
         } else {
-          // Columns beyond the volume read zero; the rows and slices beyond
-          // it are reached by no record, only by a step without an item.
-          const int n = static_cast<int>(li) < bb.ni && static_cast<int>(lj) < bb.nj ? bb.nk : 0;
+          const T *__restrict__ vrow = vb + (li * plane + static_cast<int64_t>(lj) * D2);
+          if (whole) {
 #pragma unroll
-          for (int k = 0; k < R; ++k) vv[k] = k < n ? vrow[k] : static_cast<T>(0);
+            for (int c = 0; c < R / kq; ++c)
+              *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
+          } else {
+            // Columns beyond the volume read zero; the rows and slices beyond
+            // it are reached by no record, only by a step without an item.
+            const int n = item ? nk : 0;
+#pragma unroll
+            for (int k = 0; k < R; ++k) vv[k] = k < n ? vrow[k] : static_cast<T>(0);
+          }
         }
-      }
-      T s0 = 0, s1 = 0;
-      T sl[R], e[R];
+        T s0 = 0, s1 = 0;
 #pragma unroll
-      for (int k = 0; k < R; ++k) sl[k] = fma(fma(hr[0], dxk[k], B), dxk[k], C);
-      neg_exp2_run(sl, e);
+        for (int h = 0; h < R; h += R / 2) {  // in halves: eight registers fewer
+          T sl[R / 2], e[R / 2];
+#pragma unroll
+          for (int k = 0; k < R / 2; ++k)
+            sl[k] = fma(fma(hr[0], dxk[h + k], B), dxk[h + k], C);
+          neg_exp2_run(sl, e);
+#pragma unroll
+          for (int k = 0; k < R / 2; ++k) {
+            // A failing voxel adds an exact zero whatever its upstream gradient
+            // (a non-finite one included), as when the voxel is skipped.  The
+            // product is formed unconditionally: as an operand of the
+            // conditional it would become a branch around its load and exp.
+            const T p = vv[h + k] * e[k];
+            const T wv = alpha_pass(sl[k], lim) ? p : static_cast<T>(0);
+            wk[h + k] += wv;
+            s0 += wv;
+            s1 = fma(wv, dxk[h + k], s1);
+          }
+        }
+        const T dys0 = dy * s0, dzs0 = dz * s0;
+        Y0 += dys0;
+        Z0 += dzs0;
+        YY = fma(dy, dys0, YY);
+        YZ = fma(dz, dys0, YZ);
+        ZZ = fma(dz, dzs0, ZZ);
+        Y1 = fma(dy, s1, Y1);
+        Z1 = fma(dz, s1, Z1);
+      }
+      T t0 = 0, t1 = 0, t2 = 0;
 #pragma unroll
       for (int k = 0; k < R; ++k) {
-        const T dx = dxk[k];
-        // A failing voxel adds an exact zero whatever its upstream gradient
-        // (a non-finite one included), as when the voxel is skipped.  The
-        // product is formed unconditionally: as an operand of the
-        // conditional it would become a branch around its load and exp.
-        const T p = vv[k] * e[k];
-        const T wv = alpha_pass(sl[k], lim) ? p : static_cast<T>(0);
-        wk[k] += wv;
-        s0 += wv;
-        s1 = fma(wv, dx, s1);
+        const T wx = wk[k] * dxk[k];
+        t0 += wk[k];
+        t1 += wx;
+        t2 += wx * dxk[k];
       }
-      const T dys0 = dy * s0, dzs0 = dz * s0;
-      Y0 += dys0;
-      Z0 += dzs0;
-      YY = fma(dy, dys0, YY);
-      YZ = fma(dz, dys0, YZ);
-      ZZ = fma(dz, dzs0, ZZ);
-      Y1 = fma(dy, s1, Y1);
-      Z1 = fma(dz, s1, Z1);
-    }
-    T t0 = 0, t1 = 0, t2 = 0;
+      const T sums[10] = {t0, t1, t2, Y0, Z0, Y1, Z1, YY, YZ, ZZ};
+      // One chunk index at a time, in increasing order: the records of one
+      // index are distinct, and each record's chunks are added in index order.
+      uint32_t qmask = 0;
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-      const T wx = wk[k] * dxk[k];
-      t0 += wk[k];
-      t1 += wx;
-      t2 += wx * dxk[k];
-    }
-    const T sums[10] = {t0, t1, t2, Y0, Z0, Y1, Z1, YY, YZ, ZZ};
-    // One chunk index at a time, in increasing order: the records of one
-    // index are distinct, and each record's chunks are added in index order.
-    uint32_t qmask = 0;
-#pragma unroll
-    for (int b = 0; b < R; ++b)
-      if (ballot(act && q == static_cast<uint32_t>(b)) != 0) qmask |= 1u << b;
+      for (int b = 0; b < R; ++b)
+        if (ballot(act && q == static_cast<uint32_t>(b)) != 0) qmask |= 1u << b;
 #pragma unroll 1
-    for (uint32_t mq = qmask; mq != 0u; mq &= mq - 1u) {
-      const uint32_t qq = static_cast<uint32_t>(__builtin_ctz(mq));
-      if (act && q == qq) {
+      for (uint32_t mq = qmask; mq != 0u; mq &= mq - 1u) {
+        const uint32_t qq = static_cast<uint32_t>(__builtin_ctz(mq));
+        if (act && q == qq) {
 #pragma unroll
-        for (int c = 0; c < 10; ++c) s_acc[w][c][rl] += sums[c];
+          for (int c = 0; c < 10; ++c) s_acc[w][c][rl] += sums[c];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-  }
-  if (!key_ok) return;
+  };
+  if (staged)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
   T a[10];
 #pragma unroll
   for (int c = 0; c < 10; ++c) a[c] = s_acc[w][c][lane];
-  if (apart)
-    voxel_sums_apart(means3d, conics, opac, static_cast<int64_t>(flatten_ids[r]), N,
-                     brick_of(key + koff, n2, n1, R, D2, D1, D0), v_vol, plane, D2, a[0], a[1],
-                     a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9]);
-  store_partials(rows, isect_src[r], rec, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8],
-                 a[9]);
+  finish(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9]);
 }
 
 // n0 brick layers of lists from layer z0 on (the whole grid: z0 = 0 and
