@@ -525,10 +525,11 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
 // gradient is loaded without masks.
 // kReach: the slices' row ranges come from `reach` (bit 8 * slice + row of
 // the reached rows, as voxel_bwd_chunk_kernel computes them) instead of
-// slice_rows.
+// slice_rows.  kRuns: a row's exps as one run (neg_exp2_run), where many
+// waves share a SIMD.
 // v: the gradient at the brick's first voxel, with the given slice and row
 // strides; every row 16-byte aligned.
-template <typename T, int R, bool kReach = false>
+template <typename T, int R, bool kReach = false, bool kRuns = false>
 __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const Brick &b,
                                                  const T *__restrict__ v, int64_t plane,
                                                  uint32_t D2, T dx0, T &T0, T &T1, T &T2, T &Y0,
@@ -578,8 +579,11 @@ __device__ __forceinline__ void voxel_brick_full(const BwdRecord<T> &rec, const 
       // hoisted into extra registers.
       T sl[R], e[R];
 #pragma unroll
-      for (int k = 0; k < R; ++k) sl[k] = fma(fma(rec.h[0], dxk[k], B), dxk[k], C);
-      neg_exp2_run(sl, e);
+      for (int k = 0; k < R; ++k) {
+        sl[k] = fma(fma(rec.h[0], dxk[k], B), dxk[k], C);
+        if (!kRuns) e[k] = neg_exp2(sl[k]);
+      }
+      if constexpr (kRuns) neg_exp2_run(sl, e);
 #pragma unroll
       for (int k = 0; k < R; ++k) {
         const T dx = dxk[k];
@@ -753,23 +757,11 @@ __global__ __launch_bounds__(kBwdThreads) void voxel_bwd_kernel(
 }
 
 // The row of a record's ten partials: the per-voxel terms of
-// VoxelizeToVoxelsBwd.cu:409-421 summed over the brick.  The record's opacity
-// and conic are loaded again, so that they need not stay in registers; `used`:
-// the record has sums (a skipped one's row is zero whatever its conic holds).
+// VoxelizeToVoxelsBwd.cu:409-421 summed over the brick.
 template <typename T>
-__device__ __forceinline__ void store_partials(T *__restrict__ rows, int64_t e,
-                                               const T *__restrict__ conics,
-                                               const T *__restrict__ opac, int64_t g, bool used,
-                                               T T0, T T1, T T2, T Y0, T Z0, T Y1, T Z1, T YY,
-                                               T YZ, T ZZ) {
-  T q[6], o = 0;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) q[c] = 0;
-  if (used) {
-    o = opac[g];
-#pragma unroll
-    for (int c = 0; c < 6; ++c) q[c] = conics[6 * g + c];
-  }
+__device__ __forceinline__ void store_partials(T *__restrict__ rows, int64_t e, T o,
+                                               const T (&q)[6], T T0, T T1, T T2, T Y0, T Z0,
+                                               T Y1, T Z1, T YY, T YZ, T ZZ) {
   const T half = static_cast<T>(0.5);
   const T v[10] = {o * (q[0] * T1 + q[1] * Y0 + q[2] * Z0),
                    o * (q[3] * Y0 + q[4] * Z0 + q[1] * T1),
@@ -841,18 +833,22 @@ __device__ __forceinline__ void voxel_sums_apart(const T *__restrict__ means3d,
 //
 // The lanes of a step read the gradient rows of different records: loaded
 // from memory, 64 lanes times 32 bytes through the vector cache's return path
-// each step, that path was busy 92-98 % of the kernel's time.  A block
-// therefore stages its bricks' gradients in LDS when its records lie in at
-// most kStageBricks consecutive bricks, zero beyond the volume, so that
-// ragged volumes walk like any other.  Blocks over more bricks (short lists)
-// read rows from memory, element by element at the volume's ragged ends.
-// Six bricks and the other arrays take 28 KB, which with 96 VGPRs keeps five
-// waves per SIMD: 0.399 -> 0.381 ms for 3.2 M records of a 256^3 volume, 5.49
-// -> 5.30 ms for 39 M of a 512^3 one; a 250 x 201 x 173 volume of 100k
-// Gaussians, which took the masked walk of voxel_bwd_kernel before, went from
-// 449 to 374 us forward and backward.  The records' fields reach the lanes
-// that walk them by lane shuffles from the registers of the lanes that loaded
-// them; staged in LDS (39 KB, four waves) the rows pass took 0.397 ms.
+// each step, that path was busy 92-98 % of the kernel's time.  Staged
+// (kStage), a block therefore keeps its bricks' gradients in LDS when its
+// records lie in at most kStageBricks consecutive bricks, zero beyond the
+// volume, so that ragged volumes walk like any other; a block over more
+// bricks reads rows from memory, element by element at the volume's ragged
+// ends.  Six bricks and the other arrays take 28 KB, which with 96 VGPRs and
+// no scratch keeps five waves per SIMD: 0.484 -> 0.469 ms for 3.2 M records
+// of a 256^3 volume (0.426 -> 0.388 given masks), 22.9 -> 21.9 ms for 252 M
+// of a 512^3 one (21.3 -> 19.1), 0.231 -> 0.149 ms for 1.0 M of a
+// 250 x 201 x 173 one beside the masked walk.  The records' fields reach the
+// lanes that walk them by lane shuffles from the registers of the lanes that
+// loaded them; staged in LDS (39 KB, four waves) the rows pass took longer.
+// Unstaged, for short lists of whole volumes (stage_bricks), the records'
+// fields go through LDS and every row comes from memory: 80 VGPRs, 27 KB, six
+// waves per SIMD, no barrier.  Its exps stay with their voxels: where few
+// waves run, runs of them (neg_exp2_run) only delay the sums after them.
 
 constexpr int kChunkRows = 8;
 constexpr int kChunkWaves = 4;
@@ -870,16 +866,52 @@ __device__ __forceinline__ uint64_t shfl_bits(uint64_t v, int src) {
   return static_cast<uint64_t>(__shfl(static_cast<long long>(v), src, 64));
 }
 
-// Chunks of one wave: 64 records of at most 64 rows, in chunks of up to
-// kChunkRows.  A wave over kDenseItems takes the dense walk only where its
-// bricks can be read whole, so no smaller bound holds.
-constexpr int kMaxChunks = 64 * (64 / kChunkRows);
+// Chunks of one wave of 64 records of at most 64 rows, in chunks of up to
+// kChunkRows.  Where every brick can be read whole, a wave over kDenseItems
+// takes the dense walk, and below it has at most one short chunk per record
+// beside the full ones (27 KB of LDS, six blocks per CU); staged blocks are
+// not the only ones of the staged form, so no smaller bound holds there.
+template <bool kStage>
+constexpr int kMaxChunks = kStage ? 64 * (64 / kChunkRows) : kDenseItems / kChunkRows + 64;
+
+// Whether a list's backward stages its bricks' gradients (kStage).  Blocks
+// whose records lie in too many bricks for it read memory through the general
+// code of the staged form, which is slower than the unstaged kernels, so the
+// line lies where most blocks stage.
+// Ragged volumes, whose other form is voxel_bwd_kernel's masked walk: from
+// 256 records per kStageBricks bricks on, the least that fills a block.  At
+// 37 records per brick of 250 x 201 x 173 the staged form takes 173 us and
+// the masked walk 168, at 54 147 and 230; of 90 x 61 x 77 at 41 36 and 36, at
+// 104 22 and 42.
+// Whole volumes, whose other form is the unstaged chunked walk: from 64
+// records per brick on.  Of 256 x 200 x 176 at 25 records 99 and 81 us, at 56
+// 140 and 130 (given masks 128 and 120), of 256^3 at 97 470 and 461 (given
+// masks 385 and 420), of 512^3 at 960 22.0 and 22.4 ms (19.2 and 21.0).
+// Lists of less than a block per CU wait for the staging's two barriers alone:
+// 9k records of a 32^3 volume, 29 and 26 us.  In double the staged form has
+// two waves per SIMD instead of three: 1.22 and 1.17 ms at 256^3 without
+// masks.
+template <typename T>
+inline bool stage_bricks(int64_t n_isects, int64_t n_keys, bool whole) {
+  if (!whole) return n_isects * kStageBricks >= 64 * kChunkWaves * n_keys;
+  return sizeof(T) == 4 && n_isects >= 64 * n_keys && n_isects >= 64 * kChunkWaves * 256;
+}
+
+// A record as the lanes that walk it read it from LDS (unstaged form).
+template <typename T>
+struct ChunkRecord {
+  T c[3];  // the brick's first voxel centre minus the mean (x, y, z)
+  T h[6];
+  typename Bits<T>::type lim;  // 0 for dead records
+  uint32_t brick0;             // byte offset of the brick's first voxel in v_vol
+};
 
 // kGiven: each record's reach mask comes from `reach` (stored by the forward
 // over the same lists, voxel_fwd_reach_kernel) instead of the culling
 // setup and the per-slice row ranges.
-template <typename T, bool kGiven>
-__global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxel_bwd_chunk_kernel(
+template <typename T, bool kGiven, bool kStage>
+__global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? (kStage ? 5 : 6) : 1)
+void voxel_bwd_chunk_kernel(
     const T *__restrict__ means3d, const T *__restrict__ conics, const T *__restrict__ opac,
     const int32_t *__restrict__ tile_offsets, const int64_t *__restrict__ isect_ids,
     const int32_t *__restrict__ flatten_ids, const int32_t *__restrict__ isect_src,
@@ -888,14 +920,16 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
     T *__restrict__ rows, const uint64_t *__restrict__ reach) {
   constexpr int R = kChunkRows;
   constexpr uint32_t kBrick = R * R * R;
+  constexpr int kRun = kStage ? R / 2 : 1;  // voxels per run of exps
   using Q = typename Quad<T>::type;
   constexpr int kq = Quad<T>::n;
   __shared__ uint64_t s_rows[kChunkWaves][64];  // reached rows: bit 8 * slice + row
   __shared__ T s_acc[kChunkWaves][10][64];
   // Chunk entries: record lane | first row << 6 | chunk index << 12.
-  __shared__ uint16_t s_chunk[kChunkWaves][kMaxChunks];
+  __shared__ uint16_t s_chunk[kChunkWaves][kMaxChunks<kStage>];
   __shared__ uint32_t s_key_min[kChunkWaves], s_key_max[kChunkWaves];
-  __shared__ __align__(16) T s_v[kStageBricks * kBrick];
+  __shared__ WordMajor<ChunkRecord<T>, 64> s_rec[kStage ? 1 : kChunkWaves];
+  __shared__ __align__(16) T s_v[kStage ? kStageBricks * kBrick : 1];
   const uint32_t w = wave_index(), lane = lane_id();
   // Positions in the list fit 32 bits: n_isects < 2^31 (the caller checks).
   const uint32_t rb = xcd_swizzle(blockIdx.x, gridDim.x) * (64 * kChunkWaves) + 64 * w;
@@ -908,6 +942,7 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
   const int32_t fid = in_list ? flatten_ids[r] : -1;
   const uint64_t reach_r = kGiven && in_list ? reach[r] : 0ull;
   if (rb >= n_isects) {  // uniform per wave: no records, only its share of the staging
+    if constexpr (!kStage) return;
     key_ok = false;
     key = 0;
   } else if (isect_ids != nullptr) {
@@ -917,38 +952,43 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
   } else {
     key = wave_record_key(tile_offsets, n_keys, n_isects, rb, r);
   }
-  const uint32_t k_min = wave_min(key_ok ? key : 0xffffffffu);
-  const uint32_t k_max = wave_max(key_ok ? key : 0u);
-  if (lane == 0) {
-    s_key_min[w] = k_min;
-    s_key_max[w] = k_max;
-  }
-  __syncthreads();
-  uint32_t key0 = s_key_min[0], key1 = s_key_max[0];
-#pragma unroll
-  for (uint32_t ww = 1; ww < kChunkWaves; ++ww) {
-    key0 = min(key0, s_key_min[ww]);
-    key1 = max(key1, s_key_max[ww]);
-  }
-  if (key0 > key1) return;  // uniform over the block: no record in range
   const int64_t plane = static_cast<int64_t>(D1) * D2;
-  const bool staged = key1 - key0 < kStageBricks;
-  if (staged) {
-    for (uint32_t k = key0; k <= key1; ++k) {
-      const Brick sb = brick_of(k + koff, n2, n1, R, D2, D1, D0);
-      const T *__restrict__ src = v_vol + sb.oi * plane + static_cast<int64_t>(sb.oj) * D2 + sb.ok;
-#pragma unroll
-      for (uint32_t h = 0; h < kBrick; h += 64 * kChunkWaves) {
-        const int q = static_cast<int>(h + threadIdx.x);
-        const int i = q >> 6, j = (q >> 3) & 7, c = q & 7;
-        s_v[(k - key0) * kBrick + static_cast<uint32_t>(q)] =
-            (i < sb.ni && j < sb.nj && c < sb.nk) ? src[i * plane + static_cast<int64_t>(j) * D2 + c]
-                                                  : static_cast<T>(0);
-      }
+  bool staged = false;
+  uint32_t key0 = 0;
+  if constexpr (kStage) {
+    const uint32_t k_min = wave_min(key_ok ? key : 0xffffffffu);
+    const uint32_t k_max = wave_max(key_ok ? key : 0u);
+    if (lane == 0) {
+      s_key_min[w] = k_min;
+      s_key_max[w] = k_max;
     }
     __syncthreads();
+    key0 = s_key_min[0];
+    uint32_t key1 = s_key_max[0];
+#pragma unroll
+    for (uint32_t ww = 1; ww < kChunkWaves; ++ww) {
+      key0 = min(key0, s_key_min[ww]);
+      key1 = max(key1, s_key_max[ww]);
+    }
+    if (key0 > key1) return;  // uniform over the block: no record in range
+    staged = key1 - key0 < kStageBricks;
+    if (staged) {
+      for (uint32_t k = key0; k <= key1; ++k) {
+        const Brick sb = brick_of(k + koff, n2, n1, R, D2, D1, D0);
+        const T *__restrict__ src = v_vol + sb.oi * plane + static_cast<int64_t>(sb.oj) * D2 + sb.ok;
+#pragma unroll
+        for (uint32_t h = 0; h < kBrick; h += 64 * kChunkWaves) {
+          const int q = static_cast<int>(h + threadIdx.x);
+          const int i = q >> 6, j = (q >> 3) & 7, c = q & 7;
+          s_v[(k - key0) * kBrick + static_cast<uint32_t>(q)] =
+              (i < sb.ni && j < sb.nj && c < sb.nk) ? src[i * plane + static_cast<int64_t>(j) * D2 + c]
+                                                    : static_cast<T>(0);
+        }
+      }
+      __syncthreads();
+    }
+    if (rb >= n_isects) return;  // uniform per wave; no barrier follows
   }
-  if (rb >= n_isects) return;  // uniform per wave; no barrier follows
   if (!key_ok) key = key0;
   const int64_t g = key_ok ? static_cast<int64_t>(fid) : -1;
   const Brick b = brick_of(key + koff, n2, n1, R, D2, D1, D0);
@@ -960,25 +1000,37 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
   // A record whose sigma may be NaN passes the alpha test there whatever the
   // gradient: in a ragged brick, where the walk below also evaluates columns
   // beyond the volume, it is summed apart, voxel by voxel.
-  const bool apart = rec.live && rec.lim == Bits<T>::kSign &&
+  const bool apart = kStage && rec.live && rec.lim == Bits<T>::kSign &&
                      (b.ni < R || b.nj < R || b.nk < R);
   const bool used = rec.live;
   if (apart) rec.live = false;
   const T half = static_cast<T>(0.5);
   const T dx0 = (static_cast<T>(b.ok) + half) - rec.m[0];
 
-  // The row of the lane's record from its sums over the walked rows.
+  // The row of the lane's record from its sums over the walked rows.  Staged,
+  // the record's opacity and conic and every address are loaded or formed
+  // again rather than kept in registers through the walk; a record without
+  // sums has a zero row whatever its conic holds.
   const auto finish = [&](T T0, T T1, T T2, T Y0, T Z0, T Y1, T Z1, T YY, T YZ, T ZZ) {
     if (!key_ok) return;
-    uint32_t at = r, of = key;
-    asm volatile("" : "+v"(at), "+v"(of));  // what they give is formed here, not kept till here
-    const int64_t gauss = flatten_ids[at];
-    if (apart)
-      voxel_sums_apart(means3d, conics, opac, gauss, N,
-                       brick_of(of + koff, n2, n1, R, D2, D1, D0), v_vol, plane, D2, T0, T1, T2,
-                       Y0, Z0, Y1, Z1, YY, YZ, ZZ);
-    store_partials(rows, isect_src[at], conics, opac, gauss, used, T0, T1, T2, Y0, Z0, Y1, Z1, YY,
-                   YZ, ZZ);
+    if constexpr (kStage) {
+      uint32_t at = r, of = key;
+      asm volatile("" : "+v"(at), "+v"(of));  // what they give is formed here
+      const int64_t gauss = flatten_ids[at];
+      if (apart)
+        voxel_sums_apart(means3d, conics, opac, gauss, N,
+                         brick_of(of + koff, n2, n1, R, D2, D1, D0), v_vol, plane, D2, T0, T1, T2,
+                         Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+      T o = 0, q[6] = {0, 0, 0, 0, 0, 0};
+      if (used) {
+        o = opac[gauss];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) q[c] = conics[6 * gauss + c];
+      }
+      store_partials(rows, isect_src[at], o, q, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+    } else {
+      store_partials(rows, isect_src[r], rec.o, rec.q, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
+    }
   };
 
   // The record's reached rows; the items are its set bits in increasing order.
@@ -990,18 +1042,17 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
   const int n_items = __popcll(reached);
   // Whole bricks with 16-byte rows: a row is read as vectors.
   const bool whole =
-      staged || (vec && ballot(b.ni < R || b.nj < R || b.nk < R) == 0);
+      !kStage || staged || (vec && ballot(b.ni < R || b.nj < R || b.nk < R) == 0);
   if (whole && wave_sum(n_items) > kDenseItems) {  // uniform per wave
     T T0 = 0, T1 = 0, T2 = 0, Y0 = 0, Z0 = 0, Y1 = 0, Z1 = 0, YY = 0, YZ = 0, ZZ = 0;
     if (ballot(rec.live) != 0) {
-      if (staged)
-        voxel_brick_full<T, R, true>(rec, b, s_v + (key - key0) * kBrick, R * R, R, dx0, T0, T1,
-                                     T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ, reached);
+      if (kStage && staged)
+        voxel_brick_full<T, R, true, kStage>(rec, b, s_v + (key - key0) * kBrick, R * R, R, dx0,
+                                             T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ, reached);
       else
-        voxel_brick_full<T, R, true>(rec, b,
-                                     v_vol + b.oi * plane + static_cast<int64_t>(b.oj) * D2 + b.ok,
-                                     plane, D2, dx0, T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ,
-                                     reached);
+        voxel_brick_full<T, R, true, kStage>(
+            rec, b, v_vol + b.oi * plane + static_cast<int64_t>(b.oj) * D2 + b.ok, plane, D2, dx0,
+            T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ, reached);
     }
     finish(T0, T1, T2, Y0, Z0, Y1, Z1, YY, YZ, ZZ);
     return;
@@ -1011,6 +1062,19 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
   const T c2 = (static_cast<T>(b.oi) + half) - rec.m[2];
   const typename Bits<T>::type my_lim = rec.live ? rec.lim : 0;
   s_rows[w][lane] = reached;
+  if constexpr (!kStage) {
+    ChunkRecord<T> cr;
+    cr.c[0] = dx0;
+    cr.c[1] = c1;
+    cr.c[2] = c2;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) cr.h[c] = rec.h[c];
+    cr.lim = my_lim;
+    // Below 2^32: the caller checks the volume's bytes.
+    cr.brick0 = ((static_cast<uint32_t>(b.oi) * D1 + static_cast<uint32_t>(b.oj)) * D2 +
+                 static_cast<uint32_t>(b.ok)) * static_cast<uint32_t>(sizeof(T));
+    s_rec[w].store(static_cast<int>(lane), cr);
+  }
 #pragma unroll
   for (int c = 0; c < 10; ++c) s_acc[w][c][lane] = 0;
   // Chunk list: the full chunks in (chunk index, record) order, then each
@@ -1078,16 +1142,32 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
       const bool act = ci < n_list;
       const uint32_t ent = act ? static_cast<uint32_t>(s_chunk[w][ci]) : 0u;
       const uint32_t rl = ent & 63u, pos = (ent >> 6) & 63u, q = ent >> 12;
-      // The record, from the registers of the lane that loaded it (every lane
-      // takes part); the conic scaled as scaled_conic does.
-      const int src = static_cast<int>(rl);
-      T qr[6], hr[6];
+      T hr[6], cx, cy, cz;
+      typename Bits<T>::type r_lim;
+      uint32_t at0 = 0, r_key = 0;
+      if constexpr (kStage) {
+        // The record, from the registers of the lane that loaded it (every
+        // lane takes part); the conic scaled as scaled_conic does.
+        const int src = static_cast<int>(rl);
+        T qr[6];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) qr[c] = __shfl(rec.q[c], src, 64);
-      scaled_conic(qr, hr);
-      const T cx = __shfl(dx0, src, 64), cy = __shfl(c1, src, 64), cz = __shfl(c2, src, 64);
-      const typename Bits<T>::type r_lim = shfl_bits(my_lim, src);
-      const uint32_t r_key = static_cast<uint32_t>(__shfl(static_cast<int>(key), src, 64));
+        for (int c = 0; c < 6; ++c) qr[c] = __shfl(rec.q[c], src, 64);
+        scaled_conic(qr, hr);
+        cx = __shfl(dx0, src, 64);
+        cy = __shfl(c1, src, 64);
+        cz = __shfl(c2, src, 64);
+        r_lim = shfl_bits(my_lim, src);
+        r_key = static_cast<uint32_t>(__shfl(static_cast<int>(key), src, 64));
+      } else {
+        const ChunkRecord<T> cr = s_rec[w].load(static_cast<int>(rl));
+#pragma unroll
+        for (int c = 0; c < 6; ++c) hr[c] = cr.h[c];
+        cx = cr.c[0];
+        cy = cr.c[1];
+        cz = cr.c[2];
+        r_lim = cr.lim;
+        at0 = cr.brick0;
+      }
       const uint64_t rows_m = s_rows[w][rl];
       const int n_here =
           act ? min(R, __popcll(rows_m) - static_cast<int>(q) * R) : 0;
@@ -1102,11 +1182,10 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
       }
       // The brick's gradient: staged, or in the volume.
       const T *__restrict__ vb = v_vol;
-      uint32_t sv = 0;
       int nk = R;
       if constexpr (kStaged) {
-        sv = (r_key - key0) * kBrick;
-      } else {
+        at0 = (r_key - key0) * kBrick;
+      } else if constexpr (kStage) {
         const Brick bb = brick_of(r_key + koff, n2, n1, R, D2, D1, D0);
         vb += bb.oi * plane + static_cast<int64_t>(bb.oj) * D2 + bb.ok;
         nk = bb.nk;
@@ -1130,16 +1209,26 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
         const T B = fma(hr[1], dy, hr[2] * dz);
         const T C = fma(fma(hr[3], dy, hr[4] * dz), dy, hr[5] * dz * dz);
         typename Bits<T>::type lim = item ? r_lim : 0;
-        asm volatile("" : "+v"(lim));  // one select, not a scalar AND per voxel
+        if constexpr (kStage) asm volatile("" : "+v"(lim));  // one select, not an AND per voxel
         T vv[R];
         if constexpr (kStaged) {
-          const T *vrow = s_v + (sv + p * R);
+          const T *vrow = s_v + (at0 + p * R);
 #pragma unroll
           for (int c = 0; c < R / kq; ++c)
             *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
         } else {
-          const T *__restrict__ vrow = vb + (li * plane + static_cast<int64_t>(lj) * D2);
-          if (whole) {
+          const T *__restrict__ vrow;
+          if constexpr (kStage) {
+            vrow = vb + (li * plane + static_cast<int64_t>(lj) * D2);
+          } else {
+            // Two full-rate multiply-adds: li, lj < 8 and the strides in bytes
+            // below 2^24 (the caller checks).
+            uint32_t at = __umul24(lj, D2 * static_cast<uint32_t>(sizeof(T))) + at0;
+            asm volatile("" : "+v"(at));  // not two products and a sum
+            at += __umul24(li, D1 * D2 * static_cast<uint32_t>(sizeof(T)));
+            vrow = reinterpret_cast<const T *>(reinterpret_cast<const char *>(v_vol) + at);
+          }
+          if (!kStage || whole) {
 #pragma unroll
             for (int c = 0; c < R / kq; ++c)
               *reinterpret_cast<Q *>(vv + c * kq) = *reinterpret_cast<const Q *>(vrow + c * kq);
@@ -1153,14 +1242,17 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
         }
         T s0 = 0, s1 = 0;
 #pragma unroll
-        for (int h = 0; h < R; h += R / 2) {  // in halves: eight registers fewer
-          T sl[R / 2], e[R / 2];
+        for (int h = 0; h < R; h += kRun) {
+          T sl[kRun], e[kRun];
 #pragma unroll
-          for (int k = 0; k < R / 2; ++k)
+          for (int k = 0; k < kRun; ++k)
             sl[k] = fma(fma(hr[0], dxk[h + k], B), dxk[h + k], C);
-          neg_exp2_run(sl, e);
+          if constexpr (kRun > 1)
+            neg_exp2_run(sl, e);
+          else
+            e[0] = neg_exp2(sl[0]);
 #pragma unroll
-          for (int k = 0; k < R / 2; ++k) {
+          for (int k = 0; k < kRun; ++k) {
             // A failing voxel adds an exact zero whatever its upstream gradient
             // (a non-finite one included), as when the voxel is skipped.  The
             // product is formed unconditionally: as an operand of the
@@ -1209,7 +1301,7 @@ __global__ __launch_bounds__(64 * kChunkWaves, sizeof(T) == 4 ? 5 : 3) void voxe
       }
     }
   };
-  if (staged)
+  if (kStage && staged)
     walk(std::true_type{});
   else
     walk(std::false_type{});
@@ -1394,16 +1486,29 @@ int voxel_bwd_impl(const T *means3d, const T *conics, const T *opac,
   launch_voxel_bwd<T, RR, EXACT>(means3d, conics, opac, tile_offsets, isect_ids, flatten_ids,  \
                                  isect_src, n_isects, n_keys, koff, N, v_vol, D2, D1, D0, ts,  \
                                  n2, n1, vec, v_means, v_conics, v_opac, rows, stream)
-  if (ts == 8 && rows != nullptr) {
+  const int64_t elem = static_cast<int64_t>(sizeof(T));
+  // The unstaged chunks read whole bricks at 32-bit offsets and 24-bit strides.
+  const bool whole = vec && D2 % 8 == 0 && D1 % 8 == 0 && D0 % 8 == 0 &&
+                     n2 * 8 == D2 && n1 * 8 == D1 &&
+                     (static_cast<int64_t>(z0) + n0) * 8 <= D0 &&
+                     n_vox * elem <= (int64_t{1} << 32) &&
+                     static_cast<int64_t>(D1) * D2 * elem < (int64_t{1} << 24);
+  const bool stage = stage_bricks<T>(n_isects, n_keys, whole);
+  if (ts == 8 && rows != nullptr && (stage || whole)) {
     const dim3 grid(static_cast<uint32_t>(ceil_div(n_isects, 64 * kChunkWaves)));
-    if (reach != nullptr)
-      voxel_bwd_chunk_kernel<T, true><<<grid, dim3(64 * kChunkWaves), 0, stream>>>(
-          means3d, conics, opac, tile_offsets, isect_ids, flatten_ids, isect_src, n_isects,
-          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, vec, rows, reach);
+#define R2S_VOXEL_BWD_CHUNK(GIVEN, STAGE)                                                       \
+  voxel_bwd_chunk_kernel<T, GIVEN, STAGE><<<grid, dim3(64 * kChunkWaves), 0, stream>>>(         \
+      means3d, conics, opac, tile_offsets, isect_ids, flatten_ids, isect_src, n_isects, n_keys, \
+      koff, N, v_vol, D2, D1, D0, n2, n1, vec, rows, reach)
+    if (reach != nullptr && stage)
+      R2S_VOXEL_BWD_CHUNK(true, true);
+    else if (reach != nullptr)
+      R2S_VOXEL_BWD_CHUNK(true, false);
+    else if (stage)
+      R2S_VOXEL_BWD_CHUNK(false, true);
     else
-      voxel_bwd_chunk_kernel<T, false><<<grid, dim3(64 * kChunkWaves), 0, stream>>>(
-          means3d, conics, opac, tile_offsets, isect_ids, flatten_ids, isect_src, n_isects,
-          n_keys, koff, N, v_vol, D2, D1, D0, n2, n1, vec, rows, nullptr);
+      R2S_VOXEL_BWD_CHUNK(false, false);
+#undef R2S_VOXEL_BWD_CHUNK
   } else if (ts == 8)
     R2S_VOXEL_BWD_R(8, true);
   else if (ts == 4)

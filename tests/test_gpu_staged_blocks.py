@@ -11,9 +11,10 @@ import torch
 
 from helpers import (assert_close, check_raster, check_voxel, np32, raster_references,
                      voxel_references)
+from oracle import ops
 from r2splat.cuda import _ops
 from r2splat.cuda import _wrapper as W
-from test_gpu_ops import DEV, _raster_case, _voxel_case
+from test_gpu_ops import DEV, _prepared, _raster_case, _voxel_case
 
 pytestmark = pytest.mark.gpu
 
@@ -103,23 +104,37 @@ def test_voxel_backward_blocks(dtype, n, dims, log_mu, staged):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("dims", [(90, 61, 77), (92, 61, 77), (96, 61, 80)])
-def test_voxel_backward_full_chunk_lists(dims, dtype):
-    """A few Gaussians that cover the whole volume: blocks over too many bricks to stage, whose
-    records reach every row, in bricks that cannot be read whole (ragged, or rows that no
-    16-byte load fits): the longest chunk lists."""
-    d, m3, con, ids, fl, off = _voxel_case(5, 8, dims, 8, dtype, log_mu=-0.7)
-    assert min(int(b.max() - b.min()) + 1 for b in ids.split(256)[:-1]) > 6
+@pytest.mark.parametrize("n,dims,dtype", [
+    (n, dims, dtype) for dims in ((90, 61, 77), (92, 61, 77), (96, 61, 80), (96, 64, 80))
+    for n, dtype in ((0, torch.float32), (0, torch.float64),
+                     (66_000 if dims == (96, 64, 80) else 42_000,
+                      torch.float64 if dims == (92, 61, 77) else torch.float32))])
+def test_voxel_backward_full_chunk_lists(n, dims, dtype):
+    """A few Gaussians that cover the whole volume: records that reach every row, in blocks over
+    too many bricks to stage, of bricks that cannot be read whole (ragged, or rows that no
+    16-byte load fits) and of whole ones.  n: small Gaussians that crowd a corner beside them,
+    whose records make the list one that stages where it can; the rest takes the same kernel's
+    longest chunk lists."""
+    n2, n1, n0 = (-(-x // 8) for x in dims)
+    d = _prepared(5 + n, 8, dtype, log_mu=-0.7)
+    small = ops.parameter_transform_fwd(
+        d["raw"].quats.double().numpy(), np.full((5 + n, 3), -7.0), 5e-4, 1.0)[0]
+    d["covars"][5:] = torch.as_tensor(small, dtype=dtype, device=DEV)[5:]
+    d["means"][5:] = 0.01 * d["means"][5:] - 0.94
+    ranges, centers = (torch.full((3,), x, dtype=dtype, device=DEV) for x in (2.0, 0.0))
+    m3, con, r3 = W.world_to_volume_mapping_fwd(d["means"], d["covars"], d["opac"], ranges,
+                                                centers, *dims, 1e-8, 3.0)
+    _, ids, fl = W.isect_tiles_3d(m3, r3, 8, n2, n1, n0)
+    off = W.isect_offset_encode_3d(ids, n2, n1, n0)
+    whole = all(x % 8 == 0 for x in dims)
+    assert (ids.numel() >= (65536 if whole else 256 * off.numel() / 6)) == (n > 0)
+    spans = np.array([int(b.max() - b.min()) + 1 for b in ids.split(256)[:-1]])
+    assert spans.max() > 6 and (spans.min() <= 6) == (n > 0)
     op = d["opac"]
     _, reach = _ops.voxelize_with_reach(m3, con, op, off, fl, *dims)
     rows = np.array([bin(int(x)).count("1") for x in reach.cpu().numpy().view(np.uint64)])
     chunks = np.add.reduceat(-(-rows // 8), np.arange(0, rows.size, 64))
-    n2, n1, _ = (-(-x // 8) for x in dims)
-    at = np.stack([np32(ids) % n2, np32(ids) // n2 % n1, np32(ids) // (n2 * n1)], 1)
-    ragged = ((at + 1) * 8 > np.array(dims)).any(1) | (dims[0] % 4 != 0)
-    split = np.add.reduceat(ragged, np.arange(0, rows.size, 64)) > 0
-    assert chunks[split].max() > 448, chunks
+    assert chunks[np.repeat(spans > 6, 4)[:chunks.size].nonzero()].max() > 448, chunks
     v = torch.randn((dims[2], dims[1], dims[0]), generator=d["gen"], dtype=dtype)
     refs = voxel_references(np32(m3), np32(con), np32(op), np32(off), np32(fl), *dims, 8,
                             v_volume=v.numpy())
