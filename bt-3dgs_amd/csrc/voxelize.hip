@@ -343,15 +343,34 @@ __device__ __forceinline__ uint64_t reach_mask(const BwdRecord<T> &rec, const Br
 
 // A batch of the forward below whose records reach at least this share of
 // their 64 rows on average walks every row: no set to step through, uniform
-// reads of the staged records, no transpose.  Measured on trees (7.1 M records
-// of a 250 x 201 x 173 volume, nearly every row reached) 0.888 -> 0.821 ms,
-// and 0.809 ms with equal shares per wave; from 5/8 on the same, and lists of
-// small footprints (0.62 of the rows walked) stay below it.
+// reads of the staged records, no transpose; and the wave's next batch does
+// so without its masks while half of its records look as large (box_is_dense,
+// a few operations a record where the masks take hundreds).  Measured on
+// trees (6.8 M records of a 250 x 201 x 173 volume, nearly every row reached)
+// 0.974 -> 0.785 ms, 0.883 with every batch's masks formed; and on 2000 large
+// Gaussians before 600k tiny ones at 128^3 0.207 -> 0.196 ms, where a wave
+// that never looked again took 0.253.  From 5/8 on the same; lists of small
+// footprints (0.62 of the rows walked) stay below it.
 constexpr int kDenseShareNum = 3, kDenseShareDen = 4;
+
+// Whether a record's alpha-test ellipsoid reaches about that share of its
+// brick's rows, from its half-widths along y and z through the mean:
+// sigma log2(e) = h3 dy^2 (h5 dz^2) meets the test's limit there.
+template <typename T>
+__device__ __forceinline__ bool box_is_dense(const BwdRecord<T> &rec, const Brick &b) {
+  const T limit = limit_as_value(rec.lim);
+  const T hy = cull_sqrt(limit / rec.h[3]), hz = cull_sqrt(limit / rec.h[5]);
+  const T zero = 0, eight = 8;
+  const T y = rec.m[1] - static_cast<T>(b.oj), z = rec.m[2] - static_cast<T>(b.oi);
+  const T ny = fmin(y + hy, eight) - fmax(y - hy, zero);
+  const T nz = fmin(z + hz, eight) - fmax(z - hz, zero);
+  return ny > zero && nz > zero && ny * nz * kDenseShareDen >= 64 * kDenseShareNum;
+}
 
 // Forward at brick size 8 with culled rows.  S waves per brick; lane =
 // x-row (slice lane / 8, row lane % 8), its 8 voxels in registers.  Wave w
-// takes the w-th of S equal shares of the brick's list, in batches of 64.
+// takes the batches of 64 records w, w + S, w + 2S, ... of the brick's list
+// (a list whose Gaussians differ in size along it is shared out evenly).
 // Per batch, each lane loads one record and the rows it reaches
 // (reach_mask); a 64 x 64 bit transpose hands each row's lane the set of
 // batch records that reach that row; each lane then walks its own set in
@@ -363,7 +382,7 @@ constexpr int kDenseShareNum = 3, kDenseShareDen = 4;
 // through LDS, a fixed order.  reach_out (optional): each record's reach
 // mask, stored at its list position for a backward over the same lists.
 template <typename T, int S>
-__global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
+__global__ __launch_bounds__(64 * S, sizeof(T) == 4 ? 1 : 3) void voxel_fwd_reach_kernel(
     const T *__restrict__ means3d, const T *__restrict__ conics, const T *__restrict__ opac,
     const int32_t *__restrict__ tile_offsets, const int32_t *__restrict__ flatten_ids,
     int64_t n_isects, uint32_t n_keys, uint32_t koff, int64_t N, uint32_t D2, uint32_t D1,
@@ -388,7 +407,7 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
   const T px0 = static_cast<T>(b.ok) + half;
   const int64_t l0 = tile_offsets[key];
   const int64_t l1 = (key == n_keys - 1) ? n_isects : static_cast<int64_t>(tile_offsets[key + 1]);
-  const int64_t start = l0 + (l1 - l0) * w / S, end = l0 + (l1 - l0) * (w + 1) / S;
+  const int64_t start = l0 + 64 * w, end = l1;
   T acc[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) acc[k] = 0;
@@ -413,24 +432,26 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
   // trip fewer before the records' own loads).
   int64_t idx = start + lane;
   int32_t next_id = idx < end ? flatten_ids[idx] : -1;
-  bool all_rows = false;  // uniform: an earlier batch reached nearly every row
-  for (int64_t base = start; base < end; base += 64) {
+  bool all_rows = false;  // uniform: the batch before walked every row
+  for (int64_t base = start; base < end; base += 64 * S) {
     const bool in = idx < end;
     const int64_t at = idx, g = in ? static_cast<int64_t>(next_id) : -1;
-    idx += 64;
+    idx += 64 * S;
     next_id = idx < end ? flatten_ids[idx] : -1;
+    const int cnt = static_cast<int>(min(static_cast<int64_t>(64), end - base));
     BwdRecord<T> rec;
     uint64_t reach = 0;
-    // A caller that takes the masks needs every batch's; otherwise, once a
-    // batch of the brick reached nearly every row, the next ones walk them
-    // all (a row that a record does not reach adds exact zeros).
-    const bool cull = reach_out != nullptr || !all_rows;
+    // Walking a row that a record does not reach adds exact zeros, so a dense
+    // batch needs no masks; a caller that takes the masks needs every batch's.
+    bool cull = true;
+    if (all_rows && reach_out == nullptr) {
+      load_bwd_record_plain(means3d, conics, opac, g, N, in, b, rec);
+      cull = __popcll(ballot(rec.live && box_is_dense(rec, b))) * 2 < cnt;
+    }
     if (cull) {
       load_bwd_record(means3d, conics, opac, g, N, in, b, rec);
       reach = rec.live ? reach_mask(rec, b, px0 - rec.m[0]) : 0ull;
       if (reach_out != nullptr && in) reach_out[at] = reach;
-    } else {
-      load_bwd_record_plain(means3d, conics, opac, g, N, in, b, rec);
     }
     V4 a, hq, hr, d0, d1;
     a.x = rec.m[1];
@@ -469,7 +490,6 @@ __global__ __launch_bounds__(64 * S) void voxel_fwd_reach_kernel(
     s_rec[w][lane][2] = hr;
     s_rec[w][lane][3] = d0;
     s_rec[w][lane][4] = d1;
-    const int cnt = static_cast<int>(min(static_cast<int64_t>(64), end - base));
     // Walking every row in step costs about kDenseShare of walking each
     // row's own set, record for record (uniform reads, no set to step
     // through, no transpose).

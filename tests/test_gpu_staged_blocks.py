@@ -147,6 +147,37 @@ def test_voxel_backward_full_chunk_lists(n, dims, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("dims", [(64, 64, 64), (40, 37, 33), (20, 17, 18)])
+@pytest.mark.parametrize("order", ["large first", "small first", "mixed"])
+def test_voxel_forward_over_batches_of_both_kinds(order, dims, dtype):
+    """Large Gaussians and small ones in one list: waves that walk every row of one batch and
+    each row's own set of the next, with one, two and four waves a brick.  The volume is the
+    oracle's, and the same bit for bit where every batch's masks are formed."""
+    n = 1500
+    d = _prepared(2 * n, 13, dtype, log_mu=-1.0)
+    small = ops.parameter_transform_fwd(d["raw"].quats.double().numpy(),
+                                        np.full((2 * n, 3), -3.5), 5e-4, 1.0)[0]
+    at = torch.arange(2 * n, device=DEV)
+    large = {"large first": at < 300, "small first": at >= 2 * n - 300,
+             "mixed": at // 100 % 10 == 0}[order]
+    covars = torch.where(large[:, None], d["covars"], torch.as_tensor(small, dtype=dtype).to(DEV))
+    ranges, centers = (torch.full((3,), x, dtype=dtype, device=DEV) for x in (2.0, 0.0))
+    m3, con, r3 = W.world_to_volume_mapping_fwd(d["means"], covars, d["opac"], ranges, centers,
+                                                *dims, 1e-8, 3.0)
+    grid = [-(-x // 8) for x in dims]
+    _, ids, fl = W.isect_tiles_3d(m3, r3, 8, *grid)
+    off = W.isect_offset_encode_3d(ids, *grid)
+    vol = W.voxelize_to_voxels_fwd(m3, con, d["opac"], off, fl, *dims, 8)
+    vol_r, reach = _ops.voxelize_with_reach(m3, con, d["opac"], off, fl, *dims)
+    assert torch.equal(vol, vol_r)
+    rows = np.array([bin(int(x)).count("1") for x in reach.cpu().numpy().view(np.uint64)])
+    dense = np.add.reduceat(rows, np.arange(0, rows.size, 64)) >= 48 * 64
+    assert dense.any() and not dense.all()
+    refs = voxel_references(np32(m3), np32(con), np32(d["opac"]), np32(off), np32(fl), *dims, 8)
+    print(fl.numel() // off.numel(), dense.mean(), check_voxel(refs, volume=np32(vol)))
+
+
 @pytest.mark.parametrize("first", [1, 100, 700])
 def test_offsets_that_start_after_the_first_record(first):
     """Records before a caller's first tile (brick) offset have no key to be found: they count
