@@ -652,6 +652,8 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
 // of 512^2 over half rows and 60 us over full ones (27k: 65 and 56), the same
 // from 260k on.  The two-pass form without absolute gradients takes 15.2 us
 // for 86k records by full rows and 14.0 by half rows, 308 and 304 for 4.3 M.
+// The sums add in raster_tile_walk's order, so that the one- and the two-pass
+// form differ by the order of the atomics alone.
 template <typename T, int R, bool kAbs>
 __device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &rec,
                                                         const T *__restrict__ vimg, uint32_t W,
@@ -659,7 +661,9 @@ __device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &r
   using Q = typename Quad<T>::type;
   constexpr int kq = Quad<T>::n;
   TileSums<T> s = {0, 0, 0, 0, 0, 0, 0, 0};
-  T dxk[R], wk[R];
+  constexpr int kParts = R / kChunk;
+  T dxk[R], wk[R], y0[kParts] = {}, yy[kParts] = {}, y1[kParts] = {}, ax[kParts] = {},
+                   ay[kParts] = {};
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     dxk[k] = dx0 + static_cast<T>(k);
@@ -676,9 +680,9 @@ __device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &r
     const T bdy = rec.b * dy, cdy = rec.c * dy;
     const typename Bits<T>::type lim = in_row ? rec.lim : 0;
     const T *__restrict__ vrow = vimg + static_cast<int64_t>(in_row ? i : oy) * W + ox;
-    T s0 = 0, s1 = 0, px = 0, py = 0;
 #pragma unroll
     for (int h = 0; h < R; h += kChunk) {
+      T s0 = 0, s1 = 0, px = 0, py = 0;
       T vv[kChunk];
 #pragma unroll
       for (int q = 0; q < kChunk / kq; ++q)
@@ -697,13 +701,12 @@ __device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &r
           py = fma(fabs(w), fabs(fma(rec.b, dx, cdy)), py);
         }
       }
-    }
-    s.Y0 += dy * s0;
-    s.YY += dy * (dy * s0);
-    s.Y1 += dy * s1;
-    if (kAbs) {
-      s.PX += px;
-      s.PY += py;
+      const T t = dy * s0;
+      y0[h / kChunk] += t;
+      yy[h / kChunk] = fma(dy, t, yy[h / kChunk]);
+      y1[h / kChunk] = fma(dy, s1, y1[h / kChunk]);
+      ax[h / kChunk] += px;
+      ay[h / kChunk] += py;
     }
   }
 #pragma unroll
@@ -712,6 +715,14 @@ __device__ __forceinline__ TileSums<T> raster_tile_full(const RasterRecord<T> &r
     s.T0 += wk[k];
     s.T1 += wx;
     s.T2 += wx * dxk[k];
+  }
+#pragma unroll
+  for (int c = 0; c < kParts; ++c) {
+    s.Y0 += y0[c];
+    s.YY += yy[c];
+    s.Y1 += y1[c];
+    s.PX += ax[c];
+    s.PY += ay[c];
   }
   return s;
 }
