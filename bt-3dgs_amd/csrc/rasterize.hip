@@ -1232,10 +1232,10 @@ void launch_raster_bwd(const T *means2d, const T *conics, const T *opac, const T
       n_keys, n_items, v_image, W, H, ts, tw, th, vec, v_xy_abs, v_xy, v_conic, v_opac, v_mu,    \
       rows, payload)
   if (v_xy_abs != nullptr || (rows != nullptr && absgrad)) {
-    if (rows != nullptr)
-      R2S_RASTER_BWD_LAUNCH(true, true);
-    else
+    if (rows == nullptr)
       R2S_RASTER_BWD_LAUNCH(true, false);
+    else if constexpr (!(kExact && R == 16))  // raster_bwd_split_kernel takes those
+      R2S_RASTER_BWD_LAUNCH(true, true);
   } else {
     if (rows != nullptr)
       R2S_RASTER_BWD_LAUNCH(false, true);

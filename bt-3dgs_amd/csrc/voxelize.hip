@@ -7,11 +7,11 @@
 //   sigma log2(e) = (h0 dx + B) dx + C,  h0 = p00 log2(e) / 2,
 // two FMAs per voxel and one v_exp_f32 for exp(-sigma) = 2^-(sigma log2 e).
 //
-// Forward: one workgroup per brick; each thread owns R consecutive voxels of
-// one x-row (R = ts for ts = 8, 16; R = 1 otherwise) and sums the brick's list
-// in list order, as the reference does, so the result is deterministic.
-// Records are staged in LDS in batches with their conics pre-scaled and read
-// as broadcasts.
+// Forward: one workgroup per brick.  At brick size 8 a lane owns an x-row of
+// eight voxels and one to four waves share the brick's list (in a fixed order:
+// the result is deterministic); at other sizes a thread owns a voxel and sums
+// the list in order, as the reference does.  Records are staged in LDS in
+// batches with their conics pre-scaled and read as broadcasts.
 //
 // Backward: one lane per record of the sorted list, so a wave takes 64
 // consecutive records (nearly always of one brick) and the work is balanced
@@ -85,7 +85,8 @@ __device__ __forceinline__ void scaled_conic(const T q[6], T h[6]) {
   h[5] = hl * q[5];
 }
 
-template <typename T, int R>
+// Forward for brick sizes other than 8: one thread per voxel.
+template <typename T>
 __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
     const T *__restrict__ means3d, const T *__restrict__ conics, const T *__restrict__ opac,
     const int32_t *__restrict__ tile_offsets, const int32_t *__restrict__ flatten_ids,
@@ -101,20 +102,17 @@ __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
   const uint32_t key = xcd_swizzle(blockIdx.x, n_keys);  // in the lists (koff: the grid's)
   const Brick b = brick_of(key + koff, n2, n1, ts, D2, D1, D0);
   const uint32_t tid = threadIdx.x;
-  const uint32_t per_row = ts / R;
-  const int lk0 = static_cast<int>((tid % per_row) * R);
-  const int lj = static_cast<int>((tid / per_row) % ts);
-  const int li = static_cast<int>(tid / (per_row * ts));
+  const int lk = static_cast<int>(tid % ts);
+  const int lj = static_cast<int>((tid / ts) % ts);
+  const int li = static_cast<int>(tid / (ts * ts));
   const T half = static_cast<T>(0.5);
   const T py = static_cast<T>(b.oj + lj) + half;
   const T pz = static_cast<T>(b.oi + li) + half;
-  const T px0 = static_cast<T>(b.ok + lk0) + half;
+  const T px = static_cast<T>(b.ok + lk) + half;
 
   const int64_t start = tile_offsets[key];
   const int64_t end = (key == n_keys - 1) ? n_isects : static_cast<int64_t>(tile_offsets[key + 1]);
-  T acc[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = 0;
+  T acc = 0;
   for (int64_t base = start; base < end; base += nb) {
     __syncthreads();
     const int64_t idx = base + tid;
@@ -160,31 +158,18 @@ __global__ __launch_bounds__(1024) void voxel_fwd_kernel(
       const V4 h0 = s_rec[3 * t + 1];
       const V4 h1 = s_rec[3 * t + 2];
       const typename Bits<T>::type lim = bits_of(h1.z);
-      const T dy = py - mo.y, dz = pz - mo.z;
+      const T dx = px - mo.x, dy = py - mo.y, dz = pz - mo.z;
       const T B = h0.y * dy + h0.z * dz;
       const T C = (h0.w * dy + h1.x * dz) * dy + h1.y * dz * dz;
-      constexpr int kRun = R < 8 ? R : 8;  // voxels per run of exps
-#pragma unroll
-      for (int r = 0; r < R; r += kRun) {
-        T sl[kRun], e[kRun];
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) {
-          const T dx = (px0 + static_cast<T>(r + k)) - mo.x;
-          sl[k] = fma(fma(h0.x, dx, B), dx, C);
-        }
-        neg_exp2_run(sl, e);
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) add_passing(sl[k], e[k], lim, mo.w, acc[r + k], exec);
-      }
+      const T sl[1] = {fma(fma(h0.x, dx, B), dx, C)};
+      T e[1];
+      neg_exp2_run(sl, e);
+      add_passing(sl[0], e[0], lim, mo.w, acc, exec);
     }
   }
-  if (li < b.ni && lj < b.nj) {
-    T *out = volume + static_cast<int64_t>(b.oi + li) * D1 * D2 +
-             static_cast<int64_t>(b.oj + lj) * D2 + (b.ok + lk0);
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (lk0 + r < b.nk) out[r] = acc[r];
-  }
+  if (li < b.ni && lj < b.nj && lk < b.nk)
+    volume[static_cast<int64_t>(b.oi + li) * D1 * D2 + static_cast<int64_t>(b.oj + lj) * D2 +
+           (b.ok + lk)] = acc;
 }
 
 // One backward record in registers.
@@ -641,53 +626,53 @@ __device__ __forceinline__ void voxel_brick_rows(const BwdRecord<T> &rec, const 
                                                  T &T0, T &T1, T &T2, T &Y0, T &Z0, T &Y1, T &Z1,
                                                  T &YY, T &YZ, T &ZZ) {
   const T half = static_cast<T>(0.5);
-      // Rolled loops: unrolled, the slices and rows multiply the registers.
+  // Rolled loops: unrolled, the slices and rows multiply the registers.
 #pragma unroll 1
-      for (int li = 0; li < R; ++li) {
-        if (!kExact && li >= nts) break;
-        const int i = b.oi + li;
-        const bool in_slice = rec.live && i >= rec.i0 && i <= rec.i1;
-        if (ballot(in_slice) == 0) continue;
-        const T dz = (static_cast<T>(i) + half) - rec.m[2];
-        // Rows of this slice the lane's ellipsoid can reach.
-        int j0, j1;
-        slice_rows(rec, b, in_slice, dz, dx0, j0, j1);
-        const T h4dz = rec.h[4] * dz, h5dzz = rec.h[5] * dz * dz, Bz = rec.h[2] * dz;
+  for (int li = 0; li < R; ++li) {
+    if (!kExact && li >= nts) break;
+    const int i = b.oi + li;
+    const bool in_slice = rec.live && i >= rec.i0 && i <= rec.i1;
+    if (ballot(in_slice) == 0) continue;
+    const T dz = (static_cast<T>(i) + half) - rec.m[2];
+    // Rows of this slice the lane's ellipsoid can reach.
+    int j0, j1;
+    slice_rows(rec, b, in_slice, dz, dx0, j0, j1);
+    const T h4dz = rec.h[4] * dz, h5dzz = rec.h[5] * dz * dz, Bz = rec.h[2] * dz;
 #pragma unroll 1
-        for (int lj = 0; lj < R; ++lj) {
-          if (!kExact && lj >= nts) break;
-          const int j = b.oj + lj;
-          const bool in_row = j >= j0 && j <= j1;
-          if (ballot(in_row) == 0) continue;
-          const T dy = (static_cast<T>(j) + half) - rec.m[1];
-          const T B = rec.h[1] * dy + Bz;
-          const T C = (rec.h[3] * dy + h4dz) * dy + h5dzz;
-          const T *__restrict__ vrow =
-              v_vol +
-              (in_row ? static_cast<int64_t>(i) * plane + static_cast<int64_t>(j) * D2 : 0) + b.ok;
-          T vv[R];
-          if (vec)
-            load_grad_row<T, R, true>(vrow, in_row, b.nk, nts, vv);
-          else
-            load_grad_row<T, R, false>(vrow, in_row, b.nk, nts, vv);
-          T s0 = 0, s1 = 0, s2 = 0;
-          if (guard)
-            voxel_row<T, R, kExact, true>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
-          else
-            voxel_row<T, R, kExact, false>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
-          T0 += s0;
-          T1 += s1;
-          T2 += s2;
-          const T dys0 = dy * s0, dzs0 = dz * s0;
-          Y0 += dys0;
-          Z0 += dzs0;
-          YY += dy * dys0;
-          YZ += dz * dys0;
-          ZZ += dz * dzs0;
-          Y1 += dy * s1;
-          Z1 += dz * s1;
-        }
-      }
+    for (int lj = 0; lj < R; ++lj) {
+      if (!kExact && lj >= nts) break;
+      const int j = b.oj + lj;
+      const bool in_row = j >= j0 && j <= j1;
+      if (ballot(in_row) == 0) continue;
+      const T dy = (static_cast<T>(j) + half) - rec.m[1];
+      const T B = rec.h[1] * dy + Bz;
+      const T C = (rec.h[3] * dy + h4dz) * dy + h5dzz;
+      const T *__restrict__ vrow =
+          v_vol +
+          (in_row ? static_cast<int64_t>(i) * plane + static_cast<int64_t>(j) * D2 : 0) + b.ok;
+      T vv[R];
+      if (vec)
+        load_grad_row<T, R, true>(vrow, in_row, b.nk, nts, vv);
+      else
+        load_grad_row<T, R, false>(vrow, in_row, b.nk, nts, vv);
+      T s0 = 0, s1 = 0, s2 = 0;
+      if (guard)
+        voxel_row<T, R, kExact, true>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
+      else
+        voxel_row<T, R, kExact, false>(rec, vv, dx0, b.nk, nts, B, C, s0, s1, s2);
+      T0 += s0;
+      T1 += s1;
+      T2 += s2;
+      const T dys0 = dy * s0, dzs0 = dz * s0;
+      Y0 += dys0;
+      Z0 += dzs0;
+      YY += dy * dys0;
+      YZ += dz * dys0;
+      ZZ += dz * dzs0;
+      Y1 += dy * s1;
+      Z1 += dz * s1;
+    }
+  }
 }
 
 // Records in brick order (tile_offsets, flatten_ids; isect_ids optional),
@@ -1356,16 +1341,16 @@ int check_voxel_args(int64_t n_isects, int64_t N, uint32_t D2, uint32_t D1, uint
   return R2S_OK;
 }
 
-template <typename T, int R>
+template <typename T>
 void launch_voxel_fwd(const T *means3d, const T *conics, const T *opac,
                       const int32_t *tile_offsets, const int32_t *flatten_ids, int64_t n_isects,
                       uint32_t n_keys, uint32_t koff, int64_t N, uint32_t D2, uint32_t D1,
                       uint32_t D0, uint32_t ts, uint32_t n2, uint32_t n1, T *volume,
                       hipStream_t stream) {
-  const uint32_t nt = ts * ts * (ts / R);
+  const uint32_t nt = ts * ts * ts;
   const size_t smem =
       min(nt, kFwdBatch) * (3 * sizeof(typename Vec<T>::v4));
-  voxel_fwd_kernel<T, R><<<dim3(n_keys), dim3(nt), smem, stream>>>(
+  voxel_fwd_kernel<T><<<dim3(n_keys), dim3(nt), smem, stream>>>(
       means3d, conics, opac, tile_offsets, flatten_ids, n_isects, n_keys, koff, N, D2, D1, D0, ts,
       n2, n1, volume);
 }
@@ -1411,12 +1396,10 @@ int voxel_fwd_impl(const T *means3d, const T *conics, const T *opac,
     else
       R2S_VOXEL_FWD_REACH(4);
 #undef R2S_VOXEL_FWD_REACH
-  } else if (ts == 16)
-    launch_voxel_fwd<T, 16>(means3d, conics, opac, tile_offsets, flatten_ids, n_isects, n_keys,
-                            koff, N, D2, D1, D0, ts, n2, n1, volume, stream);
-  else
-    launch_voxel_fwd<T, 1>(means3d, conics, opac, tile_offsets, flatten_ids, n_isects, n_keys,
-                           koff, N, D2, D1, D0, ts, n2, n1, volume, stream);
+  } else {
+    launch_voxel_fwd<T>(means3d, conics, opac, tile_offsets, flatten_ids, n_isects, n_keys, koff,
+                        N, D2, D1, D0, ts, n2, n1, volume, stream);
+  }
   return check_launch(name);
 }
 
