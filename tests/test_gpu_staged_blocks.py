@@ -147,6 +147,55 @@ def test_voxel_backward_full_chunk_lists(n, dims, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dims,dtype", [((80, 72, 72), torch.float32),
+                                        ((69, 64, 70), torch.float32),
+                                        ((69, 64, 70), torch.float64)])
+def test_voxel_backward_of_records_that_reach_nothing(dims, dtype):
+    """Lists that name mostly Gaussians of other bricks, as long thin Gaussians' boxes do: blocks
+    in which no record reaches a row, and blocks over too many bricks to stage whose reaching
+    records lie in few; with and without the forward's reach masks."""
+    n2, n1, n0 = (-(-x // 8) for x in dims)
+    keys = n0 * n1 * n2
+    d = _prepared(400, 8, dtype, log_mu=-4.5)
+    d["means"][:, 0] = 0.5 * d["means"][:, 0] - 0.5  # in one half of the volume
+    ranges, centers = (torch.full((3,), x, dtype=dtype, device=DEV) for x in (2.0, 0.0))
+    m3, con, r3 = W.world_to_volume_mapping_fwd(d["means"], d["covars"], d["opac"], ranges,
+                                                centers, *dims, 1e-8, 3.0)
+    rng = np.random.default_rng(3)
+    count = np.where(np.arange(keys) % 12 < 10, 25, 400)
+    fl = np.concatenate([np.sort(rng.choice(400, c, replace=False)) for c in count])
+    ids = torch.as_tensor(np.repeat(np.arange(keys), count), device=DEV)
+    off = torch.as_tensor((np.cumsum(count) - count).astype(np.int32), device=DEV)
+    off = off.reshape(n0, n1, n2)
+    order = np.argsort(fl, kind="stable")  # Gaussian by Gaussian, as the records are emitted
+    src = np.empty(fl.size, np.int32)
+    src[order] = np.arange(fl.size)
+    emit, src, fl = (torch.as_tensor(a.astype(np.int32), device=DEV) for a in (fl[order], src, fl))
+    op = d["opac"]
+    _, reach = _ops.voxelize_with_reach(m3, con, op, off, fl, *dims)
+    hit = reach.cpu().numpy() != 0
+    span = {True: 0, False: 0}
+    empty = 0
+    for h, k in zip(np.split(hit, range(256, hit.size, 256)),
+                    np.split(ids.cpu().numpy(), range(256, hit.size, 256))):
+        empty += not h.any()
+        if h.any():
+            span[np.ptp(k) >= 6 and np.ptp(k[h]) < 6] += 1
+    assert empty > 5 and span[True] > 5 and span[False] > 5, (empty, span)
+    whole = all(x % 8 == 0 for x in dims)
+    assert hit.size >= (max(65536, 64 * keys) if whole else 256 * keys / 6)  # lists that stage
+    v = torch.randn((dims[2], dims[1], dims[0]), generator=d["gen"], dtype=dtype)
+    refs = voxel_references(np32(m3), np32(con), np32(op), np32(off), np32(fl), *dims, 8,
+                            v_volume=v.numpy())
+    lists = _ops.TileLists(None, ids, fl, emit, src, off)
+    plain, given = (_ops.voxel_backward(m3, con, op, off, lists, v.to(DEV), *dims, 8, **k)
+                    for k in ({}, {"reach": reach}))
+    for name, r in check_voxel(refs, grads=[np32(t) for t in plain]).items():
+        print(name, r)
+    for a, b in zip(plain, given):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("dims", [(64, 64, 64), (40, 37, 33), (20, 17, 18)])
 @pytest.mark.parametrize("order", ["large first", "small first", "mixed"])
