@@ -58,7 +58,8 @@ __device__ __forceinline__ double fast_exp(double x) { return exp(x); }
 
 constexpr int kBwdThreads = 256;
 // Pixels of a row evaluated together: an unrolled 8-pixel body in a rolled
-// loop keeps the kernel at 62 VGPRs (8 waves per SIMD) without spills.
+// loop keeps the masked rows at 51 to 64 VGPRs in float (8 waves per SIMD)
+// without spills.
 constexpr int kChunk = 8;
 
 template <typename T>
@@ -646,7 +647,7 @@ __device__ __forceinline__ TileSums<T> raster_tile_walk(const RasterRecord<T> &r
 // The whole tile of one record by full rows, read from memory, for tiles with
 // a row in the image at least.  As raster_tile_walk, but each lane tests the
 // rows outside its own reach (and so those beyond the image) against a zero
-// limit and reads its tile's first row there.  It takes 90 to 95 registers
+// limit and reads its tile's first row there.  It takes 94 to 98 registers
 // where the half rows take 73 to 80 and is the better form where the atomics
 // after it bound the kernel: the one-pass backward took 68 us for 45k records
 // of 512^2 over half rows and 60 us over full ones (27k: 65 and 56), the same
@@ -991,13 +992,14 @@ constexpr uint32_t kStageStride = 16 * 16 + 16;
 
 // The two-pass (rows) backward with absolute gradients at tile size 16.
 // Vector issue bounds it (1.5 vector instructions in flight per SIMD).  Half
-// a tile row at a time (raster_tile_walk) it takes 75 VGPRs instead of 89,
+// a tile row at a time (raster_tile_walk) it takes 80 VGPRs instead of 89,
 // and with the gradients staged it reads LDS, where 64 lanes times 16 bytes
 // per load kept the vector cache's return path busy for 86 % of the kernel's
-// time: 0.357 -> 0.345 ms for 4.7 M records on 512^2, 0.876 -> 0.818 ms for
-// 10.9 M on 1024^2.  Image widths that no 16-byte load fits and ragged tiles
-// take the same walk: a 333 x 217 projection of 200k Gaussians, forward and
-// backward, went from 269 to 238 us.
+// time: 0.352 -> 0.351 ms for 4.4 M records on 512^2, 0.883 -> 0.833 ms for
+// 10.9 M on 1024^2 (0.344 and 0.813 with both halves of a row in one chain of
+// sums, which rounds worse).  Image widths that no 16-byte load fits and
+// ragged tiles take the same walk: a 333 x 217 projection of 200k Gaussians,
+// forward and backward, went from 269 to 238 us.
 template <typename T>
 __global__ __launch_bounds__(kSplitThreads, sizeof(T) == 4 ? 6 : 1) void raster_bwd_split_kernel(
     const T *__restrict__ payload, const int32_t *__restrict__ tile_offsets,
